@@ -32,6 +32,7 @@ struct MlpNet {
     int Np = 0;                 // padded outputs of the last layer
     float *y = nullptr;         // output [Bp][Np] FP32
     double *loss = nullptr;     // [1 + nblocks] loss accumulator
+    float *xfer = nullptr;      // parameters or gradients in the interface layout, on their way to the host
     int step = 0;               // AdamW step count (bias correction)
     uint64_t seed = 0;
 };
