@@ -42,14 +42,6 @@ static void *scratch_ptr(int device) {
     return (device >= 0 && device < MAX_DEVICES) ? g_scratch_ptr[device] : nullptr;
 }
 
-// descriptors of a plain batched synthesis: field f copied to column pair f
-__global__ void k_copy_descs(SynthDesc *__restrict__ d, unsigned char *__restrict__ rflag, int nf) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nf) return;
-    d[f] = SynthDesc{SK_COPY, f, -1, 1.0, 0.0, 0, 0};
-    rflag[f] = 0;
-}
-
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 template <typename Tin, typename Tout>
@@ -220,20 +212,26 @@ template <typename T> int Engine<T>::output(const T *d, void *p, size_t n, int d
     return 0;
 }
 
+// A caller's device buffer of the context's element type that the last kernel
+// of a transform can write itself, else null (it writes the workspace, and
+// output() converts or copies). Grids take 16-byte stores.
+template <typename T> static T *direct(void *p, int dtype, int loc, bool grid) {
+    if (!p || loc != GFSDC_DEVICE || (dtype == GFSDC_DT_F64) != (sizeof(T) == 8)) return nullptr;
+    return grid && ((uintptr_t)p & 15) ? nullptr : (T *)p;
+}
+
 template <typename T> int Engine<T>::spectogrd(const void *spec, void *grid, int nf, int dtype, int loc) {
     if (nf <= 0) return nf == 0 ? 0 : GFSDC_EINVAL;
     int rc = work_alloc(work, plan, nf);
     if (rc) return rc;
     const T *in;
     if ((rc = input(spec, (size_t)nf * plan.nlm * 2, dtype, loc, 0, &in))) return rc;
-    std::vector<SynthDesc> sd(nf);
-    for (int f = 0; f < nf; f++) sd[f] = SynthDesc{SK_COPY, f, -1, 1.0, 0.0, 0, 0};
-    if ((rc = upload_descs(sd, {}, std::vector<unsigned char>(nf, 0)))) return rc;
-    launch_synth_gather(plan, (const cplx<T> *)in, plan.nlm, 1, d_sdesc, nf, work.sx, work.ldc, 1.0, stream);
+    T *out = direct<T>(grid, dtype, loc, true);
+    launch_gather_ref(plan, (const cplx<T> *)in, nf, work.sx, work.ldc, stream);
     launch_leg_synth(plan, work.sx, work.ldc, work.fs, work.ldc, 2 * nf, stream);
-    launch_fft_synth(plan, work.fs, work.ldc, work.grid, (long)plan.nlat * plan.nlon, nf, d_rflag, stream);
+    launch_fft_synth(plan, work.fs, work.ldc, out ? out : work.grid, (long)plan.nlat * plan.nlon, nf, nullptr, stream);
     GFSDC_CHECK(hipGetLastError());
-    return output(work.grid, grid, (size_t)nf * plan.nlat * plan.nlon, dtype, loc, 1);
+    return out ? 0 : output(work.grid, grid, (size_t)nf * plan.nlat * plan.nlon, dtype, loc, 1);
 }
 
 // spectogrd on device buffers of the context's element type with every
@@ -251,8 +249,7 @@ template <typename T> int Engine<T>::spectogrd_noalloc(const void *spec, void *g
         return GFSDC_ESTATE;
     }
     const int ldc = round_up(2 * nf, COL_PAD) + COL_SKEW;
-    const size_t o_rf = align256(sizeof(SynthDesc) * nf);
-    const size_t o_sx = o_rf + align256((size_t)nf);
+    const size_t o_sx = align256(sizeof(SynthDesc) * nf) + align256((size_t)nf);  // room for a descriptor and a flag each
     const size_t o_fs = o_sx + align256(sizeof(T) * (size_t)plan.nlme * ldc);
     const size_t need = o_fs + sizeof(T) * (size_t)(plan.ntrunc + 1) * plan.nlat * ldc;
     if (need > NOALLOC_SCRATCH_BYTES) {
@@ -262,13 +259,10 @@ template <typename T> int Engine<T>::spectogrd_noalloc(const void *spec, void *g
                   " MiB (use gfsdc_spectogrd, or fewer fields per call)");
         return GFSDC_EINVAL;
     }
-    SynthDesc *desc = (SynthDesc *)base;
-    unsigned char *rflag = (unsigned char *)(base + o_rf);
     T *sx = (T *)(base + o_sx), *fs = (T *)(base + o_fs);
-    hipLaunchKernelGGL(k_copy_descs, dim3((nf + 255) / 256), dim3(256), 0, stream, desc, rflag, nf);
-    launch_synth_gather(plan, (const cplx<T> *)spec, plan.nlm, 1, desc, nf, sx, ldc, 1.0, stream);
+    launch_gather_ref(plan, (const cplx<T> *)spec, nf, sx, ldc, stream);
     launch_leg_synth(plan, sx, ldc, fs, ldc, 2 * nf, stream);
-    launch_fft_synth(plan, fs, ldc, (T *)grid, (long)plan.nlat * plan.nlon, nf, rflag, stream);
+    launch_fft_synth(plan, fs, ldc, (T *)grid, (long)plan.nlat * plan.nlon, nf, nullptr, stream);
     GFSDC_CHECK(hipGetLastError());
     return 0;
 }
@@ -280,15 +274,13 @@ template <typename T> int Engine<T>::grdtospec(const void *grid, void *spec, int
     const T *in;
     size_t ng = (size_t)plan.nlat * plan.nlon;
     if ((rc = input(grid, (size_t)nf * ng, dtype, loc, 0, &in))) return rc;
-    std::vector<AnalDesc> ad(nf);
-    for (int f = 0; f < nf; f++) ad[f] = AnalDesc{AK_COPY, f, -1, 1.0, 0, 0, -1, 0.0};
-    if ((rc = upload_descs({}, ad, std::vector<unsigned char>(nf, 0)))) return rc;
-    launch_fft_anal(plan, in, (long)ng, nf, d_rflag, work.fa, work.ldc, stream);
+    launch_fft_anal(plan, in, (long)ng, nf, nullptr, work.fa, work.ldc, stream);
     launch_leg_anal(plan, work.fa, work.ldc, work.sx, work.ldc, 2 * nf, stream);
-    T *out = work.grid;  // reuse as spectral output buffer (nf * nlm complex <= nf * ng)
-    launch_anal_scatter(plan, work.sx, work.ldc, d_adesc, nf, (cplx<T> *)out, plan.nlm, 1, 1.0, stream);
+    T *dir = direct<T>(spec, dtype, loc, false);
+    T *out = dir ? dir : work.grid;  // reuse as spectral output buffer (nf * nlm complex <= nf * ng)
+    launch_scatter_ref(plan, work.sx, work.ldc, (cplx<T> *)out, nf, stream);
     GFSDC_CHECK(hipGetLastError());
-    return output(out, spec, (size_t)nf * plan.nlm * 2, dtype, loc, 1);
+    return dir ? 0 : output(out, spec, (size_t)nf * plan.nlm * 2, dtype, loc, 1);
 }
 
 // Transform microbenchmark with device-resident buffers: per iteration a
@@ -394,32 +386,26 @@ int Engine<T>::sphtor_to_spat(const void *s, const void *t, void *u, void *v, in
     if (nf <= 0) return nf == 0 ? 0 : GFSDC_EINVAL;
     int rc = work_alloc(work, plan, 2 * nf);
     if (rc) return rc;
-    size_t ns = (size_t)nf * plan.nlm * 2;
-    // both inputs in one device buffer [2 nf][nlm]
-    if ((rc = ensure_stage(2, 2 * ns * sizeof(T)))) return rc;
-    T *both = (T *)stage[2];
-    const T *in;
-    if (s) {
-        if ((rc = input(s, ns, dtype, loc, 0, &in))) return rc;
-        GFSDC_CHECK(hipMemcpyAsync(both, in, ns * sizeof(T), hipMemcpyDeviceToDevice, stream));
-    } else {
-        GFSDC_CHECK(hipMemsetAsync(both, 0, ns * sizeof(T), stream));
+    const size_t ns = (size_t)nf * plan.nlm * 2, ng = (size_t)plan.nlat * plan.nlon;
+    const T *is = nullptr, *it;
+    if (s && (rc = input(s, ns, dtype, loc, 0, &is))) return rc;
+    if ((rc = input(t, ns, dtype, loc, 2, &it))) return rc;
+    // the Fourier synthesis writes the caller's two grids, or both into the workspace
+    T *du = direct<T>(u, dtype, loc, true), *dv = direct<T>(v, dtype, loc, true);
+    const bool dir = du && dv;
+    if (!dir) {
+        du = work.grid;
+        dv = work.grid + nf * ng;
     }
-    if ((rc = input(t, ns, dtype, loc, 0, &in))) return rc;
-    GFSDC_CHECK(hipMemcpyAsync(both + ns, in, ns * sizeof(T), hipMemcpyDeviceToDevice, stream));
-    std::vector<SynthDesc> sd(2 * nf);
-    for (int f = 0; f < nf; f++) {
-        sd[f] = SynthDesc{SK_UHAT, f, nf + f, sscale, tscale, sinv, tinv};
-        sd[nf + f] = SynthDesc{SK_VHAT, f, nf + f, sscale, tscale, sinv, tinv};
-    }
-    if ((rc = upload_descs(sd, {}, std::vector<unsigned char>(2 * nf, 1)))) return rc;
-    launch_synth_gather(plan, (const cplx<T> *)both, plan.nlm, 1, d_sdesc, 2 * nf, work.sx, work.ldc, 1.0, stream);
+    launch_gather_ref_vec(plan, (const cplx<T> *)is, (const cplx<T> *)it, nf, work.sx, work.ldc, sscale, sinv, tscale,
+                          tinv, stream);
     launch_leg_synth(plan, work.sx, work.ldc, work.fs, work.ldc, 4 * nf, stream);
-    size_t ng = (size_t)plan.nlat * plan.nlon;
-    launch_fft_synth(plan, work.fs, work.ldc, work.grid, (long)ng, 2 * nf, d_rflag, stream);
+    launch_fft_synth(plan, work.fs, work.ldc, du, (long)ng, 2 * nf, nullptr, stream, (const T *)nullptr, nullptr, 0,
+                     nullptr, nullptr, 0.0, FftOpt<T>{dv, nf, 1});
     GFSDC_CHECK(hipGetLastError());
-    if ((rc = output(work.grid, u, nf * ng, dtype, loc, 1))) return rc;
-    return output(work.grid + nf * ng, v, nf * ng, dtype, loc, 1);
+    if (dir) return 0;
+    if ((rc = output(du, u, nf * ng, dtype, loc, 1))) return rc;
+    return output(dv, v, nf * ng, dtype, loc, 1);
 }
 
 // (Vt, Vp) -> vorticity / divergence (lap/rsphere S, lap/rsphere T), or SHTns (S, T) when inv = 1.
@@ -429,28 +415,24 @@ int Engine<T>::spat_to_sphtor(const void *u, const void *v, void *s, void *t, in
     if (nf <= 0) return nf == 0 ? 0 : GFSDC_EINVAL;
     int rc = work_alloc(work, plan, 2 * nf);
     if (rc) return rc;
-    size_t ng = (size_t)plan.nlat * plan.nlon;
-    if ((rc = ensure_stage(2, 2 * nf * ng * sizeof(T)))) return rc;
-    T *both = (T *)stage[2];
-    const T *in;
-    if ((rc = input(u, nf * ng, dtype, loc, 0, &in))) return rc;
-    GFSDC_CHECK(hipMemcpyAsync(both, in, nf * ng * sizeof(T), hipMemcpyDeviceToDevice, stream));
-    if ((rc = input(v, nf * ng, dtype, loc, 0, &in))) return rc;
-    GFSDC_CHECK(hipMemcpyAsync(both + nf * ng, in, nf * ng * sizeof(T), hipMemcpyDeviceToDevice, stream));
-    std::vector<AnalDesc> ad(2 * nf);
-    for (int f = 0; f < nf; f++) {
-        ad[f] = AnalDesc{AK_VRT, f, nf + f, 1.0, inv, 0, -1, 0.0};
-        ad[nf + f] = AnalDesc{AK_DIV, f, nf + f, 1.0, inv, 0, -1, 0.0};
-    }
-    if ((rc = upload_descs({}, ad, std::vector<unsigned char>(2 * nf, 1)))) return rc;
-    launch_fft_anal(plan, both, (long)ng, 2 * nf, d_rflag, work.fa, work.ldc, stream);
+    const size_t ng = (size_t)plan.nlat * plan.nlon, ns = (size_t)nf * plan.nlm * 2;
+    const T *iu, *iv;
+    if ((rc = input(u, nf * ng, dtype, loc, 0, &iu))) return rc;
+    if ((rc = input(v, nf * ng, dtype, loc, 2, &iv))) return rc;
+    launch_fft_anal(plan, iu, (long)ng, 2 * nf, nullptr, work.fa, work.ldc, stream, nullptr,
+                    FftOpt<const T>{iv, nf, 1});
     launch_leg_anal(plan, work.fa, work.ldc, work.sx, work.ldc, 4 * nf, stream);
-    T *out = work.grid;
-    launch_anal_scatter(plan, work.sx, work.ldc, d_adesc, 2 * nf, (cplx<T> *)out, plan.nlm, 1, rsphere, stream);
+    T *os = direct<T>(s, dtype, loc, false), *ot = direct<T>(t, dtype, loc, false);
+    const bool dir = os && ot;
+    if (!dir) {
+        os = work.grid;
+        ot = work.grid + ns;
+    }
+    launch_scatter_ref_vec(plan, work.sx, work.ldc, (cplx<T> *)os, (cplx<T> *)ot, nf, rsphere, inv, stream);
     GFSDC_CHECK(hipGetLastError());
-    size_t ns = (size_t)nf * plan.nlm * 2;
-    if ((rc = output(out, s, ns, dtype, loc, 1))) return rc;
-    return output(out + ns, t, ns, dtype, loc, 1);
+    if (dir) return 0;
+    if ((rc = output(os, s, ns, dtype, loc, 1))) return rc;
+    return output(ot, t, ns, dtype, loc, 1);
 }
 
 template struct Engine<float>;

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -192,16 +193,35 @@ void launch_synth_gather(const Plan<T> &p, const cplx<T> *src, long sf, long sk,
 template <typename T>
 void launch_leg_synth(const Plan<T> &p, const T *sx, int ldx, T *fs, int ldf, int ncol, hipStream_t s,
                       const int *nfdyn = nullptr);
+// gather and scatter of caller fields in the reference layout [field][nlm] (see
+// k_gather_ref); qs may be null (a zero S)
+template <typename T>
+void launch_gather_ref(const Plan<T> &p, const cplx<T> *q, int nf, T *sx, int ldx, hipStream_t s);
+template <typename T>
+void launch_gather_ref_vec(const Plan<T> &p, const cplx<T> *qs, const cplx<T> *qt, int np, T *sx, int ldx, double sa,
+                           int inva, double sb, int invb, hipStream_t s);
+template <typename T>
+void launch_scatter_ref(const Plan<T> &p, const T *sx, int ldx, cplx<T> *q, int nf, hipStream_t s);
+template <typename T>
+void launch_scatter_ref_vec(const Plan<T> &p, const T *sx, int ldx, cplx<T> *qv, cplx<T> *qd, int np, double rsphere,
+                            int inv, hipStream_t s);
+// Grid fields of a Fourier transform in two buffers: fields >= nsplit are those
+// of second, from its start. rall is every field's 1/cos flag where no array
+// of flags is given.
+template <typename T> struct FftOpt {
+    T *second = nullptr;
+    int nsplit = INT_MAX, rall = 0;
+};
 // fmap (with rdx = 1 / a for its x-gradients) maps the grid fields to the
 // Legendre fields they read; the mean is indexed by the Legendre field
 template <typename T>
 void launch_fft_synth(const Plan<T> &p, const T *fs, int ldf, T *grid, long gstride, int nf,
                       const unsigned char *rcos_flag, hipStream_t s, const T *mean = nullptr,
                       const int *slot = nullptr, int fofs = 0, const int *nfdyn = nullptr,
-                      const FieldMap *fmap = nullptr, double rdx = 0.0);
+                      const FieldMap *fmap = nullptr, double rdx = 0.0, const FftOpt<T> &o = {});
 template <typename T>
 void launch_fft_anal(const Plan<T> &p, const T *grid, long gstride, int nf, const unsigned char *rcos_flag,
-                     T *fa, int ldf, hipStream_t s, const int *nfdyn = nullptr);
+                     T *fa, int ldf, hipStream_t s, const int *nfdyn = nullptr, const FftOpt<const T> &o = {});
 template <typename T>
 void launch_leg_anal(const Plan<T> &p, const T *fa, int ldf, T *sx, int ldx, int ncol, hipStream_t s,
                      const int *nfdyn = nullptr);

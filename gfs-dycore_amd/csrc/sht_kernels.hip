@@ -14,6 +14,7 @@
 #include <climits>
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "gfsdc_internal.h"
 
@@ -1013,7 +1014,7 @@ __host__ __device__ constexpr int fft_threads(int nfft, int nc) { return fft_wav
 
 template <typename T, int NFFT, int MAXN, int NC>
 __global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_synth(const T *__restrict__ fs, int ldf, T *__restrict__ grid,
-                                                   long gstride, int nf, const unsigned char *__restrict__ rflag,
+                                                   T *__restrict__ grid2, int nsplit, long gstride, int nf, const unsigned char *__restrict__ rflag, int rall,
                                                    const T *__restrict__ mean, const int *__restrict__ slot,
                                                    const T *__restrict__ rcos, const cplx<T> *__restrict__ tw,
                                                    int nlon, int nlat, int ntrunc, Radices rd, int fofs,
@@ -1062,7 +1063,7 @@ __global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_synth(const T *__
         bool dxw;
         const int lw = lfield(tid >> 6, dxw);
         const T rc = rcos[j];  // unconditional, so that no load waits for another
-        w_s = rflag[fw] ? rc : T(1);
+        w_s = (rflag ? rflag[fw] : rall) ? rc : T(1);
         w_c = mean ? mean[lw] : T(0);
         if (dxw) w_c = T(0);
         w_g = slot ? slot[fw] : fw;
@@ -1131,7 +1132,8 @@ __global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_synth(const T *__
         if (f >= nf) return;
         const T s = w_s, c = w_c;
         const long gf = w_g;  // grid field the transform is written to
-        T *gn = grid + gf * gstride + (long)j * nlon, *gs = grid + gf * gstride + (long)j2 * nlon;
+        T *go = gf < nsplit ? grid + gf * gstride : grid2 + (gf - nsplit) * gstride;
+        T *gn = go + (long)j * nlon, *gs = go + (long)j2 * nlon;
         auto none = [](int, int) { return cplx<T>{T(0), T(0)}; };
         constexpr RadPlan P = rad_plan(NC);
         if constexpr (QUADL) {
@@ -1193,10 +1195,11 @@ __global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_synth(const T *__
         if (f >= nf) break;
         bool dxf;
         const int lf = lfield(q, dxf);  // the mean belongs to the Legendre field; an x-gradient has none
-        const T s = rflag[f] ? rc : T(1);
+        const T s = (rflag ? rflag[f] : rall) ? rc : T(1);
         const T c = (mean && !dxf) ? mean[lf] : T(0);
         const long gf = slot ? slot[f] : f;  // grid field the transform is written to
-        T *gn = grid + gf * gstride + (long)j * nlon, *gs = grid + gf * gstride + (long)j2 * nlon;
+        T *go = gf < nsplit ? grid + gf * gstride : grid2 + (gf - nsplit) * gstride;
+        T *gn = go + (long)j * nlon, *gs = go + (long)j2 * nlon;
         const cplx<T> *bq = buf + q * NP;
         for (int i = tid; i < N; i += 256) {
             const cplx<T> z = bq[fft_pad(i)];
@@ -1209,8 +1212,9 @@ __global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_synth(const T *__
 // Fourier analysis: rows of a latitude pair -> weighted symmetric / antisymmetric
 // Fourier coefficients, m = 0..T. Grid rows are loaded in one batch per thread.
 template <typename T, int NFFT, int MAXN, int NC>
-__global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_anal(const T *__restrict__ grid, long gstride, int nf,
-                                                  const unsigned char *__restrict__ rflag,
+__global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_anal(const T *__restrict__ grid,
+                                                  const T *__restrict__ grid2, int nsplit, long gstride, int nf,
+                                                  const unsigned char *__restrict__ rflag, int rall,
                                                   const T *__restrict__ rcos, const T *__restrict__ wfac,
                                                   const cplx<T> *__restrict__ tw, T *__restrict__ fa, int ldf,
                                                   int nlon, int nlat, int nhp, int ntrunc, Radices rd,
@@ -1233,7 +1237,8 @@ __global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_anal(const T *__r
         // a field past nf repeats field nf - 1 and is not stored
         constexpr RadPlan P = rad_plan(NC);
         const int q = tid >> 6, f = min(f0 + q, nf - 1);
-        const T *gn = grid + f * gstride + (long)j * nlon, *gs = grid + f * gstride + (long)j2 * nlon;
+        const T *gi = f < nsplit ? grid + f * gstride : grid2 + (f - nsplit) * gstride;
+        const T *gn = gi + (long)j * nlon, *gs = gi + (long)j2 * nlon;
         cplx<T> *bq = buf + q * NP;
         if constexpr (!GTW)
             for (int t = tid; t < N; t += NT) tws[t] = tw[t];
@@ -1264,8 +1269,9 @@ __global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_anal(const T *__r
             if (t < NFFT * N) {
                 int q = t / N, i = t - q * N, f = f0 + q;
                 if (f < nf) {
-                    xv[c] = grid[f * gstride + (long)j * nlon + i];
-                    yv[c] = grid[f * gstride + (long)j2 * nlon + i];
+                    const T *gi = f < nsplit ? grid + f * gstride : grid2 + (f - nsplit) * gstride;
+                    xv[c] = gi[(long)j * nlon + i];
+                    yv[c] = gi[(long)j2 * nlon + i];
                 }
             }
         }
@@ -1288,7 +1294,7 @@ __global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_anal(const T *__r
     // its weight is formed once
     static_assert(NT % NFFT == 0, "output field per thread");
     const int qo = tid % NFFT, fo = f0 + qo;
-    const T wf = rflag[min(fo, nf - 1)] ? wf_j * rc_j : wf_j;
+    const T wf = (rflag ? rflag[min(fo, nf - 1)] : rall) ? wf_j * rc_j : wf_j;
     for (int idx = tid; idx < (ntrunc + 1) * NFFT; idx += NT) {
         int m = idx / NFFT, q = qo, f = fo;
         if (f >= nf) continue;
@@ -1299,6 +1305,167 @@ __global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_anal(const T *__r
         T *po = fa + ((long)(2 * m + 1) * nhp + jp) * ldf + 2 * f;
         *(cplx<T> *)pe = cplx<T>{wf * (xr + yr), wf * (xi + yi)};
         *(cplx<T> *)po = cplx<T>{wf * (xr - yr), wf * (xi - yi)};
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Gather and scatter for caller fields in the reference layout, q[field][k] with
+// the coefficients contiguous. The work columns have the fields contiguous, so
+// both transpose a tile of REF_K extended coefficients x REF_F fields through
+// LDS: global accesses are runs of 64 coefficients on the caller's side and of
+// 32 (FP64: 16) fields, 256 bytes, on the work side. The general kernels below
+// read such fields with a stride of a whole field between lanes: 256 fields at
+// T254 in FP32 (67 MB in, 67 MB out) took 57 us to gather and 73 us to scatter.
+// What to do is the same for every field of a call, so there are no descriptors
+// to upload either. Fields f < nsplit are in the first buffer, the others in
+// the second (f - nsplit). Extended coefficient ke = (m, n <= T + 1) is
+// coefficient k = ke - m of a field, for n <= T.
+constexpr int REF_K = 64;
+template <typename T> constexpr int REF_F = sizeof(T) == 4 ? 32 : 16;
+template <typename T> constexpr int REF_P = REF_K + 3;  // LDS pitch of a field: odd, with a halo row on either side
+
+// VEC = false: sx column f = field f. VEC = true: the S and T of pair f are
+// field f of the first and of the second buffer (the first may be null: S = 0);
+// with the multipliers sa, sb and, where inv is set, the inverse Laplacian,
+// column f = U = (n-1) eps_n S_{n-1} - (n+2) eps_{n+1} S_{n+1} + i m T_n and
+// column np + f = V = i m S_n - (n-1) eps_n T_{n-1} + (n+2) eps_{n+1} T_{n+1}.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void k_gather_ref(const cplx<T> *__restrict__ qa, const cplx<T> *__restrict__ qb,
+                                                    int np, T *__restrict__ sx, int ldx,
+                                                    const int2 *__restrict__ kemn, const T *__restrict__ eps,
+                                                    const int *__restrict__ eoff, int ntrunc, int nlm, int nke, T sa,
+                                                    T sb, int inva, int invb) {
+    constexpr int F = REF_F<T>, P = REF_P<T>, NA = VEC ? 2 : 1, R = REF_K + 2;
+    __shared__ cplx<T> buf[NA][F][P];  // row r: ke0 - 1 + r, the first and the last for the recurrences only
+    __shared__ T cm[REF_K], cp[REF_K];
+    __shared__ int2 nm[REF_K];
+    const int tid = threadIdx.x, ke0 = blockIdx.y * REF_K, f0 = blockIdx.x * F, nf = min(F, np - f0);
+    const int lane = tid & 63, w = tid >> 6;
+    // N coefficients of one row, of fields f, f + step, ..: all loads first (fields
+    // clamped into the tile, a row of degree T + 1 to its neighbour and zeroed)
+    auto load = [&](int row, int f, int step, auto N) {
+        const int ke = ke0 - 1 + row;
+        if (ke < 0 || ke >= nke) return;
+        const int2 mn = kemn[ke];
+        const bool ok = mn.y <= ntrunc;
+        const long o = (long)f0 * nlm + ke - mn.x - (ok ? 0 : 1);
+        cplx<T> a[N()], b[N()];
+#pragma unroll
+        for (int i = 0; i < N(); i++) {
+            const long of = o + (long)min(f + i * step, nf - 1) * nlm;
+            if constexpr (VEC) {
+                a[i] = qa ? qa[of] : cplx<T>{T(0), T(0)};
+                b[i] = qb[of];
+            } else {
+                a[i] = qa[of];
+            }
+        }
+        T ca = sa, cb = sb;
+        if constexpr (VEC) {
+            const T il = (mn.y == 0) ? T(0) : T(-1.0 / ((double)mn.y * (mn.y + 1.0)));
+            if (inva) ca *= il;
+            if (invb) cb *= il;
+        }
+#pragma unroll
+        for (int i = 0; i < N(); i++) {
+            const int fi = f + i * step;
+            if (fi >= nf) break;
+            const cplx<T> z{T(0), T(0)};
+            if constexpr (VEC) {
+                buf[0][fi][row] = ok ? cplx<T>{a[i].x * ca, a[i].y * ca} : z;
+                buf[1][fi][row] = ok ? cplx<T>{b[i].x * cb, b[i].y * cb} : z;
+            } else {
+                buf[0][fi][row] = ok ? a[i] : z;
+            }
+        }
+    };
+    load(lane + 1, w, 4, std::integral_constant<int, F / 4>());
+    if constexpr (VEC) {
+        if (tid < 2 * nf) load(tid < nf ? 0 : R - 1, tid < nf ? tid : tid - nf, 1, std::integral_constant<int, 1>());
+        if (tid < REF_K && ke0 + tid < nke) {
+            const int2 mn = kemn[ke0 + tid];
+            const T *ep = eps + eoff[mn.x] + mn.y - mn.x;
+            nm[tid] = mn;
+            cm[tid] = T(mn.y - 1) * ep[0];
+            cp[tid] = T(mn.y + 2) * ep[1];
+        }
+    }
+    __syncthreads();
+    const int f = tid % F;
+    if (f >= nf) return;
+    for (int r = tid / F; r < REF_K && ke0 + r < nke; r += 256 / F) {
+        T *o = sx + (long)(ke0 + r) * ldx + 2 * (f0 + f);
+        if constexpr (!VEC) {
+            *(cplx<T> *)o = buf[0][f][r + 1];
+        } else {
+            const cplx<T> s = buf[0][f][r + 1], t = buf[1][f][r + 1];
+            const int2 mn = nm[r];
+            const T c1 = cm[r], c2 = cp[r], m = T(mn.x);
+            // degrees m - 1 and above T have no coefficient
+            const bool lo = mn.y > mn.x, hi = mn.y < ntrunc;
+            const cplx<T> z{T(0), T(0)};
+            const cplx<T> sl = lo ? buf[0][f][r] : z, tl = lo ? buf[1][f][r] : z;
+            const cplx<T> sh = hi ? buf[0][f][r + 2] : z, th = hi ? buf[1][f][r + 2] : z;
+            *(cplx<T> *)o = cplx<T>{c1 * sl.x - c2 * sh.x - m * t.y, c1 * sl.y - c2 * sh.y + m * t.x};
+            *(cplx<T> *)(o + 2 * np) = cplx<T>{-m * s.y - c1 * tl.x + c2 * th.x, m * s.x - c1 * tl.y + c2 * th.y};
+        }
+    }
+}
+
+// VEC = false: field f = column f. VEC = true, with U and V the columns f and
+// np + f: vorticity and divergence of pair f into the first and second buffer,
+//   vrt = (i m V_n - n eps_{n+1} U_{n+1} + (n+1) eps_n U_{n-1}) / a
+//   div = (i m U_n + n eps_{n+1} V_{n+1} - (n+1) eps_n V_{n-1}) / a,
+// times the inverse Laplacian where inv is set.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void k_scatter_ref(const T *__restrict__ sx, int ldx, cplx<T> *__restrict__ qa,
+                                                     cplx<T> *__restrict__ qb, int np, const int2 *__restrict__ kemn,
+                                                     const T *__restrict__ eps, const int *__restrict__ eoff,
+                                                     int ntrunc, int nlm, int nke, T rrs, int inv) {
+    constexpr int F = REF_F<T>, P = REF_P<T>, NA = VEC ? 2 : 1, R = REF_K + 2;
+    __shared__ cplx<T> buf[NA][F][P];
+    const int tid = threadIdx.x, ke0 = blockIdx.y * REF_K, f0 = blockIdx.x * F, nf = min(F, np - f0);
+    const int fl = tid % F;
+    if (fl < nf) {
+        constexpr int RPT = (R * F + 255) / 256;
+#pragma unroll
+        for (int i = 0; i < RPT; i++) {
+            const int row = tid / F + i * (256 / F), ke = ke0 - 1 + row;
+            if (row < R && ke >= 0 && ke < nke) {
+                const T *X = sx + (long)ke * ldx + 2 * (f0 + fl);
+                buf[0][fl][row] = *(const cplx<T> *)X;
+                if constexpr (VEC) buf[1][fl][row] = *(const cplx<T> *)(X + 2 * np);
+            }
+        }
+    }
+    __syncthreads();
+    const int r = (tid & 63) + 1, ke = ke0 - 1 + r;
+    if (ke >= nke) return;
+    const int2 mn = kemn[ke];
+    const int m = mn.x, n = mn.y;
+    if (n > ntrunc) return;
+    T cp = T(0), cm = T(0), il = T(1);
+    if constexpr (VEC) {
+        const T *ep = eps + eoff[m] + n - m;
+        cm = T(n + 1) * ep[0];
+        cp = T(n) * ep[1];
+        if (inv) il = (n == 0) ? T(0) : T(-1.0 / ((double)n * (n + 1.0)));
+    }
+    const T fm = T(m);
+    for (int f = tid >> 6; f < nf; f += 4) {
+        const long o = (long)(f0 + f) * nlm + ke - m;
+        if constexpr (!VEC) {
+            qa[o] = buf[0][f][r];
+        } else {
+            const cplx<T> u = buf[0][f][r], v = buf[1][f][r], uh = buf[0][f][r + 1], vh = buf[1][f][r + 1];
+            cplx<T> ul{T(0), T(0)}, vl = ul;
+            if (n > m) {
+                ul = buf[0][f][r - 1];
+                vl = buf[1][f][r - 1];
+            }
+            qa[o] = cplx<T>{il * ((-fm * v.y - (cp * uh.x - cm * ul.x)) * rrs), il * ((fm * v.x - (cp * uh.y - cm * ul.y)) * rrs)};
+            qb[o] = cplx<T>{il * ((-fm * u.y + (cp * vh.x - cm * vl.x)) * rrs), il * ((fm * u.x + (cp * vh.y - cm * vl.y)) * rrs)};
+        }
     }
 }
 
@@ -1698,6 +1865,36 @@ void launch_synth_gather(const Plan<T> &p, const cplx<T> *src, long sf, long sk,
                        p.eps, p.eoff, p.ntrunc, p.nlme, mean, nfdyn);
 }
 
+template <typename T> static dim3 ref_grid(const Plan<T> &p, int nf) {
+    return dim3((nf + REF_F<T> - 1) / REF_F<T>, (p.nlme + REF_K - 1) / REF_K);
+}
+
+template <typename T>
+void launch_gather_ref(const Plan<T> &p, const cplx<T> *q, int nf, T *sx, int ldx, hipStream_t s) {
+    hipLaunchKernelGGL((k_gather_ref<T, false>), ref_grid(p, nf), dim3(256), 0, s, q, (const cplx<T> *)nullptr, nf, sx,
+                       ldx, p.kemn, p.eps, p.eoff, p.ntrunc, p.nlm, p.nlme, T(1), T(1), 0, 0);
+}
+
+template <typename T>
+void launch_gather_ref_vec(const Plan<T> &p, const cplx<T> *qs, const cplx<T> *qt, int np, T *sx, int ldx, double sa,
+                           int inva, double sb, int invb, hipStream_t s) {
+    hipLaunchKernelGGL((k_gather_ref<T, true>), ref_grid(p, np), dim3(256), 0, s, qs, qt, np, sx, ldx, p.kemn, p.eps,
+                       p.eoff, p.ntrunc, p.nlm, p.nlme, (T)sa, (T)sb, inva, invb);
+}
+
+template <typename T>
+void launch_scatter_ref(const Plan<T> &p, const T *sx, int ldx, cplx<T> *q, int nf, hipStream_t s) {
+    hipLaunchKernelGGL((k_scatter_ref<T, false>), ref_grid(p, nf), dim3(256), 0, s, sx, ldx, q, (cplx<T> *)nullptr, nf,
+                       p.kemn, p.eps, p.eoff, p.ntrunc, p.nlm, p.nlme, T(1), 0);
+}
+
+template <typename T>
+void launch_scatter_ref_vec(const Plan<T> &p, const T *sx, int ldx, cplx<T> *qv, cplx<T> *qd, int np, double rsphere,
+                            int inv, hipStream_t s) {
+    hipLaunchKernelGGL((k_scatter_ref<T, true>), ref_grid(p, np), dim3(256), 0, s, sx, ldx, qv, qd, np, p.kemn, p.eps,
+                       p.eoff, p.ntrunc, p.nlm, p.nlme, (T)(1.0 / rsphere), inv);
+}
+
 // The BF16x3 Legendre kernels take no device field count: they transform every
 // column of the launch (the columns past it hold earlier data and are not read).
 template <typename T>
@@ -1740,12 +1937,12 @@ static Radices radices_of(int n, const int *r) {
 template <typename T, int NF>
 static void fft_synth_nf(const Plan<T> &p, const T *fs, int ldf, T *grid, long gstride, int nf,
                          const unsigned char *rflag, const T *mean, const int *slot, int fofs, hipStream_t s,
-                         const int *nfdyn, const FieldMap &fmap, T rdx) {
+                         const int *nfdyn, const FieldMap &fmap, T rdx, const FftOpt<T> &o) {
     constexpr int MN = FftCfg<T>::MAXN;
     dim3 g(p.nhalf * ((nf + NF - 1) / NF));
 #define FFT_SYN(NC)                                                                                             \
-    hipLaunchKernelGGL((k_fft_synth<T, NF, MN, NC>), g, dim3(fft_threads(NF, NC)), 0, s, fs, ldf, grid, gstride, nf,   \
-                       rflag, mean, slot,                                                                     \
+    hipLaunchKernelGGL((k_fft_synth<T, NF, MN, NC>), g, dim3(fft_threads(NF, NC)), 0, s, fs, ldf, grid, o.second, o.nsplit, gstride, nf,   \
+                       rflag, o.rall, mean, slot,                                                                     \
                        p.rcos, (const cplx<T> *)p.tw, p.nlon, p.nlat, p.ntrunc, radices_of(p.nrad, p.rad), fofs, \
                        nfdyn, fmap, rdx)
     switch (p.nlon) {
@@ -1759,11 +1956,11 @@ static void fft_synth_nf(const Plan<T> &p, const T *fs, int ldf, T *grid, long g
 
 template <typename T, int NF>
 static void fft_anal_nf(const Plan<T> &p, const T *grid, long gstride, int nf, const unsigned char *rflag, T *fa,
-                        int ldf, hipStream_t s, const int *nfdyn) {
+                        int ldf, hipStream_t s, const int *nfdyn, const FftOpt<const T> &o) {
     constexpr int MN = FftCfg<T>::MAXN;
     dim3 g(p.nhalf * ((nf + NF - 1) / NF));
 #define FFT_ANA(NC)                                                                                             \
-    hipLaunchKernelGGL((k_fft_anal<T, NF, MN, NC>), g, dim3(fft_threads(NF, NC)), 0, s, grid, gstride, nf, rflag,    \
+    hipLaunchKernelGGL((k_fft_anal<T, NF, MN, NC>), g, dim3(fft_threads(NF, NC)), 0, s, grid, o.second, o.nsplit, gstride, nf, rflag, o.rall, \
                        p.rcos, p.wfac,                                                                        \
                        (const cplx<T> *)p.tw, fa, ldf, p.nlon, p.nlat, p.nhp, p.ntrunc, radices_of(p.nrad, p.rad), \
                        nfdyn)
@@ -1783,22 +1980,22 @@ static void fft_anal_nf(const Plan<T> &p, const T *grid, long gstride, int nf, c
 template <typename T>
 void launch_fft_synth(const Plan<T> &p, const T *fs, int ldf, T *grid, long gstride, int nf,
                       const unsigned char *rflag, hipStream_t s, const T *mean, const int *slot, int fofs,
-                      const int *nfdyn, const FieldMap *fmap, double rdx) {
+                      const int *nfdyn, const FieldMap *fmap, double rdx, const FftOpt<T> &o) {
     const FieldMap id{}, &fm = fmap ? *fmap : id;
     switch (p.fft_nf) {
-    case 2: fft_synth_nf<T, 2>(p, fs, ldf, grid, gstride, nf, rflag, mean, slot, fofs, s, nfdyn, fm, (T)rdx); break;
-    case 4: fft_synth_nf<T, 4>(p, fs, ldf, grid, gstride, nf, rflag, mean, slot, fofs, s, nfdyn, fm, (T)rdx); break;
-    default: fft_synth_nf<T, 8>(p, fs, ldf, grid, gstride, nf, rflag, mean, slot, fofs, s, nfdyn, fm, (T)rdx); break;
+    case 2: fft_synth_nf<T, 2>(p, fs, ldf, grid, gstride, nf, rflag, mean, slot, fofs, s, nfdyn, fm, (T)rdx, o); break;
+    case 4: fft_synth_nf<T, 4>(p, fs, ldf, grid, gstride, nf, rflag, mean, slot, fofs, s, nfdyn, fm, (T)rdx, o); break;
+    default: fft_synth_nf<T, 8>(p, fs, ldf, grid, gstride, nf, rflag, mean, slot, fofs, s, nfdyn, fm, (T)rdx, o); break;
     }
 }
 
 template <typename T>
 void launch_fft_anal(const Plan<T> &p, const T *grid, long gstride, int nf, const unsigned char *rflag, T *fa,
-                     int ldf, hipStream_t s, const int *nfdyn) {
+                     int ldf, hipStream_t s, const int *nfdyn, const FftOpt<const T> &o) {
     switch (p.fft_nf_an) {
-    case 2: fft_anal_nf<T, 2>(p, grid, gstride, nf, rflag, fa, ldf, s, nfdyn); break;
-    case 4: fft_anal_nf<T, 4>(p, grid, gstride, nf, rflag, fa, ldf, s, nfdyn); break;
-    default: fft_anal_nf<T, 8>(p, grid, gstride, nf, rflag, fa, ldf, s, nfdyn); break;
+    case 2: fft_anal_nf<T, 2>(p, grid, gstride, nf, rflag, fa, ldf, s, nfdyn, o); break;
+    case 4: fft_anal_nf<T, 4>(p, grid, gstride, nf, rflag, fa, ldf, s, nfdyn, o); break;
+    default: fft_anal_nf<T, 8>(p, grid, gstride, nf, rflag, fa, ldf, s, nfdyn, o); break;
     }
 }
 
@@ -1819,14 +2016,20 @@ void launch_anal_scatter(const Plan<T> &p, const T *sx, int ldx, const AnalDesc 
     template void work_free<T>(Work<T> &);                                                                     \
     template void launch_synth_gather<T>(const Plan<T> &, const cplx<T> *, long, long, const SynthDesc *, int,  \
                                          T *, int, double, hipStream_t, T *, const int *);                     \
+    template void launch_gather_ref<T>(const Plan<T> &, const cplx<T> *, int, T *, int, hipStream_t);          \
+    template void launch_gather_ref_vec<T>(const Plan<T> &, const cplx<T> *, const cplx<T> *, int, T *, int,   \
+                                           double, int, double, int, hipStream_t);                             \
+    template void launch_scatter_ref<T>(const Plan<T> &, const T *, int, cplx<T> *, int, hipStream_t);         \
+    template void launch_scatter_ref_vec<T>(const Plan<T> &, const T *, int, cplx<T> *, cplx<T> *, int, double, \
+                                            int, hipStream_t);                                                 \
     template void launch_leg_synth<T>(const Plan<T> &, const T *, int, T *, int, int, hipStream_t,             \
                                       const int *);                                                            \
     template void launch_leg_anal<T>(const Plan<T> &, const T *, int, T *, int, int, hipStream_t, const int *); \
     template void launch_fft_synth<T>(const Plan<T> &, const T *, int, T *, long, int, const unsigned char *,  \
                                       hipStream_t, const T *, const int *, int, const int *, const FieldMap *, \
-                                      double);                                                                 \
+                                      double, const FftOpt<T> &);                                                                 \
     template void launch_fft_anal<T>(const Plan<T> &, const T *, long, int, const unsigned char *, T *, int,   \
-                                     hipStream_t, const int *);                                                \
+                                     hipStream_t, const int *, const FftOpt<const T> &);                                             \
     template void launch_anal_scatter<T>(const Plan<T> &, const T *, int, const AnalDesc *, int, cplx<T> *,    \
                                          long, long, double, hipStream_t, const int *, bool);
 INST(float)

@@ -1,5 +1,7 @@
 """Kernels at the sizes where their tiling can go wrong: partial tiles,
 remainders, the smallest and the largest of their range."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -30,3 +32,79 @@ def test_mlp_layout_and_gradient(nlev, hidden, nlay, batch):
     lo, go, _ = O.Mlp(g.mlp_nin, g.mlp_nout, hidden, nlay).loss_grad(p, x, t, grad=True, bf16=True)
     assert abs(loss - lo) < 1e-3 * lo
     assert np.linalg.norm(grad - go) < 6e-3 * np.linalg.norm(go)
+
+
+# every transform length with kernels of its own but the three of test_gpu_transforms, and two without (72, 162)
+GRIDS = [(64, 32, 21), (96, 48, 31), (192, 94, 62), (256, 128, 84), (288, 144, 95), (512, 256, 170), (576, 288, 190),
+         (72, 36, 23), (162, 82, 53)]
+A = 6.3712e6
+
+
+def rel(a, b):
+    return np.abs(a - b).max() / np.abs(b).max()
+
+
+def device_call(g, fn, ins, outs, nf, *extra, shift=0):
+    """fn of the C ABI on device buffers of the context's own type, from the HIP runtime that libgfsdc links; each
+    output, of the shapes and types in outs, starts shift bytes past an allocation's start"""
+    import gfsdc
+    L, H = gfsdc.load(), C.CDLL("libamdhip64.so.7")
+    H.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+    H.hipFree.argtypes = [C.c_void_p]
+    H.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    ins = [np.ascontiguousarray(x) for x in ins]
+    res = [np.full(s, np.nan, t) for s, t in outs]
+    buf = []
+    try:
+        for x, off in [(x, 0) for x in ins] + [(x, shift) for x in res]:
+            p = C.c_void_p()
+            assert H.hipMalloc(C.byref(p), x.nbytes + off) == 0
+            buf.append((p, C.c_void_p(p.value + off)))
+            assert H.hipMemcpy(buf[-1][1], x.ctypes.data, x.nbytes, 1) == 0
+        dt = gfsdc.DT_F64 if g.precision == gfsdc.FP64 else gfsdc.DT_F32
+        assert getattr(L, fn)(g.h, *[q for _, q in buf], nf, *extra, dt, gfsdc.DEVICE) == 0
+        g.sync()
+        for x, (_, q) in zip(res, buf[len(ins):]):
+            assert H.hipMemcpy(x.ctypes.data, q, x.nbytes, 2) == 0
+    finally:
+        for p, _ in buf:
+            H.hipFree(p)
+    return res
+
+
+# the transposing gather and scatter hold 32 (FP64: 16) fields a tile and 64 coefficients
+@pytest.mark.parametrize("nf", [1, 33, 64])
+@pytest.mark.parametrize("grid", GRIDS, ids=lambda g: f"{g[0]}x{g[1]}")
+def test_transforms_every_length(grid, nf):
+    """Scalar and vector transforms, both directions, against the oracle at the bounds of test_gpu_transforms
+    (FP64 1e-11; FP32 2e-6 scalar, 2e-5 vector), and the same call on device buffers, aligned and off a 16-byte
+    boundary, bit for bit."""
+    import gfsdc
+    nlon, nlat, T = grid
+    o = O.Sht(nlon, nlat, T)
+    rng = np.random.default_rng(nf)
+    n = np.maximum(o.degree, 1).astype(float)
+    q = n ** -1.5 * np.exp(2j * np.pi * rng.random((2, nf, o.nlm)))
+    q[..., o.order == 0] = q[..., o.order == 0].real
+    vrt, div = 1e-5 * q[0], 1e-6 * q[1]
+    grid_o, (u0, v0), (gx0, gy0) = o.spectogrd(q[0]), o.getuv(vrt, div, A), o.getgrad(q[0], A)
+    z0, d0 = o.getvrtdivspec(u0, v0, A)
+    for prec, ts, tv in ((gfsdc.FP64, 1e-11, 1e-11), (gfsdc.FP32, 2e-6, 2e-5)):
+        g, dt = gfsdc.Context(nlon, nlat, T, prec), 0 if prec == gfsdc.FP64 else 1
+        ct, rt = (np.complex64, np.float32) if dt else (np.complex128, np.float64)
+        S, G = ((nf, o.nlm), ct), ((nf, nlat, nlon), rt)
+        a, b, w, g0, uu, vv = (x.astype(t) for x, t in ((q[0], ct), (vrt, ct), (div, ct), (grid_o, rt), (u0, rt), (v0, rt)))
+        scale = max(np.abs(z0).max(), np.abs(d0).max())
+        for fn, ins, outs, ref, host, tol in (
+                ("gfsdc_spectogrd", [a], [G], [grid_o], [g.spectogrd(a, dt)], ts),
+                ("gfsdc_grdtospec", [g0], [S], [o.grdtospec(grid_o)], [g.grdtospec(g0, dt)], ts),
+                ("gfsdc_getuv", [b, w], [G, G], [u0, v0], g.getuv(b, w, A, dt), tv),
+                ("gfsdc_getgrad", [a], [G, G], [gx0, gy0], g.getgrad(a, A, dt), tv),
+                ("gfsdc_getvrtdivspec", [uu, vv], [S, S], [z0, d0], g.getvrtdivspec(uu, vv, A, dt), tv)):
+            for r, h in zip(ref, host):
+                s = scale if fn == "gfsdc_getvrtdivspec" else np.abs(r).max()
+                assert np.abs(h - r).max() < tol * s, (fn, prec, np.abs(h - r).max() / s)
+            extra = () if fn in ("gfsdc_spectogrd", "gfsdc_grdtospec") else (C.c_double(A),)
+            for shift in (0, rt().itemsize):
+                for x, h in zip(device_call(g, fn, ins, outs, nf, *extra, shift=shift), host):
+                    assert np.array_equal(x, h), (fn, prec, shift)
