@@ -996,9 +996,16 @@ __device__ __forceinline__ void fft_stages(cplx<T> *buf, const cplx<T> *tw, int 
 }
 
 
-template <typename T> struct FftCfg;
-template <> struct FftCfg<float> { static constexpr int NFFT = 4, MAXN = 768; };
-template <> struct FftCfg<double> { static constexpr int NFFT = 4, MAXN = 768; };
+// Fields per workgroup unless the autotuner or GFSDC_FFT_NF chooses: 4, but 8
+// for the FP32 transforms of 512 and 768 points, whose last stage runs quads of
+// butterflies (256 fields, synthesis + analysis: 768 points 290 us with 4 and
+// 246 us with 8, 512 points 114 and 110 us). At 576 points (144 and 150 us), at
+// 384 and below (equal to 2 %) and in FP64 (768 points 492 and 543 us: the LDS
+// of 8 fields leaves one workgroup per CU) 4 is as fast or faster.
+template <typename T> struct FftCfg {
+    static constexpr int MAXN = 768;
+    static constexpr int nfft(int nlon) { return sizeof(T) == 4 && (nlon == 512 || nlon == 768) ? 8 : 4; }
+};
 static_assert(fft_pitch(FftCfg<double>::MAXN) * 8 * 16 + FftCfg<double>::MAXN * 16 <= 160 * 1024, "FFT LDS budget");
 
 // Fourier synthesis: one workgroup per latitude pair and NFFT fields. The
@@ -1705,7 +1712,7 @@ template <typename T> int plan_create(Plan<T> &p, int nlon, int nlat, int ntrunc
     p.nlme = p.nlm + ntrunc + 1;
     p.nrad = rd.n;
     for (int i = 0; i < rd.n; i++) p.rad[i] = rd.r[i];
-    p.fft_nf = FftCfg<T>::NFFT;
+    p.fft_nf = FftCfg<T>::nfft(nlon);
     if (const char *e = getenv("GFSDC_FFT_NF")) {
         int v = atoi(e);
         if (v == 2 || v == 4 || v == 8) p.fft_nf = v;
@@ -1945,6 +1952,19 @@ static void fft_synth_nf(const Plan<T> &p, const T *fs, int ldf, T *grid, long g
                        rflag, o.rall, mean, slot,                                                                     \
                        p.rcos, (const cplx<T> *)p.tw, p.nlon, p.nlat, p.ntrunc, radices_of(p.nrad, p.rad), fofs, \
                        nfdyn, fmap, rdx)
+    // the lengths of spectral models' grids, one wavefront per field (the general
+    // kernel, any 2^a 3^b, takes workgroup barriers and run-time divisors: 256 FP32
+    // fields at 192 points 29.0 us against 11.8, at 512 points 101.9 against 50.4)
+    if constexpr (NF > 2)
+        switch (p.nlon) {
+        case 64: FFT_SYN(64); return;
+        case 96: FFT_SYN(96); return;
+        case 192: FFT_SYN(192); return;
+        case 256: FFT_SYN(256); return;
+        case 288: FFT_SYN(288); return;
+        case 512: FFT_SYN(512); return;
+        case 576: FFT_SYN(576); return;
+        }
     switch (p.nlon) {
     case 768: FFT_SYN(768); break;
     case 384: FFT_SYN(384); break;
@@ -1964,6 +1984,16 @@ static void fft_anal_nf(const Plan<T> &p, const T *grid, long gstride, int nf, c
                        p.rcos, p.wfac,                                                                        \
                        (const cplx<T> *)p.tw, fa, ldf, p.nlon, p.nlat, p.nhp, p.ntrunc, radices_of(p.nrad, p.rad), \
                        nfdyn)
+    if constexpr (NF > 2)  // as fft_synth_nf
+        switch (p.nlon) {
+        case 64: FFT_ANA(64); return;
+        case 96: FFT_ANA(96); return;
+        case 192: FFT_ANA(192); return;
+        case 256: FFT_ANA(256); return;
+        case 288: FFT_ANA(288); return;
+        case 512: FFT_ANA(512); return;
+        case 576: FFT_ANA(576); return;
+        }
     switch (p.nlon) {
     case 768: FFT_ANA(768); break;
     case 384: FFT_ANA(384); break;

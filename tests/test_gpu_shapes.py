@@ -75,11 +75,13 @@ def device_call(g, fn, ins, outs, nf, *extra, shift=0):
 # the transposing gather and scatter hold 32 (FP64: 16) fields a tile and 64 coefficients
 @pytest.mark.parametrize("nf", [1, 33, 64])
 @pytest.mark.parametrize("grid", GRIDS, ids=lambda g: f"{g[0]}x{g[1]}")
-def test_transforms_every_length(grid, nf):
+def test_transforms_every_length(grid, nf, monkeypatch):
     """Scalar and vector transforms, both directions, against the oracle at the bounds of test_gpu_transforms
     (FP64 1e-11; FP32 2e-6 scalar, 2e-5 vector), and the same call on device buffers, aligned and off a 16-byte
-    boundary, bit for bit."""
+    boundary, bit for bit. One batch each with the default, 8 and 2 fields per Fourier workgroup."""
     import gfsdc
+    if nf > 1:
+        monkeypatch.setenv("GFSDC_FFT_NF", "8" if nf == 33 else "2")
     nlon, nlat, T = grid
     o = O.Sht(nlon, nlat, T)
     rng = np.random.default_rng(nf)
