@@ -689,6 +689,17 @@ __global__ __launch_bounds__(256) void k_leg_anal_b3(const float *__restrict__ p
 template <typename T> __device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T> b) {
     return cplx<T>{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
 }
+// a b with the products' fusing written out. Left to the compiler it differs
+// from kernel to kernel; so written, a transform rounds alike in the general
+// kernel and in one of its own length, and a length that gets a kernel of its
+// own keeps its bits. The lengths that always had one (128, 384, 768) keep
+// theirs by cmul.
+template <typename T, int N = 0> __device__ __forceinline__ cplx<T> cmul_tw(cplx<T> a, cplx<T> b) {
+    if constexpr (N == 128 || N == 384 || N == 768)
+        return cmul(a, b);
+    else
+        return cplx<T>{T(fma(a.x, b.x, -(a.y * b.y))), T(fma(a.y, b.x, a.x * b.y))};
+}
 
 template <typename T, int R> __device__ __forceinline__ void small_dft(cplx<T> *v, int sign) {
     if (R == 2) {
@@ -769,7 +780,7 @@ static_assert(split_all(768, 4, 1, true) && split_all(768, 4, 4, true) && split_
                   split_all(768, 3, 256, false),
               "the 768-point stages take the split LDS indices");
 
-template <typename T, int R, int MAXB>
+template <typename T, int R, int MAXB, int N_ = 0>
 __device__ __forceinline__ void fft_stage(cplx<T> *buf, int N, int nfft, int Ns, const cplx<T> *__restrict__ tw,
                                  int sign) {
     const int nbf = N / R, total = nbf * nfft, NP = fft_pitch(N);
@@ -794,7 +805,7 @@ __device__ __forceinline__ void fft_stage(cplx<T> *buf, int N, int nfft, int Ns,
             for (int r = 1; r < R; r++) {
                 cplx<T> t = tw[Ns - 1 + (r - 1) * Ns + jm];  // = w^(jm r tstep), stage-ordered table
                 if (sign > 0) t.y = -t.y;
-                v[bb][r] = cmul(v[bb][r], t);
+                v[bb][r] = cmul_tw<T, N_>(v[bb][r], t);
             }
             small_dft<T, R>(v[bb], sign);
             int idx = (j / Ns) * Ns * R + jm;
@@ -930,7 +941,7 @@ __device__ __forceinline__ void fft_stage_w(const cplx<T> *__restrict__ tw, int 
                 for (int r = 1; r < R; r++) {
                     cplx<T> t = tc.t[bb][r - 1];
                     if (sign > 0) t.y = -t.y;
-                    v[bb][r] = cmul(v[bb][r], t);
+                    v[bb][r] = cmul_tw<T, N>(v[bb][r], t);
                 }
             }
             small_dft<T, R>(v[bb], sign);
@@ -990,7 +1001,7 @@ __device__ __forceinline__ void fft_stages(cplx<T> *buf, const cplx<T> *tw, int 
     constexpr RadPlan P = rad_plan(N);
     if constexpr (S < P.n) {
         constexpr int R = P.r[S];
-        fft_stage<T, R, (NFFT * N / R + 255) / 256>(buf, N, NFFT, Ns, tw, sign);
+        fft_stage<T, R, (NFFT * N / R + 255) / 256, N>(buf, N, NFFT, Ns, tw, sign);
         fft_stages<T, NFFT, N, S + 1, Ns * R>(buf, tw, sign);
     }
 }
@@ -1162,7 +1173,7 @@ __global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_synth(const T *__
                 for (int r = 1; r < RL; r++) {
                     cplx<T> t = tl.t[bb][r - 1];
                     t.y = -t.y;  // sign +1
-                    v[bb][r] = cmul(v[bb][r], t);
+                    v[bb][r] = cmul_tw<T, NC>(v[bb][r], t);
                 }
                 small_dft<T, RL>(v[bb], +1);
             }
