@@ -65,7 +65,7 @@ struct DycoreBuffers {
     void *tphys = nullptr;                       // physics tendencies
     void *gsyn = nullptr, *gan = nullptr;        // grid fields (T)
     void *gmean = nullptr;                       // global means added back by the Fourier synthesis (nm * nsyn)
-    void *etadot = nullptr, *dlnpdt = nullptr;   // per member (nl+1)*ng (etadot less -ps bk dlnpsdt), nl*ng
+    void *etadot = nullptr, *dlnpdt = nullptr;   // per member (nl+1)*ng, nl*ng
     void *psg = nullptr, *dlnpsdt = nullptr;     // per member ng
     void *dphisdx = nullptr, *dphisdy = nullptr; // per member ng
     void *topo = nullptr;                        // spectral orography per member (complex)
@@ -219,23 +219,34 @@ static void drop_graph(DycoreBuffers *B) {
 // thickness is dp = dak + dbk ps from the FP64 differences of ak and bk (the
 // difference of the rounded interface pressures would carry their rounding,
 // amplified by p/dp).
-template <typename T> struct LayerCoef {
-    T rlnp, alfa, cofa, dbp;  // dbp = bk_K / p2 - bk_{K-1} / p1
-};
 // 1 / x: the hardware reciprocal (1 ulp) in FP32, where it feeds products and
 // never a cancellation; a division in FP64
 __device__ __forceinline__ float recip(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ double recip(double x) { return 1.0 / x; }
+// x at p + v + s bytes (v in a vector, s in a scalar register), below 4 GiB past p
+typedef unsigned bufu2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, 0xFFFFFFFFu, 0x00020000);  // raw, 32-bit data
+}
+__device__ __forceinline__ float buf_load(const float *p, unsigned v, unsigned s) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buf_rsrc(p), v, s, 0));
+}
+__device__ __forceinline__ double buf_load(const double *p, unsigned v, unsigned s) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(buf_rsrc(p), v, s, 0));
+}
+__device__ __forceinline__ void buf_store(float *p, unsigned v, unsigned s, float x) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), buf_rsrc(p), v, s, 0);
+}
+__device__ __forceinline__ void buf_store(double *p, unsigned v, unsigned s, double x) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(bufu2, x), buf_rsrc(p), v, s, 0);
+}
 template <typename T>
-__device__ inline LayerCoef<T> layer_coef(T p1, T p2, T dpk, T bk1, T bk2, T ck, T dbk) {
-    LayerCoef<T> c;
+__device__ __forceinline__ void layer_log(T p1, T p2, T dpk, T rp1, T rdp, T &rlnp, T &alfa) {
     if constexpr (sizeof(T) == 4) {
-        // hardware reciprocals (1 ulp): these feed products, never a cancellation
-        const T rp1 = __builtin_amdgcn_rcpf(p1), rp2 = __builtin_amdgcn_rcpf(p2), rdp = __builtin_amdgcn_rcpf(dpk);
         const T x = dpk * rp1;
         T y;
         if (x <= T(1)) {
-            const T u = x * __builtin_amdgcn_rcpf(T(2) + x), u2 = u * u;
+            const T u = x * recip(T(2) + x), u2 = u * u;
             y = T(2) * u *
                 (T(1) + u2 * (T(1.0 / 3.0) +
                               u2 * (T(0.2) + u2 * (T(1.0 / 7.0) + u2 * (T(1.0 / 9.0) +
@@ -244,26 +255,376 @@ __device__ inline LayerCoef<T> layer_coef(T p1, T p2, T dpk, T bk1, T bk2, T ck,
         } else {
             y = log1p(x);
         }
-        c.rlnp = y;
+        rlnp = y;
         if (y <= T(1)) {
             const T y2 = y * y;
-            c.alfa = y * T(0.5) -
-                     y2 * (T(1.0 / 12.0) -
-                           y2 * (T(1.0 / 720.0) -
-                                 y2 * (T(1.0 / 30240.0) - y2 * (T(1.0 / 1209600.0) - y2 * T(1.0 / 47900160.0)))));
+            alfa = y * T(0.5) -
+                   y2 * (T(1.0 / 12.0) -
+                         y2 * (T(1.0 / 720.0) -
+                               y2 * (T(1.0 / 30240.0) - y2 * (T(1.0 / 1209600.0) - y2 * T(1.0 / 47900160.0)))));
         } else {
-            c.alfa = T(1) - (p1 * rdp) * y;
+            alfa = T(1) - (p1 * rdp) * y;
         }
-        c.cofa = ck * rdp * (c.alfa - dpk * rp2) * rp1;
-        c.dbp = -ck * rp1 * rp2;
     } else {
-        const T rp1 = T(1) / p1, rp2 = T(1) / p2, rdp = T(1) / dpk;
-        c.rlnp = log(p2 * rp1);
-        c.alfa = T(1) - (p1 * rdp) * c.rlnp;
-        c.cofa = -rdp * (bk2 * p1 * rp2 - bk1 + c.rlnp * (bk1 - p1 * dbk * rdp));
-        c.dbp = bk2 * rp2 - bk1 * rp1;
+        rlnp = log(p2 * rp1);
+        alfa = T(1) - (p1 * rdp) * rlnp;
     }
-    return c;
+}
+// dbp = bk_K / p2 - bk_{K-1} / p1
+template <typename T>
+__device__ __forceinline__ void layer_rest(T p1, T dpk, T bk1, T bk2, T ck, T dbk, T rp1, T rp2, T rdp, T rlnp, T alfa,
+                                           T &cofa, T &dbp) {
+    if constexpr (sizeof(T) == 4) {
+        cofa = ck * rdp * (alfa - dpk * rp2) * rp1;
+        dbp = -ck * rp1 * rp2;
+    } else {
+        cofa = -rdp * (bk2 * p1 * rp2 - bk1 + rlnp * (bk1 - p1 * dbk * rdp));
+        dbp = bk2 * rp2 - bk1 * rp1;
+    }
+}
+
+// Column kernel: calc_pressdata + getomega (+ getpresgrad, getvadv, getvadv_tracers
+// and the tendency assembly unless COL_INV). A workgroup holds NC grid columns of
+// one member with the levels split over CH threads of each column, up to LPC
+// consecutive layers a thread, so that a layer's inputs are read once, all loads
+// of a thread are in flight together and the layers' terms stay in registers
+// between the two halves: first every thread forms its layers' terms and their
+// sums, then it takes the sums over the layers above (getomega's) and below
+// (getpresgrad's) it from the other threads' sums in LDS.
+// Measured in kernel traces, which start every kernel with cold caches (us a
+// launch, against one thread per column, whose bottom-up pass read u, v and the
+// divergence again): T254L64 FP32 192 from 228, 838 MB at 4.4 TB/s where a large
+// copy reaches 4.6-5.3; 16 members T126L64 664 from 827; T126L64 54 from 106, with
+// a tracer 87 from 223; T42L20 FP64 9 from 28. Whole steps: T42L20 FP64 1.17 times
+// as fast, T126L64 with a tracer 1.07, T254L64 1.05. 8 chunks of 8 layers in 128
+// registers keep two workgroups on a CU: 16 chunks of 4 took 270 at T254L64, 8
+// without the bound (141 registers, one workgroup) 258.
+// Index conventions: K counts interfaces/layers top -> bottom (1-based, as pk,
+// dpk, alfa, rlnp, etadot), L = nl + 1 - K model levels bottom -> top (as u, v, tv).
+// getomega's two running sums, of div dp and of (V . grad ln ps) dbk over the
+// layers above, appear only as s = db + ps cb: omega / p = (workc - alfa t - rlnp s) / dp
+// with the layer's own t = div dp + ps (V . grad ln ps) dbk, etadot = -s - ps bk dlnpsdt,
+// dlnpsdt = -s(surface) / ps. s is summed in FP64.
+// COL_VC adds the vorticity-confinement flux (dyn_run.f90:230-248) from the
+// vorticity gradient vcg [member][2 nl][ng] (x then y), with speed vcamp
+// times 1 + vfsvc[level] svcg (the svc pattern grid [member][ng]) when svcg is set.
+enum ColMode { COL_DYN = 0, COL_VC = 1, COL_INV = 2 };
+template <typename T> struct ColCfg { static constexpr int NC = 64, CH = 8; };
+template <> struct ColCfg<double> { static constexpr int NC = 32, CH = 16; };  // twice the registers a value
+template <typename T, int MODE, int LPC, bool TR>
+__global__ __launch_bounds__(ColCfg<T>::NC * ColCfg<T>::CH, sizeof(T) * LPC <= 16 || sizeof(T) == 4 ? 4 : 2) void k_columns(
+    const T *__restrict__ gsyn, T *__restrict__ gan, T *__restrict__ etadot, T *__restrict__ dlnpdt,
+    T *__restrict__ psg_out, T *__restrict__ dlnpsdt_out, const T *__restrict__ dphisdx,
+    const T *__restrict__ dphisdy, const T *__restrict__ ak_, const T *__restrict__ bk_,
+    const T *__restrict__ ck_, const T *__restrict__ dbk_, const T *__restrict__ dak_, const T *__restrict__ sinlat,
+    int nl, int ntr_, int nsyn, int nan, long ng, int nlon, T rd, T kappa, T cvcp, T twoom,
+    const cplx<T> *__restrict__ spec, int nfs, T *__restrict__ colq, const T *__restrict__ vcg,
+    const T *__restrict__ svcg, const T *__restrict__ vfsvc, T vcamp, int store) {
+    constexpr int NC = ColCfg<T>::NC, CH = ColCfg<T>::CH;
+    constexpr bool DYN = MODE != COL_INV, VC = MODE == COL_VC;
+    const int ntr = TR ? ntr_ : 0;  // TR: there are tracers
+    __shared__ T ak[MAXLEV + 1], bk[MAXLEV + 1], ck[MAXLEV], dbk[MAXLEV], dak[MAXLEV];
+    __shared__ double ssum[CH][NC];
+    // per chunk and column: the column tracer mass, getpresgrad's three sums, u, v
+    // and tv of the chunk's first and last layer
+    enum { S_CQ, S_COF, S_PX, S_PY, S_U0, S_V0, S_T0, S_U1, S_V1, S_T1, S_N };
+    __shared__ T sh[DYN ? S_N : S_COF][CH][NC];
+    const int tid = threadIdx.x, ln = tid % NC;
+    const int w = NC == 64 ? __builtin_amdgcn_readfirstlane(tid / NC) : tid / NC;  // chunk
+    for (int i = tid; i <= nl; i += NC * CH) {
+        ak[i] = ak_[i];
+        bk[i] = bk_[i];
+        if (i < nl) {
+            ck[i] = ck_[i];
+            dbk[i] = dbk_[i];
+            dak[i] = dak_[i];
+        }
+    }
+    const int mem = blockIdx.y, lpc = (nl + CH - 1) / CH;
+    const int K0 = w * lpc, cnt = min(max(nl - K0, 0), lpc);  // layers K0 + 1 .. K0 + cnt
+    const long c_ = (long)xcd_tile(blockIdx.x, gridDim.x) * NC + ln;  // neighbours on one XCD: ensemble 708 -> 664 us
+    const bool valid = c_ < ng;
+    const unsigned col = (unsigned)(valid ? c_ : ng - 1), cb = col * (unsigned)sizeof(T);
+    const T *G = gsyn + (long)mem * nsyn * ng;
+    const T *U = G, *V = G + (long)nl * ng, *VRT = G + 2L * nl * ng, *DIV = G + 3L * nl * ng;
+    const T *TV = G + 4L * nl * ng, *TX = G + 5L * nl * ng, *TY = G + 6L * nl * ng, *Q = G + 7L * nl * ng;
+    const T *LNPS = G + (7L + 3L * ntr) * nl * ng;
+    // this column's value at level lev = L - 1 = nl - K of a field of nl (+ 1) levels:
+    // a descriptor in scalar registers, the level's offset in one and the column's
+    // in a vector register, so that no access takes vector arithmetic
+    const unsigned lb = (unsigned)(ng * sizeof(T));
+    auto ld = [&](const T *P, int lev) { return buf_load(P, cb, (unsigned)lev * lb); };
+    auto st = [&](T *P, int lev, T x) { buf_store(P, cb, (unsigned)lev * lb, x); };
+    T u[LPC], v[LPC], dv[LPC], tv[LPC], tx[LPC], ty[LPC], vr[LPC], q1[LPC];
+#pragma unroll
+    for (int i = 0; i < LPC; i++)
+        if (i < lpc) {
+            const int lev = max(nl - (K0 + 1 + i), 0);  // clamped: past the lowest layer nothing is used
+            u[i] = ld(U, lev);
+            v[i] = ld(V, lev);
+            dv[i] = ld(DIV, lev);
+            if constexpr (DYN) {
+                tv[i] = ld(TV, lev);
+                tx[i] = ld(TX, lev);
+                ty[i] = ld(TY, lev);
+                vr[i] = ld(VRT, lev);
+                if constexpr (TR) q1[i] = ld(Q, lev);
+            }
+        }
+    const T dpx = ld(LNPS, 1), dpy = ld(LNPS, 2);
+    const double c0 = (double)spec[(long)mem * nfs + 3L * nl + (long)ntr * nl].x * 0.28209479177387814;  // 1/sqrt(4 pi)
+    const T ps = (T)exp(c0 + (double)ld(LNPS, 0));
+    const T gpx = ps * dpx, gpy = ps * dpy;
+    const T alfa1 = T(SGLF(0.69314718055994530942)), rlnp1 = T(SGLF(99999.99));
+    __syncthreads();  // the level tables
+    auto pk = [&](int K) -> T { return ak[K - 1] + bk[K - 1] * ps; };
+    auto dp = [&](int K) -> T { return fma(dbk[K - 1], ps, dak[K - 1]); };  // pk(K + 1) - pk(K), one rounding
+    // the layers' terms, bottom -> top; fx0, fy0 are the fluxes with the pressure
+    // gradient of the sums over the chunk's own layers below
+    T f = T(0), dphx = T(0), dphy = T(0);
+    if constexpr (DYN) {
+        f = twoom * sinlat[col / (unsigned)nlon];
+        dphx = dphisdx[(long)mem * ng + col];
+        dphy = dphisdy[(long)mem * ng + col];
+    }
+    T q[LPC], w1[LPC], w2[LPC], adv[LPC], fx0[LPC], fy0[LPC];
+    T cof = T(0), px = T(0), py = T(0);
+    T p2 = pk(min(K0 + cnt, nl) + 1), rp2 = recip(p2);
+#pragma unroll
+    for (int i = LPC - 1; i >= 0; i--)
+        if (i < cnt) {
+            const int K = K0 + 1 + i;
+            const T dpk = dp(K), p1 = pk(K), rp1 = recip(p1), cg = gpx * u[i] + gpy * v[i];
+            const T t = fma(cg, dbk[K - 1], dv[i] * dpk);
+            q[i] = t;
+            const T rdp = recip(dpk);
+            T rlnp = rlnp1, alfa = alfa1, cofa, dbp, cofb0, workc, workb = t;
+            if (K == 1) {
+                cofa = -rdp * (bk[1] * p1 * rp2 - bk[0] + rlnp * (bk[0] - p1 * dbk[0] * rdp));
+                dbp = T(0);  // no layer above takes it
+                cofb0 = -rdp * (alfa * dbk[0]);
+                workc = cg * dbk[0];
+                workb = dv[i] * dpk + workc * dbk[0];
+                w1[i] = T(0);
+            } else {
+                layer_log(p1, p2, dpk, rp1, rdp, rlnp, alfa);
+                layer_rest(p1, dpk, bk[K - 1], bk[K], ck[K - 1], dbk[K - 1], rp1, rp2, rdp, rlnp, alfa, cofa, dbp);
+                cofb0 = -rdp * (bk[K - 1] * rlnp + alfa * dbk[K - 1]);
+                w1[i] = rlnp * rdp;
+                workc = cg * (dbk[K - 1] + ck[K - 1] * w1[i]);
+            }
+            w2[i] = (workc - alfa * workb) * rdp;
+            if constexpr (DYN) {
+                // prsgx = c ps dpx + px - rd alfa tx - dphx, c and px with the sums below
+                const T rt = rd * tv[i], c = (cofb0 - cofa) * rt + cof, z = vr[i] + f;
+                fx0[i] = u[i] * z - (c * gpy + (py - rd * alfa * ty[i]));
+                fy0[i] = v[i] * z + (c * gpx + (px - rd * alfa * tx[i]));
+                adv[i] = -u[i] * tx[i] - v[i] * ty[i];
+                cof -= dbp * rt;
+                px -= rd * rlnp * tx[i];
+                py -= rd * rlnp * ty[i];
+            }
+            p2 = p1;
+            rp2 = rp1;
+        }
+    // s within the chunk, over the layers down to and including i
+    double sum = 0.0;
+#pragma unroll
+    for (int i = 0; i < LPC; i++)
+        if (i < cnt) {
+            sum += (double)q[i];
+            q[i] = (T)sum;
+        }
+    ssum[w][ln] = sum;
+    if constexpr (DYN) {
+        sh[S_COF][w][ln] = cof;
+        sh[S_PX][w][ln] = px;
+        sh[S_PY][w][ln] = py;
+        sh[S_U0][w][ln] = u[0];
+        sh[S_V0][w][ln] = v[0];
+        sh[S_T0][w][ln] = tv[0];
+#pragma unroll
+        for (int i = 0; i < LPC; i++)
+            if (i == cnt - 1) {
+                sh[S_U1][w][ln] = u[i];
+                sh[S_V1][w][ln] = v[i];
+                sh[S_T1][w][ln] = tv[i];
+            }
+    }
+    if (TR && colq) {
+        // column tracer mass of the dry-mass diagnostic (dyn_run.f90:138-145)
+        T s = T(0);
+        for (int i = 0; i < cnt; i++) {
+            T qs = T(0);
+            for (int nt = 0; nt < ntr; nt++) qs += ld(Q + (long)nt * nl * ng, nl - (K0 + 1 + i));
+            s += dp(K0 + 1 + i) * qs;
+        }
+        sh[S_CQ][w][ln] = s;
+    }
+    __syncthreads();
+    // s over the chunks above this one, over those and this one, over the column
+    double sa = 0.0, sb = 0.0, tot = 0.0;
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+        if (c == w) sa = tot;
+        tot += ssum[c][ln];
+        if (c == w) sb = tot;
+    }
+    const T dlnpsdt = -(T)tot / ps, ah = (T)sa, al = (T)(sa - (double)ah), bh = (T)sb;
+    if (w == 0 && valid) {
+        psg_out[(long)mem * ng + col] = ps;
+        dlnpsdt_out[(long)mem * ng + col] = dlnpsdt;
+        if (TR && colq) {
+            T s = T(0);
+            for (int c = 0; c < CH; c++) s += sh[S_CQ][c][ln];
+            colq[(long)mem * ng + col] = s;
+        }
+    }
+    if (!valid) return;
+    // s over the layers above layer i of the chunk (i = cnt: above the next chunk)
+    auto above = [&](int i) { return i == 0 ? ah : i == cnt ? bh : ah + (al + q[i > 0 ? i - 1 : 0]); };
+    // etadot at the top interface of layer i of the chunk, K = K0 + i (0 and nl: zero)
+    auto eta = [&](int i, T s) {
+        const int K = K0 + i;
+        return (K > 0 && K < nl) ? -s - (ps * bk[K]) * dlnpsdt : T(0);
+    };
+    T *ET = etadot + (long)mem * (nl + 1) * ng, *WD = dlnpdt + (long)mem * nl * ng;
+    if constexpr (!DYN) {
+#pragma unroll
+        for (int i = 0; i < LPC; i++)
+            if (i < cnt) {
+                const int K = K0 + 1 + i;
+                const T s = above(i);
+                st(WD, nl - K, w2[i] - w1[i] * s);
+                st(ET, K - 1, eta(i, s));
+                if (K == nl) st(ET, nl, T(0));
+            }
+    } else {
+        cof = px = py = T(0);
+#pragma unroll
+        for (int c = CH - 1; c > 0; c--)
+            if (c > w) {  // getpresgrad's sums over the chunks below
+                cof += sh[S_COF][c][ln];
+                px += sh[S_PX][c][ln];
+                py += sh[S_PY][c][ln];
+            }
+        const T bx = cof * gpx + (px - dphx), by = cof * gpy + (py - dphy);
+        T *A = gan + (long)mem * nan * ng;
+        T *TT = A, *FX = A + (long)nl * ng, *FY = A + 2L * nl * ng, *KE = A + 3L * nl * ng;
+        if (w == 0) A[4L * nl * ng + col] = dlnpsdt;
+        T um = T(0), vm = T(0), tm = T(0);  // the level below the chunk
+        if (K0 + cnt < nl) {
+            um = sh[S_U0][w + 1][ln];
+            vm = sh[S_V0][w + 1][ln];
+            tm = sh[S_T0][w + 1][ln];
+        }
+        T ua = T(0), va = T(0), ta = T(0);  // the level above it
+        if (w > 0) {
+            ua = sh[S_U1][w - 1][ln];
+            va = sh[S_V1][w - 1][ln];
+            ta = sh[S_T1][w - 1][ln];
+        }
+        T eb = eta(cnt, bh);  // etadot at the bottom of layer i; zero at the surface, and at the top
+#pragma unroll
+        for (int i = LPC - 1; i >= 0; i--)
+            if (i < cnt) {
+                const int K = K0 + 1 + i, lev = nl - K;
+                const T up = i > 0 ? u[i > 0 ? i - 1 : 0] : ua, vp = i > 0 ? v[i > 0 ? i - 1 : 0] : va;
+                const T tp = i > 0 ? tv[i > 0 ? i - 1 : 0] : ta;
+                const T s = above(i), ea = eta(i, s), om = w2[i] - w1[i] * s;
+                if (store) {
+                    st(WD, lev, om);
+                    st(ET, K - 1, ea);
+                    if (K == nl) st(ET, nl, T(0));
+                }
+                // getvadv for u, v, tv
+                const T h = T(0.5) * recip(dp(K)), hb = h * eb, ha = h * ea;
+                const T vu = hb * (um - u[i]) + ha * (u[i] - up);
+                const T vv = hb * (vm - v[i]) + ha * (v[i] - vp);
+                const T vt = hb * (tm - tv[i]) + ha * (tv[i] - tp);
+                T vq = kappa * om * tv[i];
+                if constexpr (TR) vq = vq / (T(1) + cvcp * q1[i]);
+                st(TT, lev, adv[i] - vt + vq);
+                T fx = fx0[i] + vv - by, fy = fy0[i] - vu + bx;
+                if constexpr (VC) {
+                    // up-gradient vorticity flux vc |vrt| grad(vrt) / |grad(vrt)|
+                    const T *VCX = vcg + (long)mem * 2 * nl * ng, *VCY = VCX + (long)nl * ng;
+                    const T gx = ld(VCX, lev), gy = ld(VCY, lev), ag = sqrt(gx * gx + gy * gy);
+                    T vcl = vcamp;
+                    if (svcg) vcl = (T(1) + vfsvc[lev] * svcg[(long)mem * ng + col]) * vcl;
+                    if (ag > T(FLT_MIN)) {
+                        const T av = fabs(ld(VRT, lev));
+                        fx += vcl * (gx / ag) * av;
+                        fy += vcl * (gy / ag) * av;
+                    }
+                }
+                st(FX, lev, fx);
+                st(FY, lev, fy);
+                st(KE, lev, T(0.5) * (u[i] * u[i] + v[i] * v[i]));
+                um = u[i];
+                vm = v[i];
+                tm = tv[i];
+                eb = ea;
+            }
+        // tracers (dyn_run.f90:279-291): horizontal advection with the synthesised
+        // gradient and the Thuburn (1993) flux-limited vertical advection of
+        // getvadv_tracers (dyn_run.f90:478-603) with layer values D_K = q at L = nl + 1 - K.
+        // Half-level values need D from two layers above to two below; a chunk
+        // recomputes that of its top interface.
+        const T *QX = Q + (long)ntr * nl * ng, *QY = QX + (long)ntr * nl * ng;
+        const T tiny = std::numeric_limits<T>::min();
+        auto guard = [&](T d) { return fabs(d) < tiny ? copysign(tiny, d) : d; };
+        for (int nt = 0; nt < ntr && cnt > 0; nt++) {
+            const T *Qn = Q + (long)nt * nl * ng, *QXn = QX + (long)nt * nl * ng, *QYn = QY + (long)nt * nl * ng;
+            T *DQ = A + (4L * nl + 1 + (long)nt * nl) * ng;
+            T D[LPC + 4], gx[LPC], gy[LPC];  // D[i] = D_{K0 - 1 + i}, clamped to the column
+#pragma unroll
+            for (int i = 0; i < LPC + 4; i++)
+                if (i < lpc + 4) D[i] = ld(Qn, nl - min(max(K0 - 1 + i, 1), nl));
+#pragma unroll
+            for (int i = 0; i < LPC; i++)
+                if (i < lpc) {
+                    const int lev = max(nl - (K0 + 1 + i), 0);
+                    gx[i] = ld(QXn, lev);
+                    gy[i] = ld(QYn, lev);
+                }
+            // dd_K, K = K0 - 1 + i: D_{K+1} - D_K, guarded; at the top and the surface from two layers
+            auto dd = [&](int i) {
+                const int K = K0 - 1 + i;
+                if (K <= 0) {
+                    const T a = D[i + 1], mx = T(2) * a - D[i + 2];
+                    return a >= T(0) ? a - fmax(T(0), mx) : a - fmin(T(0), mx);
+                }
+                if (K >= nl) {
+                    const T a = D[i], mb = T(2) * a - D[i > 0 ? i - 1 : 0];
+                    return a >= T(0) ? fmax(T(0), mb) - a : fmin(T(0), mb) - a;
+                }
+                return guard(D[i + 1] - D[i]);
+            };
+            // the value at interface K0 + i, where etadot is e
+            auto half = [&](int i, T e) {
+                const int K = K0 + i;
+                if (K <= 0) return D[i + 2];
+                if (K >= nl) return D[i + 1];
+                const T a = D[i + 1], b = D[i + 2], h = T(0.5) * (b + a), dk = dd(i + 1);
+                const T phi = (e > T(0) ? dd(i) : dd(i + 2)) / dk;
+                const T lim = (phi + fabs(phi)) / (T(1) + fabs(phi));
+                return e > T(0) ? a + lim * (h - a) : b + lim * (h - b);
+            };
+            T et = eta(0, ah), hp = half(0, et);
+#pragma unroll
+            for (int i = 0; i < LPC; i++)
+                if (i < cnt) {
+                    const int K = K0 + 1 + i;
+                    const T eb2 = eta(i + 1, above(i + 1));
+                    const T hk = half(i + 1, eb2), Dk = D[i + 2];
+                    const T vadv = recip(dp(K)) * ((hk * eb2 - hp * et) + (Dk * (et - eb2)));
+                    st(DQ, nl - K, -u[i] * gx[i] - v[i] * gy[i] - vadv);
+                    hp = hk;
+                    et = eb2;
+                }
+        }
+    }
 }
 
 // getomega's layer terms, evaluated identically wherever they are needed: with
@@ -302,22 +663,26 @@ template <typename T> struct PairSum {
     }
 };
 
-// Column kernel: calc_pressdata + getomega (+ getpresgrad, getvadv and the
-// tendency assembly unless inverse_only). One thread per grid column and member.
-// Level indices: K counts interfaces/layers top -> bottom (1-based, as pk, dpk,
-// alfa, rlnp, etadot), L counts model levels bottom -> top (as u, v, tv).
-// VC adds the vorticity-confinement flux (dyn_run.f90:230-248) from the
-// vorticity gradient vcg [member][2 nl][ng] (x then y), with speed vcamp
-// times 1 + vfsvc[level] svcg (the svc pattern grid [member][ng]) when svcg is set.
-template <typename T, bool VC = false>
-__global__ __launch_bounds__(256) void k_columns(
-    const T *__restrict__ gsyn, T *__restrict__ gan, T *__restrict__ etadot, T *__restrict__ dlnpdt,
-    T *__restrict__ psg_out, T *__restrict__ dlnpsdt_out, const T *__restrict__ dphisdx,
-    const T *__restrict__ dphisdy, const T *__restrict__ ak_, const T *__restrict__ bk_,
-    const T *__restrict__ ck_, const T *__restrict__ dbk_, const T *__restrict__ dak_, const T *__restrict__ sinlat,
-    int nl, int ntr, int nsyn, int nan, long ng, int nlon, T rd, T kappa, T cvcp, T twoom, int inverse_only,
-    const cplx<T> *__restrict__ spec, int nfs, T *__restrict__ colq, const T *__restrict__ vcg,
-    const T *__restrict__ svcg, const T *__restrict__ vfsvc, T vcamp, int store) {
+// columns of a member from which a getdyntend call takes k_columns_serial (FP32)
+static bool columns_serial(long ng) { return ng >= 100000; }
+// The dynamics columns with one thread per column, every sum in the order of the
+// reference's recursions (FP32). The curl of the pressure gradient nearly
+// vanishes, so the vorticity tendency carries the rounding of getpresgrad's
+// terms and sums: 5e-5 of itself at T254, 3e-5 at T170, and k_columns' order of
+// them moves it by 3e-5 and 2e-5. Inside advance that is a few parts in 1e6 of
+// the state; a getdyntend call hands the tendency itself out, and takes this
+// kernel where the columns fill the chip with one thread each (columns_serial):
+// 232 us at T254L64, k_columns 193.
+template <bool VC>
+__global__ __launch_bounds__(256) void k_columns_serial(
+    const float *__restrict__ gsyn, float *__restrict__ gan, float *__restrict__ etadot, float *__restrict__ dlnpdt,
+    float *__restrict__ psg_out, float *__restrict__ dlnpsdt_out, const float *__restrict__ dphisdx,
+    const float *__restrict__ dphisdy, const float *__restrict__ ak_, const float *__restrict__ bk_,
+    const float *__restrict__ ck_, const float *__restrict__ dbk_, const float *__restrict__ dak_, const float *__restrict__ sinlat,
+    int nl, int ntr, int nsyn, int nan, long ng, int nlon, float rd, float kappa, float cvcp, float twoom,
+    const cplx<float> *__restrict__ spec, int nfs, float *__restrict__ colq, const float *__restrict__ vcg,
+    const float *__restrict__ svcg, const float *__restrict__ vfsvc, float vcamp, int) {
+    typedef float T;
     __shared__ T ak[MAXLEV + 1], bk[MAXLEV + 1], ck[MAXLEV], dbk[MAXLEV], dak[MAXLEV];
     for (int i = threadIdx.x; i <= nl; i += blockDim.x) {
         ak[i] = ak_[i];
@@ -344,8 +709,8 @@ __global__ __launch_bounds__(256) void k_columns(
     T *WD = dlnpdt + (long)mem * nl * ng + col;
     const T alfa1 = T(SGLF(0.69314718055994530942)), rlnp1 = T(SGLF(99999.99));
 #define LV(P, L) (P)[(long)((L) - 1) * ng]
-    auto pk = [&](int K) { return ak[K - 1] + bk[K - 1] * ps; };
-    auto dp = [&](int K) { return fma(dbk[K - 1], ps, dak[K - 1]); };  // pk(K + 1) - pk(K), one rounding
+    auto pk = [&](int K) -> T { return ak[K - 1] + bk[K - 1] * ps; };
+    auto dp = [&](int K) -> T { return fma(dbk[K - 1], ps, dak[K - 1]); };  // pk(K + 1) - pk(K), one rounding
     // omega / p of layer K (getomega's workb, workc) from the sums db, cb over
     // the layers above it
     auto omega_p = [&](int K, T dba, T cba, const OmegaTerms<T> &o, T dv, T dpk, T rdp, T rlnp, T alfa) {
@@ -359,20 +724,10 @@ __global__ __launch_bounds__(256) void k_columns(
         }
         return (workc - workb) * rdp;
     };
-    // pass 1 (top -> bottom): getomega's running sums db, cb and their column
-    // totals. Where a caller sees the grids (store) it also writes omega/p
-    // (dlnpdtg) on layers and etadot at interfaces less its term -ps bk_K
-    // dlnpsdt, which needs the column totals; the etadot buffer keeps that
-    // partial value and its readers add the term (pass 4 here, which needs it
-    // with tracers, and k_etadot_complete for the grid handed to callers).
-    // Pass 3 recomputes both from the layer data and the compensated sums.
-    const bool st_et = store || ntr > 0;
+    // pass 1 (top -> bottom): getomega's sums db, cb and their column totals
     T db = 0, cb = 0;
     PairSum<T> sdb, scb;
-    if (st_et) {
-        ET[0] = T(0);
-        ET[(long)nl * ng] = T(0);
-    }
+    ET[(long)nl * ng] = T(0);
     constexpr int P1G = 4;  // levels whose loads are issued together
     for (int K0 = 1; K0 <= nl; K0 += P1G) {
         T gu[P1G], gv[P1G], gd[P1G];
@@ -387,28 +742,14 @@ __global__ __launch_bounds__(256) void k_columns(
         for (int i = 0; i < P1G; i++) {
             const int K = K0 + i;
             if (K > nl) break;
-            int L = nl + 1 - K;
-            const T dpk = dp(K), dv = gd[i];
-            const OmegaTerms<T> o = omega_terms(gu[i], gv[i], dv, dpx, dpy, dpk, dbk[K - 1]);
-            if (store) {
-                T p1 = pk(K), p2 = pk(K + 1), rdp = recip(dpk);
-                T rlnp = rlnp1, alfa = alfa1;
-                if (K > 1) {
-                    const LayerCoef<T> lc = layer_coef(p1, p2, dpk, bk[K - 1], bk[K], ck[K - 1], dbk[K - 1]);
-                    rlnp = lc.rlnp;
-                    alfa = lc.alfa;
-                }
-                LV(WD, L) = omega_p(K, db, cb, o, dv, dpk, rdp, rlnp, alfa);
-            }
+            const OmegaTerms<T> o = omega_terms(gu[i], gv[i], gd[i], dpx, dpy, dp(K), dbk[K - 1]);
             db += o.tdb;
             cb += o.tcb;
             sdb.add(o.tdb);
             scb.add(o.tcb);
-            if (st_et && K <= nl - 1) ET[(long)K * ng] = -(ps * cb) - db;
         }
     }
     const T dlnpsdt = -db / ps - cb;
-    auto et_fix = [&](int K) { return -(ps * bk[K]) * dlnpsdt; };  // etadot - stored value, 0 < K < nl
     psg_out[(long)mem * ng + col] = ps;
     dlnpsdt_out[(long)mem * ng + col] = dlnpsdt;
     if (colq) {
@@ -421,7 +762,6 @@ __global__ __launch_bounds__(256) void k_columns(
         }
         colq[(long)mem * ng + col] = s;
     }
-    if (inverse_only) return;
     T *A = gan + (long)mem * nan * ng + col;
     T *TT = A, *FX = A + (long)nl * ng, *FY = A + 2L * nl * ng, *KE = A + 3L * nl * ng;
     A[4L * nl * ng] = dlnpsdt;
@@ -469,20 +809,16 @@ __global__ __launch_bounds__(256) void k_columns(
             rcb.add(o.tcb);
             const T dba = sdb.minus(rdb), cba = scb.minus(rcb);  // sums over the layers above K
             T ea = T(0);                                   // etadot at the top interface K - 1
-            if (K > 1) ea = (-(ps * cba) - dba) + et_fix(K - 1);
-            T rlnp, alfa, cofa, dbp;
+            if (K > 1) ea = (-(ps * cba) - dba) - (ps * bk[K - 1]) * dlnpsdt;
+            ET[(long)(K - 1) * ng] = ea;
+            T rlnp = rlnp1, alfa = alfa1, cofa, dbp;
+            const T rp1 = recip(p1), rp2 = recip(p2);
             if (K == 1) {
-                const T rp1 = recip(p1), rp2 = recip(p2);
-                rlnp = rlnp1;
-                alfa = alfa1;
                 cofa = -rdp * (bk[K] * p1 * rp2 - bk[K - 1] + rlnp * (bk[K - 1] - p1 * dbk[K - 1] * rdp));
                 dbp = bk[K] * rp2 - bk[K - 1] * rp1;
             } else {
-                const LayerCoef<T> lc = layer_coef(p1, p2, dpk, bk[K - 1], bk[K], ck[K - 1], dbk[K - 1]);
-                rlnp = lc.rlnp;
-                alfa = lc.alfa;
-                cofa = lc.cofa;
-                dbp = lc.dbp;
+                layer_log(p1, p2, dpk, rp1, rdp, rlnp, alfa);
+                layer_rest(p1, dpk, bk[K - 1], bk[K], ck[K - 1], dbk[K - 1], rp1, rp2, rdp, rlnp, alfa, cofa, dbp);
             }
             T cofb0 = (K == 1) ? -rdp * (alfa * dbk[0]) : -rdp * (bk[K - 1] * rlnp + alfa * dbk[K - 1]);
             T tx = gtx[i], ty = gty[i];
@@ -506,7 +842,9 @@ __global__ __launch_bounds__(256) void k_columns(
                 vv = h * (eb * (vm - v) + ea * (v - vp));
                 vt = h * (eb * (tm - tv) + ea * (tv - tp));
             }
-            T vq = kappa * omega_p(K, dba, cba, o, dv, dpk, rdp, rlnp, alfa) * tv;
+            const T om = omega_p(K, dba, cba, o, dv, dpk, rdp, rlnp, alfa);
+            LV(WD, L) = om;
+            T vq = kappa * om * tv;
             if (ntr > 0) vq = vq / (T(1) + cvcp * LV(Q, L));
             vv -= prsgy;
             vu -= prsgx;
@@ -556,9 +894,7 @@ __global__ __launch_bounds__(256) void k_columns(
         T ddk = guard(Dk1 - Dk);                                                    // dd_1
         T hprev = Dk;                                                                // half_0
         for (int K = 1; K <= nl; K++) {
-            // the interfaces 0 and nl are exactly zero; the others are completed here
-            const T etop = (K > 1) ? ET[(long)(K - 1) * ng] + et_fix(K - 1) : T(0);
-            const T ebot = (K < nl) ? ET[(long)K * ng] + et_fix(K) : T(0);
+            const T etop = ET[(long)(K - 1) * ng], ebot = ET[(long)K * ng];
             const T dpk = dp(K);
             T hk, Dk2 = T(0), ddn = T(0);
             if (K <= nl - 1) {
@@ -2111,23 +2447,6 @@ __global__ void k_pack(cplx<T> *__restrict__ spec, const cplx<T> *__restrict__ r
 }
 
 // grid fields of a member-major field set -> caller layout
-// etadot handed to callers: the column kernel stores interface K (0 < K < nl)
-// without its term -ps bk_K dlnpsdt (added by its readers); this adds it to a
-// gathered copy, [member][nl + 1 interfaces][ng]
-template <typename T>
-__global__ void k_etadot_complete(T *__restrict__ et, const T *__restrict__ psg, const T *__restrict__ dlnpsdt,
-                                  const T *__restrict__ bk, int nl, long ng, int nm) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long per = (long)(nl + 1) * ng;
-    if (i >= per * nm) return;
-    const int mem = (int)(i / per);
-    const long r = i - mem * per;
-    const int K = (int)(r / ng);
-    const long col = r - K * ng;
-    if (K == 0 || K == nl) return;
-    et[i] += -(psg[(long)mem * ng + col] * bk[K]) * dlnpsdt[(long)mem * ng + col];
-}
-
 template <typename T>
 __global__ void k_grid_gather(const T *__restrict__ src, long mstride, T *__restrict__ dst, long per_mem, int nm) {
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2880,22 +3199,41 @@ template <typename T> struct Step {
     }
     void columns(int inverse_only, bool colq = false) {
         const gfsdc_cfg &c = E.cfg;
-        dim3 g((unsigned)((B.ng + 255) / 256), B.nm);
         const bool vc = B.vc_on && !inverse_only;
         // the omega / p and etadot grids are stored where a caller sees them: by
         // the inverse pass of the physics, a getdyntend call, or with no physics
         // the dynamics passes themselves
         const int store = (inverse_only || grids || c.physics == GFSDC_PHYS_NONE) ? 1 : 0;
         if (vc) synth_vc();
-        auto kern = vc ? k_columns<T, true> : k_columns<T, false>;
-        hipLaunchKernelGGL(kern, g, dim3(256), 0, s, (const T *)B.gsyn, (T *)B.gan, (T *)B.etadot,
+        auto launch = [&](auto kern, unsigned nblk, unsigned nthr) {
+            hipLaunchKernelGGL(kern, dim3(nblk, B.nm), dim3(nthr), 0, s, (const T *)B.gsyn, (T *)B.gan, (T *)B.etadot,
                            (T *)B.dlnpdt, (T *)B.psg, (T *)B.dlnpsdt, (const T *)B.dphisdx, (const T *)B.dphisdy,
                            (const T *)B.ak, (const T *)B.bk, (const T *)B.ck, (const T *)B.dbk,
                            (const T *)B.dak, (const T *)B.sinlat, B.nl, B.ntr, B.nsyn, B.nan, B.ng, E.plan.nlon, (T)c.rd,
-                           (T)(c.rd / c.cp), (T)(c.cvap / c.cp - 1.0), (T)(2.0 * c.omega), inverse_only,
+                           (T)(c.rd / c.cp), (T)(c.cvap / c.cp - 1.0), (T)(2.0 * c.omega),
                            (const cplx<T> *)B.spec, B.nfs, colq ? (T *)B.colq : (T *)nullptr, (const T *)B.vcg,
                            B.st_on[0] ? (const T *)B.st_grd : (const T *)nullptr, (const T *)B.st_vf,
                            (T)B.sc.vcamp, store);
+        };
+        if constexpr (sizeof(T) == 4)
+            if (grids && !inverse_only && columns_serial(B.ng)) {
+                launch(vc ? k_columns_serial<true> : k_columns_serial<false>, (unsigned)((B.ng + 255) / 256), 256);
+                mark("columns");
+                return;
+            }
+        constexpr int NC = ColCfg<T>::NC, CH = ColCfg<T>::CH, LPC = MAXLEV / CH;
+        const bool half = B.nl <= CH * LPC / 2;  // half the registers for the layers where they suffice
+        auto pick = [&](auto mode, auto tr) {
+            constexpr int M = decltype(mode)::value;
+            constexpr bool TR = decltype(tr)::value;
+            return half ? k_columns<T, M, LPC / 2, TR> : k_columns<T, M, LPC, TR>;
+        };
+        auto mode = [&](auto tr) {
+            return vc ? pick(std::integral_constant<int, COL_VC>(), tr)
+                      : inverse_only ? pick(std::integral_constant<int, COL_INV>(), tr)
+                                     : pick(std::integral_constant<int, COL_DYN>(), tr);
+        };
+        launch(B.ntr > 0 ? mode(std::true_type()) : mode(std::false_type()), (unsigned)((B.ng + NC - 1) / NC), NC * CH);
         mark(inverse_only ? "columns_inverse" : "columns");
     }
     // FP64 area sums: S(psg) -> pmean, S(b) -> bsum; pdryini = S(psg) - S(b) where 0;
@@ -4363,11 +4701,6 @@ template <typename T> int Engine<T>::get_grid(int which, void *out, int dtype, i
     hipLaunchKernelGGL(k_grid_gather<T>, dim3((unsigned)((per * nm + 255) / 256)), dim3(256), 0, stream, src,
                        mstride, (T *)stage[3], per, nm);
     GFSDC_CHECK(hipGetLastError());
-    if (which == GF_ETADOT) {  // the column kernel keeps etadot without its -ps bk dlnpsdt term
-        hipLaunchKernelGGL(k_etadot_complete<T>, dim3((unsigned)((per * nm + 255) / 256)), dim3(256), 0, stream,
-                           (T *)stage[3], (const T *)B->psg, (const T *)B->dlnpsdt, (const T *)B->bk, nl, ng, nm);
-        GFSDC_CHECK(hipGetLastError());
-    }
     return output((const T *)stage[3], out, (size_t)per * nm, dtype, loc, 1);
 }
 

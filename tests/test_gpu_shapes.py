@@ -110,3 +110,40 @@ def test_transforms_every_length(grid, nf, monkeypatch):
             for shift in (0, rt().itemsize):
                 for x, h in zip(device_call(g, fn, ins, outs, nf, *extra, shift=shift), host):
                     assert np.array_equal(x, h), (fn, prec, shift)
+
+
+# chunks of layers: one per thread, most empty, partial, full and half full ones; a member's columns on and off the
+# 64 (FP64: 32) of a workgroup; T170 has the columns for which a getdyntend call takes one thread per column in FP32
+@pytest.mark.parametrize("grid,nlev,ntrac", [((64, 32, 21), 2, 1), ((64, 32, 21), 7, 0), ((72, 36, 23), 17, 2),
+                                             ((72, 36, 23), 32, 1), ((64, 32, 21), 33, 1), ((72, 36, 23), 63, 0),
+                                             ((64, 32, 21), 64, 2), ((512, 256, 170), 5, 1)])
+def test_columns_every_chunk(grid, nlev, ntrac):
+    """Tendencies, omega/p and etadot grids of getdyntend and of its inverse-only form, two members, against the
+    oracle at the bounds of test_gpu_dycore (FP64 1e-9, FP32 2e-4)."""
+    import cases
+    import gfsdc
+    nlon, nlat, T = grid
+    ak, bk = levels.hybrid_levels(nlev)
+    o = O.Model(nlon, nlat, T, nlev, ak, bk, 600.0, ntrac=ntrac)
+    st = []
+    for mem in range(2):
+        vrt, div, tv, lnps = cases.perturbed_state(o.sht.degree, o.sht.order, nlev, seed=3 + mem, amp=0.3)
+        q = np.zeros((ntrac, nlev, o.sht.nlm), complex)
+        for t in range(ntrac):
+            q[t] = 1e-4 * cases.perturbed_state(o.sht.degree, o.sht.order, nlev, seed=9 + t + mem, amp=1.0)[2][0]
+            q[t, :, 0] = 0.01 * np.linspace(1.0, 0.2, nlev) * np.sqrt(4 * np.pi)
+        st.append((vrt[0], div[0], tv[0], lnps[0], q))
+    for prec, tol in ((gfsdc.FP64, 1e-9), (gfsdc.FP32, 2e-4)):
+        g = gfsdc.Context(nlon, nlat, T, prec, nlev=nlev, ak=ak, bk=bk, dt=600.0, ntrac=ntrac, nmem=2)
+        a = [np.stack(x) for x in zip(*st)]
+        g.set_state(a[0], a[1], a[2], a[3], trac=a[4] if ntrac else None)
+        for inverse in (False, True):
+            tg = g.getdyntend(1, inverse_only=inverse)
+            grids = {k: g.grid(k) for k in ("dlnpdtg", "etadot", "psg", "dlnpsdt")}
+            for mem in range(2):
+                o.set_state(st[mem][0], st[mem][1], st[mem][2], st[mem][3], *([st[mem][4]] if ntrac else []))
+                to = o.getdyntend(1)
+                for k in () if inverse else ("dvrt", "ddiv", "dtv", "dlnps") + (("dtrac",) if ntrac else ()):
+                    assert rel(tg[k][mem], to[k]) < tol, (prec, k, mem, rel(tg[k][mem], to[k]))
+                for k, x in grids.items():
+                    assert rel(x[mem], o.grid(k)) < tol, (prec, inverse, k, mem, rel(x[mem], o.grid(k)))
