@@ -180,11 +180,12 @@ __device__ inline float4 vkeep(const float4 &x, bool keep) {
 __device__ inline double2 vkeep(const double2 &x, bool keep) { return double2{keep ? x.x : 0.0, keep ? x.y : 0.0}; }
 
 // One LDS chunk of a wave's 32 x (16 WB) tile. GUARD skips (wave-uniformly) the
-// k-steps of 4 at or beyond kmax and the 16-column blocks at or beyond nbj, so a
-// partial last chunk or column tile issues only the MFMAs it needs.
+// k-steps of 4 at or beyond kmax, the 16-column blocks at or beyond nbj and the
+// 16-row blocks at or beyond nbi, so a partial last chunk, column tile or
+// latitude tile issues only the MFMAs it needs.
 template <typename T, bool GUARD, typename Acc>
 __device__ inline void gemm_chunk(T (*As)[GEMM_BM + LDS_PAD], T (*Bs)[GT<T>::BN + LDS_PAD], Acc (&E)[2][GT<T>::WB],
-                                  int lane, int wm, int wn, int kmax = GEMM_BK, int nbj = GT<T>::WB) {
+                                  int lane, int wm, int wn, int kmax = GEMM_BK, int nbj = GT<T>::WB, int nbi = 2) {
     constexpr int NK = GEMM_BK / 4, WB = GT<T>::WB;
     const int li = lane & 15, kl = lane >> 4;
     if constexpr (!GUARD) {
@@ -224,6 +225,7 @@ __device__ inline void gemm_chunk(T (*As)[GEMM_BM + LDS_PAD], T (*Bs)[GT<T>::BN 
             T b = Bs[kr][wn + bj * 16 + li];
 #pragma unroll
             for (int bi = 0; bi < 2; bi++) {
+                if (GUARD && bi >= nbi) break;
                 if (Vec<T>::swap)
                     E[bi][bj] = MF<T>::mma(b, a[bi], E[bi][bj]);
                 else
@@ -312,16 +314,19 @@ __global__ __launch_bounds__(256) void k_leg_synth(const T *__restrict__ plm, co
     constexpr bool PREFETCH = sizeof(T) == 4;
     // valid 16-column blocks of this wave (the last column tile is partial)
     const int nbj = min(WB, max(0, (ncol - c0 - wn + 15) / 16));
+    // and 16-row blocks: the last latitude tile is partial (32 of 64 rows at T42, 31 of
+    // 64 in the second tile at T126)
+    const int nbi = min(2, max(0, (nhalf - j0 - wm + 15) / 16));
     if (PREFETCH && Kp > 0) load(0);
     for (int k0 = 0; k0 < Kp; k0 += GEMM_BK) {
         if (!PREFETCH) load(k0);
         store(k0);
         __syncthreads();
         if (PREFETCH && k0 + GEMM_BK < Kp) load(k0 + GEMM_BK);
-        if (nbj == WB && k0 + GEMM_BK <= Kp)
+        if (nbj == WB && nbi == 2 && k0 + GEMM_BK <= Kp)
             gemm_chunk<T, false>(As, Bs, E, lane, wm, wn);
-        else
-            gemm_chunk<T, true>(As, Bs, E, lane, wm, wn, Kp - k0, nbj);
+        else if (nbi > 0)
+            gemm_chunk<T, true>(As, Bs, E, lane, wm, wn, Kp - k0, nbj, nbi);
         __syncthreads();
     }
     const int nm1 = ntrunc + 1;
@@ -415,8 +420,8 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_leg_anal(const T *__restrict__ plmt, const long *__restrict__ tpoff,
                                                   const int *__restrict__ keoff, const int *__restrict__ mtile_m,
                                                   const int *__restrict__ mtile_i, const T *__restrict__ fa,
-                                                  int ldf, T *__restrict__ sx, int ldx, int nhp, int ntrunc, int ncol,
-                                                  int nmt, const int *__restrict__ nfdyn) {
+                                                  int ldf, T *__restrict__ sx, int ldx, int nhalf, int nhp, int ntrunc,
+                                                  int ncol, int nmt, const int *__restrict__ nfdyn) {
     typedef typename MF<T>::acc acc_t;
     typedef typename Vec<T>::t V;
     constexpr int VW = Vec<T>::n;
@@ -480,12 +485,14 @@ __global__ __launch_bounds__(256) void k_leg_anal(const T *__restrict__ plmt, co
     const int ne = min(2, max(0, (Kp - i0 - wm + 15) / 16));
     const int nbj = min(WB, max(0, (ncol - c0 - wn + 15) / 16));
     const bool full = ne == 2 && nbj == WB;
+    // the sum ends with the last latitude pair, not with the padding of the table's rows
+    // (32 of 64 at T42, 95 of 128 at T126; the rest is zero)
     if (PREFETCH) load(0);
-    for (int j0 = 0; j0 < nhp; j0 += GEMM_BK) {
+    for (int j0 = 0; j0 < nhalf; j0 += GEMM_BK) {
         if (!PREFETCH) load(j0);
         store();
         __syncthreads();
-        if (PREFETCH && j0 + GEMM_BK < nhp) load(j0 + GEMM_BK);
+        if (PREFETCH && j0 + GEMM_BK < nhalf) load(j0 + GEMM_BK);
         if (full)
             gemm_chunk1<T, false, WB>(&As[0][0], Bs[0], BN + LDS_PAD, E, lane, wm, wn);
         else
@@ -618,7 +625,7 @@ __global__ __launch_bounds__(256) void k_leg_synth_b3(const float *__restrict__ 
 __global__ __launch_bounds__(256) void k_leg_anal_b3(const float *__restrict__ plm, const long *__restrict__ poff,
                                                      const int *__restrict__ keoff, const int *__restrict__ mtile_m,
                                                      const int *__restrict__ mtile_i, const float *__restrict__ fa,
-                                                     int ldf, float *__restrict__ sx, int ldx, int nhp, int ntrunc) {
+                                                     int ldf, float *__restrict__ sx, int ldx, int nhalf, int nhp, int ntrunc) {
     const int tc = blockIdx.x;
     const int m = mtile_m[blockIdx.y], i0 = mtile_i[blockIdx.y];
     const int K = ntrunc + 2 - m, Ke = (K + 1) >> 1, Ko = K >> 1;
@@ -634,7 +641,7 @@ __global__ __launch_bounds__(256) void k_leg_anal_b3(const float *__restrict__ p
     for (int a = 0; a < 2; a++)
 #pragma unroll
         for (int b = 0; b < 4; b++) E[a][b] = O[a][b] = b3f4{0.f, 0.f, 0.f, 0.f};
-    for (int j0 = 0; j0 < nhp; j0 += B3K) {
+    for (int j0 = 0; j0 < nhalf; j0 += B3K) {
 #pragma unroll
         for (int par = 0; par < 2; par++) {
             const float *Pp = par ? P1 : P0;
@@ -1937,12 +1944,12 @@ void launch_leg_anal(const Plan<T> &p, const T *fa, int ldf, T *sx, int ldx, int
     if constexpr (sizeof(T) == 4) {
         if (p.leg_bf16x3) {
             hipLaunchKernelGGL(k_leg_anal_b3, dim3((ncol + GEMM_BN - 1) / GEMM_BN, p.n_mtiles), dim3(256), 0, s, p.plm,
-                               p.poff, p.keoff, p.mtile_m, p.mtile_i, fa, ldf, sx, ldx, p.nhp, p.ntrunc);
+                               p.poff, p.keoff, p.mtile_m, p.mtile_i, fa, ldf, sx, ldx, p.nhalf, p.nhp, p.ntrunc);
             return;
         }
     }
     hipLaunchKernelGGL(k_leg_anal<T>, dim3(ntc * p.n_mtiles * 2), dim3(256), 0, s, p.plmt, p.tpoff, p.keoff,
-                       p.mtile_m, p.mtile_i, fa, ldf, sx, ldx, p.nhp, p.ntrunc, ncol, p.n_mtiles, nfdyn);
+                       p.mtile_m, p.mtile_i, fa, ldf, sx, ldx, p.nhalf, p.nhp, p.ntrunc, ncol, p.n_mtiles, nfdyn);
 }
 
 static Radices radices_of(int n, const int *r) {
