@@ -2445,21 +2445,66 @@ template <typename T> __global__ void k_copy(T *__restrict__ dst, const T *__res
     for (; i < n; i += stride) dst[i] = src[i];
 }
 
-// reference layout (ndimspec, nfield-run) <-> state layout spec[k][member*nfs + off + f]
+// The fields of a state, by name, in the reference layout [member][field][nlm],
+// each null where it is left out; off[i] is field run i's first field in a
+// member's state fields, off[5] their number.
+struct PackParts {
+    const void *p[5];
+    int off[6];
+};
+// reference layout <-> state layout spec[k][member * nfs + f]: 64 coefficients x 32
+// (FP64: 16) state fields of whatever runs a tile are transposed through LDS, so
+// that both sides move in runs of 256 bytes. One launch takes a whole state: a
+// launch per field run with one element a thread, a field apart in the state,
+// took 6.2 us for 64 levels at T126 (23 us at T254) and wrote a copy of each run.
+constexpr int PACK_K = 64;
+template <typename T> constexpr int PACK_F = sizeof(T) == 4 ? 32 : 16;
 template <typename T>
-__global__ void k_pack(cplx<T> *__restrict__ spec, const cplx<T> *__restrict__ ref, int nfr, int off, int nfs,
-                       int nm, int nlm, int to_state) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    long tot = (long)nfr * nm * nlm;
-    if (i >= tot) return;
-    int k = (int)(i % nlm);
-    long fr = i / nlm;  // member * nfr + f
-    int mem = (int)(fr / nfr), f = (int)(fr % nfr);
-    long si = (long)k * nfs * nm + (long)mem * nfs + off + f;
-    if (to_state)
-        spec[si] = ref[i];
-    else
-        const_cast<cplx<T> *>(ref)[i] = spec[si];
+__global__ __launch_bounds__(256) void k_pack(cplx<T> *__restrict__ spec, PackParts pp, int nfs, int nm, int nlm,
+                                              int to_state) {
+    constexpr int F = PACK_F<T>;
+    __shared__ cplx<T> buf[F][PACK_K + 1];
+    __shared__ cplx<T> *row[F];  // the reference row of each state field of the tile
+    const int tid = threadIdx.x, k0 = blockIdx.x * PACK_K, c0 = blockIdx.y * F, NFS = nfs * nm;
+    if (tid < F) {
+        cplx<T> *r = nullptr;
+        if (c0 + tid < NFS) {
+            const int mem = (c0 + tid) / nfs, f = c0 + tid - mem * nfs;
+#pragma unroll
+            for (int i = 0; i < 5; i++)
+                if (f >= pp.off[i] && f < pp.off[i + 1] && pp.p[i])
+                    r = (cplx<T> *)const_cast<void *>(pp.p[i]) +
+                        ((long)mem * (pp.off[i + 1] - pp.off[i]) + f - pp.off[i]) * nlm;
+        }
+        row[tid] = r;
+    }
+    __syncthreads();
+    const int kl = tid % PACK_K, fl = tid % F;
+    if (to_state) {
+        cplx<T> v[F / 4];
+#pragma unroll
+        for (int i = 0; i < F / 4; i++) {
+            const cplx<T> *r = row[4 * i + tid / PACK_K];
+            if (r && k0 + kl < nlm) v[i] = r[k0 + kl];
+        }
+#pragma unroll
+        for (int i = 0; i < F / 4; i++) buf[4 * i + tid / PACK_K][kl] = v[i];
+        __syncthreads();
+        if (row[fl])
+            for (int k = tid / F; k < PACK_K && k0 + k < nlm; k += 256 / F)
+                spec[(long)(k0 + k) * NFS + c0 + fl] = buf[fl][k];
+    } else {
+        if (row[fl])
+#pragma unroll
+            for (int i = 0; i < PACK_K * F / 256; i++) {
+                const int k = tid / F + i * (256 / F);
+                buf[fl][k] = spec[(long)min(k0 + k, nlm - 1) * NFS + c0 + fl];
+            }
+        __syncthreads();
+        if (k0 + kl < nlm)
+            for (int f = tid / PACK_K; f < F; f += 4)
+                if (row[f]) row[f][k0 + kl] = buf[f][kl];
+    }
 }
 
 // grid fields of a member-major field set -> caller layout
@@ -3950,6 +3995,65 @@ template <typename T> int Engine<T>::mlp_adamw_host(const float *grad, double lr
     return rc;
 }
 
+template <typename T> static PackParts pack_parts(const DycoreBuffers *B, const void *const (&p)[5]) {
+    const int nl = B->nl, t = B->ntr * nl;
+    PackParts pp{{p[0], p[1], p[2], p[3], p[4]}, {0, nl, 2 * nl, 3 * nl, 3 * nl + t, 3 * nl + t + 1}};
+    return pp;
+}
+
+template <typename T> static void launch_pack(const Plan<T> &p, const DycoreBuffers *B, cplx<T> *spec, const PackParts &pp,
+                                              bool to_state, hipStream_t s) {
+    dim3 g((unsigned)((p.nlm + PACK_K - 1) / PACK_K), (unsigned)((B->nfs * B->nm + PACK_F<T> - 1) / PACK_F<T>));
+    hipLaunchKernelGGL(k_pack<T>, g, dim3(256), 0, s, spec, pp, B->nfs, B->nm, p.nlm, to_state ? 1 : 0);
+}
+
+// caller's vrt, div, tv, tracers, ln ps (null: left alone) -> state layout
+template <typename T> int Engine<T>::pack_in(void *spec, const void *const (&p)[5], int dtype, int loc) {
+    DycoreBuffers *B = dyn;
+    const PackParts all = pack_parts<T>(B, p);
+    PackParts dir = all;
+    for (int i = 0; i < 5; i++) {
+        const int nfr = all.off[i + 1] - all.off[i];
+        if (!p[i] || nfr == 0 || is_direct<T>(dtype, loc)) continue;
+        dir.p[i] = nullptr;
+        const T *in;
+        int rc = input(p[i], (size_t)nfr * B->nm * plan.nlm * 2, dtype, loc, 0, &in);
+        if (rc) return rc;
+        PackParts one = all;
+        for (int j = 0; j < 5; j++) one.p[j] = j == i ? in : nullptr;
+        launch_pack(plan, B, (cplx<T> *)spec, one, true, stream);
+    }
+    if (is_direct<T>(dtype, loc)) launch_pack(plan, B, (cplx<T> *)spec, dir, true, stream);
+    GFSDC_CHECK(hipGetLastError());
+    return 0;
+}
+
+// state layout -> the caller's buffers (null: not wanted)
+template <typename T> int Engine<T>::pack_out(const void *spec, void *const (&p)[5], int dtype, int loc) {
+    DycoreBuffers *B = dyn;
+    const void *cp[5] = {p[0], p[1], p[2], p[3], p[4]};
+    const PackParts all = pack_parts<T>(B, cp);
+    cplx<T> *sp = (cplx<T> *)const_cast<void *>(spec);
+    if (is_direct<T>(dtype, loc)) {
+        launch_pack(plan, B, sp, all, false, stream);
+        GFSDC_CHECK(hipGetLastError());
+        return 0;
+    }
+    for (int i = 0; i < 5; i++) {
+        const int nfr = all.off[i + 1] - all.off[i];
+        if (!p[i] || nfr == 0) continue;
+        const size_t n = (size_t)nfr * B->nm * plan.nlm;
+        int rc = ensure_stage(3, n * sizeof(cplx<T>));
+        if (rc) return rc;
+        PackParts one = all;
+        for (int j = 0; j < 5; j++) one.p[j] = j == i ? stage[3] : nullptr;
+        launch_pack(plan, B, sp, one, false, stream);
+        GFSDC_CHECK(hipGetLastError());
+        if ((rc = output((const T *)stage[3], p[i], n * 2, dtype, loc, 1))) return rc;
+    }
+    return 0;
+}
+
 template <typename T>
 int Engine<T>::set_state(const void *vrt, const void *div, const void *tv, const void *trac, const void *lnps,
                          int dtype, int loc) {
@@ -3958,23 +4062,9 @@ int Engine<T>::set_state(const void *vrt, const void *div, const void *tv, const
         set_error("context has no dycore (nlev == 0)");
         return GFSDC_ESTATE;
     }
-    const int nl = B->nl, nlm = plan.nlm, nm = B->nm;
-    struct Part {
-        const void *p;
-        int nfr, off;
-    } parts[] = {{vrt, nl, 0}, {div, nl, nl}, {tv, nl, 2 * nl}, {trac, B->ntr * nl, 3 * nl},
-                 {lnps, 1, 3 * nl + B->ntr * nl}};
-    for (auto &pt : parts) {
-        if (!pt.p || pt.nfr == 0) continue;
-        const T *in;
-        size_t n = (size_t)pt.nfr * nm * nlm * 2;
-        int rc = input(pt.p, n, dtype, loc, 0, &in);
-        if (rc) return rc;
-        long tot = (long)pt.nfr * nm * nlm;
-        hipLaunchKernelGGL(k_pack<T>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, stream,
-                           (cplx<T> *)B->spec, (const cplx<T> *)in, pt.nfr, pt.off, B->nfs, nm, nlm, 1);
-        GFSDC_CHECK(hipGetLastError());
-    }
+    const void *const parts[5] = {vrt, div, tv, trac, lnps};
+    int rc = pack_in(B->spec, parts, dtype, loc);
+    if (rc) return rc;
     GFSDC_CHECK(hipStreamSynchronize(stream));
     return 0;
 }
@@ -3986,23 +4076,8 @@ int Engine<T>::get_state(void *vrt, void *div, void *tv, void *trac, void *lnps,
         set_error("context has no dycore (nlev == 0)");
         return GFSDC_ESTATE;
     }
-    const int nl = B->nl, nlm = plan.nlm, nm = B->nm;
-    struct Part {
-        void *p;
-        int nfr, off;
-    } parts[] = {{vrt, nl, 0}, {div, nl, nl}, {tv, nl, 2 * nl}, {trac, B->ntr * nl, 3 * nl},
-                 {lnps, 1, 3 * nl + B->ntr * nl}};
-    for (auto &pt : parts) {
-        if (!pt.p || pt.nfr == 0) continue;
-        size_t n = (size_t)pt.nfr * nm * nlm;
-        int rc = ensure_stage(3, n * sizeof(cplx<T>));
-        if (rc) return rc;
-        hipLaunchKernelGGL(k_pack<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, (cplx<T> *)B->spec,
-                           (const cplx<T> *)stage[3], pt.nfr, pt.off, B->nfs, nm, nlm, 0);
-        GFSDC_CHECK(hipGetLastError());
-        if ((rc = output((const T *)stage[3], pt.p, n * 2, dtype, loc, 1))) return rc;
-    }
-    return 0;
+    void *const parts[5] = {vrt, div, tv, trac, lnps};
+    return pack_out(B->spec, parts, dtype, loc);
 }
 
 template <typename T> int Engine<T>::set_topo(const void *topo, int dtype, int loc) {
@@ -4067,23 +4142,8 @@ int Engine<T>::getdyntend(int rkstage, int inverse_only, void *dvrt, void *ddiv,
     if (rkstage == 1) st.area_sums(B->ntr > 0 ? B->colq : nullptr, nullptr, nullptr, true);
     st.analyse(B->adesc_dyn, B->rflag_an, B->nm * B->nan, (cplx<T> *)B->ten[0]);
     GFSDC_CHECK(hipGetLastError());
-    const int nl = B->nl, nlm = plan.nlm, nm = B->nm;
-    struct Part {
-        void *p;
-        int nfr, off;
-    } parts[] = {{dvrt, nl, 0}, {ddiv, nl, nl}, {dtv, nl, 2 * nl}, {dtrac, B->ntr * nl, 3 * nl},
-                 {dlnps, 1, 3 * nl + B->ntr * nl}};
-    for (auto &pt : parts) {
-        if (!pt.p || pt.nfr == 0) continue;
-        size_t n = (size_t)pt.nfr * nm * nlm;
-        int rc = ensure_stage(3, n * sizeof(cplx<T>));
-        if (rc) return rc;
-        hipLaunchKernelGGL(k_pack<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
-                           (cplx<T> *)B->ten[0], (const cplx<T> *)stage[3], pt.nfr, pt.off, B->nfs, nm, nlm, 0);
-        GFSDC_CHECK(hipGetLastError());
-        if ((rc = output((const T *)stage[3], pt.p, n * 2, dtype, loc, 1))) return rc;
-    }
-    return 0;
+    void *const parts[5] = {dvrt, ddiv, dtv, dtrac, dlnps};
+    return pack_out(B->ten[0], parts, dtype, loc);
 }
 
 template <typename T> int Engine<T>::advance(int nsteps, int use_graph) {
@@ -4205,24 +4265,19 @@ int Engine<T>::iau_set(int nfiles, const double *fhrs, double delthrs, const voi
         return GFSDC_ENOMEM;
     }
     const size_t esz = dtype == GFSDC_DT_F32 ? 4 : 8;
-    struct Part {
-        const void *p;
-        int nfr, off;
-    } parts[] = {{vrt, nl, 0}, {div, nl, nl}, {tv, nl, 2 * nl}, {trac, B->ntr * nl, 3 * nl},
-                 {lnps, 1, 3 * nl + B->ntr * nl}};
-    for (auto &pt : parts) {
-        if (pt.nfr == 0) continue;
-        const size_t nper = (size_t)pt.nfr * nm * nlm * 2;  // reals per file
-        for (int f = 0; f < nfiles; f++) {
-            const T *in;
-            if ((rc = input((const char *)pt.p + f * nper * esz, nper, dtype, loc, 0, &in))) return rc;
-            long tot = (long)pt.nfr * nm * nlm;
-            hipLaunchKernelGGL(k_pack<T>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, stream,
-                               (cplx<T> *)B->iau_inc + (long)f * len, (const cplx<T> *)in, pt.nfr, pt.off, B->nfs,
-                               nm, nlm, 1);
-            GFSDC_CHECK(hipGetLastError());
-            GFSDC_CHECK(hipStreamSynchronize(stream));
+    const void *const parts[5] = {vrt, div, tv, B->ntr ? trac : nullptr, lnps};
+    const int nfr[5] = {nl, nl, nl, B->ntr * nl, 1};
+    for (int f = 0; f < nfiles; f++) {
+        const void *at[5];
+        for (int i = 0; i < 5; i++) {
+            if (nfr[i] && !parts[i]) {
+                set_error("null buffer");
+                return GFSDC_EINVAL;
+            }
+            at[i] = nfr[i] ? (const char *)parts[i] + (size_t)f * nfr[i] * nm * nlm * 2 * esz : nullptr;
         }
+        if ((rc = pack_in((cplx<T> *)B->iau_inc + (long)f * len, at, dtype, loc))) return rc;
+        GFSDC_CHECK(hipStreamSynchronize(stream));
     }
     B->iau_n = nfiles;
     B->iau_dt = delthrs * 3600.;
@@ -4630,21 +4685,8 @@ template <typename T>
 int Engine<T>::pack_tphys(void *dvrt, void *ddiv, void *dtv, void *dtrac, int dtype, int loc) {
     DycoreBuffers *B = dyn;
     GFSDC_CHECK(hipGetLastError());
-    const int nl = B->nl, nlm = plan.nlm, nm = B->nm;
-    struct Part {
-        void *p;
-        int nf, off;
-    } parts[] = {{dvrt, nl, 0}, {ddiv, nl, nl}, {dtv, nl, 2 * nl}, {dtrac, B->ntr * nl, 3 * nl}};
-    for (auto &pt : parts) {
-        if (!pt.p || pt.nf == 0) continue;
-        size_t n = (size_t)pt.nf * nm * nlm;
-        int rc = ensure_stage(3, n * sizeof(cplx<T>));
-        if (rc) return rc;
-        hipLaunchKernelGGL(k_pack<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, (cplx<T> *)B->tphys,
-                           (const cplx<T> *)stage[3], pt.nf, pt.off, B->nfs, nm, nlm, 0);
-        if ((rc = output((const T *)stage[3], pt.p, n * 2, dtype, loc, 1))) return rc;
-    }
-    return 0;
+    void *const parts[5] = {dvrt, ddiv, dtv, dtrac, nullptr};
+    return pack_out(B->tphys, parts, dtype, loc);
 }
 
 template <typename T> int Engine<T>::hs_phytend(void *dvrt, void *ddiv, void *dtv, int dtype, int loc) {

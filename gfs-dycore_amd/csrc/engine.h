@@ -15,6 +15,12 @@ enum GridField : int {
 
 struct DycoreBuffers;  // defined in dycore.hip
 
+// whether a caller's buffer is in device memory in the element type T, so that a
+// kernel can read or write it itself
+template <typename T> inline bool is_direct(int dtype, int loc) {
+    return loc == GFSDC_DEVICE && dtype == (sizeof(T) == 8 ? GFSDC_DT_F64 : GFSDC_DT_F32);
+}
+
 template <typename T> struct Engine {
     gfsdc_cfg cfg{};
     std::vector<double> ak, bk;
@@ -54,6 +60,8 @@ template <typename T> struct Engine {
                        int dtype, int loc);
 
     // dycore (dycore.hip)
+    int pack_in(void *spec, const void *const (&p)[5], int dtype, int loc);
+    int pack_out(const void *spec, void *const (&p)[5], int dtype, int loc);
     int dyn_init();
     void dyn_destroy();
     int set_state(const void *vrt, const void *div, const void *tv, const void *trac, const void *lnps,

@@ -216,7 +216,7 @@ template <typename T> int Engine<T>::output(const T *d, void *p, size_t n, int d
 // of a transform can write itself, else null (it writes the workspace, and
 // output() converts or copies). Grids take 16-byte stores.
 template <typename T> static T *direct(void *p, int dtype, int loc, bool grid) {
-    if (!p || loc != GFSDC_DEVICE || (dtype == GFSDC_DT_F64) != (sizeof(T) == 8)) return nullptr;
+    if (!p || !is_direct<T>(dtype, loc)) return nullptr;
     return grid && ((uintptr_t)p & 15) ? nullptr : (T *)p;
 }
 

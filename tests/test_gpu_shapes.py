@@ -147,3 +147,45 @@ def test_columns_every_chunk(grid, nlev, ntrac):
                     assert rel(tg[k][mem], to[k]) < tol, (prec, k, mem, rel(tg[k][mem], to[k]))
                 for k, x in grids.items():
                     assert rel(x[mem], o.grid(k)) < tol, (prec, inverse, k, mem, rel(x[mem], o.grid(k)))
+
+
+# coefficients and state fields on and off the 64 x 32 (FP64: 64 x 16) tiles of the packing kernel
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("grid,nlev,ntrac,nmem", [((64, 32, 21), 5, 2, 3), ((96, 48, 30), 21, 0, 1), ((72, 36, 23), 20, 1, 2)])
+def test_state_packing(grid, nlev, ntrac, nmem, prec):
+    """A state comes back bit for bit through host and through device buffers, whole and with field runs left out."""
+    import gfsdc
+    nlon, nlat, T = grid
+    ak, bk = levels.hybrid_levels(nlev)
+    p = gfsdc.FP64 if prec == "fp64" else gfsdc.FP32
+    ct = np.complex128 if prec == "fp64" else np.complex64
+    dt = gfsdc.DT_F64 if prec == "fp64" else gfsdc.DT_F32
+    g = gfsdc.Context(nlon, nlat, T, p, nlev=nlev, ak=ak, bk=bk, dt=600.0, ntrac=ntrac, nmem=nmem)
+    rng = np.random.default_rng(1)
+    shapes = [(nmem, nlev, g.nlm)] * 3 + [(nmem, ntrac, nlev, g.nlm), (nmem, g.nlm)]
+    x = [(rng.standard_normal(s) + 1j * rng.standard_normal(s)).astype(np.complex64).astype(ct) for s in shapes]
+    g.set_state(x[0], x[1], x[2], x[4], trac=x[3] if ntrac else None)
+    st = g.get_state()
+    for k, v in zip(("vrt", "div", "tv", "trac", "lnps"), x):
+        assert np.array_equal(st[k], v), k
+    # device buffers: the second state without its div and lnps, then everything back but tv
+    L, H = gfsdc.load(), C.CDLL("libamdhip64.so.7")
+    H.hipMalloc.argtypes, H.hipFree.argtypes = [C.POINTER(C.c_void_p), C.c_size_t], [C.c_void_p]
+    H.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    y = [np.ascontiguousarray(2 * v) for v in x]
+    d = [C.c_void_p() for _ in y]
+    try:
+        for q, v in zip(d, y):
+            assert H.hipMalloc(C.byref(q), max(v.nbytes, 16)) == 0 and H.hipMemcpy(q, v.ctypes.data, v.nbytes, 1) == 0
+        assert L.gfsdc_set_state(g.h, d[0], None, d[2], d[3], None, dt, gfsdc.DEVICE) == 0
+        for q, v in zip(d, y):
+            assert H.hipMemcpy(q, np.zeros_like(v).ctypes.data, v.nbytes, 1) == 0
+        assert L.gfsdc_get_state(g.h, d[0], d[1], None, d[3], d[4], dt, gfsdc.DEVICE) == 0
+        g.sync()
+        for i, want in enumerate((y[0], x[1], None, y[3], x[4])):
+            got = np.empty_like(y[i])
+            assert H.hipMemcpy(got.ctypes.data, d[i], got.nbytes, 2) == 0
+            assert np.array_equal(got, want if want is not None else np.zeros_like(got)), i
+    finally:
+        for q in d:
+            H.hipFree(q)
