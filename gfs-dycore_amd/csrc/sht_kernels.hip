@@ -524,169 +524,188 @@ __global__ __launch_bounds__(256) void k_leg_anal(const T *__restrict__ plmt, co
 // BF16x3 Legendre GEMMs (FP32 plan option): each FP32 operand x is split into
 // bf16 hi = rn(x) and lo = rn(x - hi); a product is hi.hi + hi.lo + lo.hi
 // (the lo.lo term, ~2^-16 relative, is dropped) on the bf16 matrix cores
-// (v_mfma_f32_16x16x32_bf16, FP32 accumulation). Same tiling as the FP32
-// kernels (64 x 128 per workgroup, both parities); operands are staged in LDS
-// k-contiguous ([row][k], 8 consecutive k per lane and MFMA) and the MFMA
-// operands are swapped so a lane's four accumulators are four consecutive
-// output columns (16-byte stores).
+// (v_mfma_f32_16x16x32_bf16, FP32 accumulation). Tiles as in the FP32 kernels, 64
+// rows x 128 columns and one parity a workgroup. The operands are staged in LDS
+// k-contiguous, 8 consecutive k per lane and MFMA: the Legendre operand comes
+// from the copy of its table that has k contiguous (latitude-major for the
+// synthesis, degree-major for the analysis), the other one is loaded 8 rows x 2
+// columns a thread and turned around in registers, so every LDS store is 16
+// bytes. The MFMA operands are swapped so a lane's four accumulators are four
+// consecutive output columns. The matrix cores are a third of a chunk's time;
+// the conversions and the output bound the rest. 128 fields at T254: synthesis
+// 46 us, analysis 45 us (93 and 113 with both parities in a workgroup,
+// 2-byte transposing LDS stores and the rounding in integer arithmetic).
 typedef unsigned short b3u8 __attribute__((ext_vector_type(8)));
+typedef unsigned b3w4 __attribute__((ext_vector_type(4)));
 typedef __bf16 b3bf8 __attribute__((ext_vector_type(8)));
 typedef float b3f4 __attribute__((ext_vector_type(4)));
 constexpr int B3K = 32, B3P = B3K + 8;
 
-__device__ inline unsigned short b3_rn(float f) {
-    unsigned int u = __builtin_bit_cast(unsigned int, f);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
+// two floats to packed bf16, round to nearest even
+__device__ __forceinline__ unsigned b3_pack(float a, float b) {
+    return (unsigned)__builtin_bit_cast(unsigned short, (__bf16)a) |
+           ((unsigned)__builtin_bit_cast(unsigned short, (__bf16)b) << 16);
 }
-__device__ inline void b3_split(float x, unsigned short &hi, unsigned short &lo) {
-    hi = b3_rn(x);
-    lo = b3_rn(x - __builtin_bit_cast(float, (unsigned int)hi << 16));
+// 8 consecutive k of one row, split, into its hi and lo rows (16-byte aligned)
+__device__ __forceinline__ void b3_store(const float (&x)[8], unsigned short *hi, unsigned short *lo) {
+    b3w4 h, l;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float a = x[2 * i], b = x[2 * i + 1];
+        h[i] = b3_pack(a, b);
+        l[i] = b3_pack(a - __builtin_bit_cast(float, h[i] << 16), b - __builtin_bit_cast(float, h[i] & 0xFFFF0000u));
+    }
+    *(b3w4 *)hi = h;
+    *(b3w4 *)lo = l;
 }
-__device__ inline b3f4 b3_mma3(const unsigned short *bh, const unsigned short *bl, const unsigned short *ah,
-                               const unsigned short *al, b3f4 c) {
-    const b3bf8 Bh = __builtin_bit_cast(b3bf8, *(const b3u8 *)bh), Bl = __builtin_bit_cast(b3bf8, *(const b3u8 *)bl);
-    const b3bf8 Ah = __builtin_bit_cast(b3bf8, *(const b3u8 *)ah), Al = __builtin_bit_cast(b3bf8, *(const b3u8 *)al);
+__device__ inline b3f4 b3_mma3(const b3bf8 &Bh, const b3bf8 &Bl, const b3bf8 &Ah, const b3bf8 &Al, b3f4 c) {
     c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Bl, Ah, c, 0, 0, 0);
     c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Bh, Al, c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(Bh, Ah, c, 0, 0, 0);
 }
 
-__global__ __launch_bounds__(256) void k_leg_synth_b3(const float *__restrict__ plm, const long *__restrict__ poff,
-                                                      const int *__restrict__ keoff, const float *__restrict__ sx,
-                                                      int ldx, float *__restrict__ fs, int ldf, int nhalf, int nhp,
-                                                      int nlat, int ntrunc, int ntj) {
-    const int tc = blockIdx.x, mt = blockIdx.y;
-    const int m = mt / ntj, tj = mt - m * ntj;
-    const int K = ntrunc + 2 - m, Ke = (K + 1) >> 1, Ko = K >> 1;
-    const float *P0 = plm + poff[m], *P1 = P0 + (long)Ke * nhp;
-    const float *S = sx + (long)keoff[m] * ldx;
-    const int j0 = tj * GEMM_BM, c0 = tc * GEMM_BN;
-    __shared__ __attribute__((aligned(16))) unsigned short Ah[2][GEMM_BM][B3P], Al[2][GEMM_BM][B3P];
-    __shared__ __attribute__((aligned(16))) unsigned short Bh[2][GEMM_BN][B3P], Bl[2][GEMM_BN][B3P];
+struct B3Lds {
+    unsigned short Ah[GEMM_BM][B3P], Al[GEMM_BM][B3P], Bh[GEMM_BN][B3P], Bl[GEMM_BN][B3P];
+};
+
+// The k-loop of one 64 x 128 tile over k = 0 .. kn: arow(i, k) points at 8
+// consecutive k of A's row i (in bounds for every row of the tile), brow(k) at
+// B's row k (columns from the tile's first on); rows of A from na on and of B
+// from kn on count as zero.
+template <typename FA, typename FB>
+__device__ __forceinline__ void b3_loop(B3Lds &L, FA arow, FB brow, int na, int kn, b3f4 (&E)[2][4]) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
-    b3f4 E[2][4], O[2][4];
+    const int ai = tid >> 2, ak = (tid & 3) * 8, bc = 2 * (tid & 63), bk = (tid >> 6) * 8;
+    float a[8];
+    float2 b[8];
+    auto load = [&](int k0) {
+        const float *pa = arow(ai, k0 + ak);
+        const float4 x = *(const float4 *)pa, y = *(const float4 *)(pa + 4);
+        a[0] = x.x, a[1] = x.y, a[2] = x.z, a[3] = x.w, a[4] = y.x, a[5] = y.y, a[6] = y.z, a[7] = y.w;
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+        for (int i = 0; i < 8; i++) b[i] = *(const float2 *)(brow(min(k0 + bk + i, kn - 1)) + bc);
+    };
+    auto store = [&](int k0) {
+        float x[8], y[8];
 #pragma unroll
-        for (int b = 0; b < 4; b++) E[a][b] = O[a][b] = b3f4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < Ke; k0 += B3K) {
+        for (int i = 0; i < 8; i++) x[i] = ai < na ? a[i] : 0.f;
+        b3_store(x, &L.Ah[ai][ak], &L.Al[ai][ak]);
 #pragma unroll
-        for (int par = 0; par < 2; par++) {
-            const float *Pp = par ? P1 : P0;
-            const int Kpp = par ? Ko : Ke;
-#pragma unroll
-            for (int u = 0; u < 2; u++) {  // P: 32 degrees x 64 latitudes
-                const int v = tid + 256 * u, kk = v >> 4, jj = (v & 15) * 4, i = k0 + kk;
-                float4 x = *(const float4 *)(Pp + (long)min(i, Kpp - 1) * nhp + j0 + jj);
-                x = vkeep(x, i < Kpp);
-                b3_split(x.x, Ah[par][jj][kk], Al[par][jj][kk]);
-                b3_split(x.y, Ah[par][jj + 1][kk], Al[par][jj + 1][kk]);
-                b3_split(x.z, Ah[par][jj + 2][kk], Al[par][jj + 2][kk]);
-                b3_split(x.w, Ah[par][jj + 3][kk], Al[par][jj + 3][kk]);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {  // S: 32 degrees x 128 columns
-                const int v = tid + 256 * u, kk = v >> 5, cc = (v & 31) * 4, i = k0 + kk;
-                float4 x = *(const float4 *)(S + (long)(2 * min(i, Kpp - 1) + par) * ldx + c0 + cc);
-                x = vkeep(x, i < Kpp);
-                b3_split(x.x, Bh[par][cc][kk], Bl[par][cc][kk]);
-                b3_split(x.y, Bh[par][cc + 1][kk], Bl[par][cc + 1][kk]);
-                b3_split(x.z, Bh[par][cc + 2][kk], Bl[par][cc + 2][kk]);
-                b3_split(x.w, Bh[par][cc + 3][kk], Bl[par][cc + 3][kk]);
-            }
+        for (int i = 0; i < 8; i++) {
+            const bool ok = k0 + bk + i < kn;
+            x[i] = ok ? b[i].x : 0.f;
+            y[i] = ok ? b[i].y : 0.f;
         }
+        b3_store(x, &L.Bh[bc][bk], &L.Bl[bc][bk]);
+        b3_store(y, &L.Bh[bc + 1][bk], &L.Bl[bc + 1][bk]);
+    };
+    const int r = lane & 15, kq = 8 * (lane >> 4);
+    if (kn > 0) load(0);
+    for (int k0 = 0; k0 < kn; k0 += B3K) {
+        store(k0);
         __syncthreads();
-        const int r = lane & 15, kq = 8 * (lane >> 4);
+        if (k0 + B3K < kn) load(k0 + B3K);
+        b3bf8 Ah[2], Al[2];
 #pragma unroll
-        for (int bi = 0; bi < 2; bi++)
-#pragma unroll
-            for (int bj = 0; bj < 4; bj++) {
-                const int jr = wm + bi * 16 + r, cr = wn + bj * 16 + r;
-                E[bi][bj] = b3_mma3(&Bh[0][cr][kq], &Bl[0][cr][kq], &Ah[0][jr][kq], &Al[0][jr][kq], E[bi][bj]);
-                O[bi][bj] = b3_mma3(&Bh[1][cr][kq], &Bl[1][cr][kq], &Ah[1][jr][kq], &Al[1][jr][kq], O[bi][bj]);
-            }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int bi = 0; bi < 2; bi++)
+        for (int bi = 0; bi < 2; bi++) {
+            Ah[bi] = __builtin_bit_cast(b3bf8, *(const b3u8 *)&L.Ah[wm + bi * 16 + r][kq]);
+            Al[bi] = __builtin_bit_cast(b3bf8, *(const b3u8 *)&L.Al[wm + bi * 16 + r][kq]);
+        }
 #pragma unroll
         for (int bj = 0; bj < 4; bj++) {
-            const int j = j0 + wm + bi * 16 + (lane & 15), c = c0 + wn + bj * 16 + 4 * (lane >> 4);
-            if (j < nhalf) {  // even sum to row j, odd sum to row nlat-1-j (as k_leg_synth)
-                const b3f4 e = E[bi][bj], o = O[bi][bj];
-                *(float4 *)(fs + fs_index(j, m, c, ldf, ntrunc + 1)) = float4{e[0], e[1], e[2], e[3]};
-                *(float4 *)(fs + fs_index(nlat - 1 - j, m, c, ldf, ntrunc + 1)) = float4{o[0], o[1], o[2], o[3]};
-            }
+            const b3bf8 Bh = __builtin_bit_cast(b3bf8, *(const b3u8 *)&L.Bh[wn + bj * 16 + r][kq]);
+            const b3bf8 Bl = __builtin_bit_cast(b3bf8, *(const b3u8 *)&L.Bl[wn + bj * 16 + r][kq]);
+#pragma unroll
+            for (int bi = 0; bi < 2; bi++) E[bi][bj] = b3_mma3(Bh, Bl, Ah[bi], Al[bi], E[bi][bj]);
         }
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(256) void k_leg_synth_b3(const float *__restrict__ plmt, const long *__restrict__ tpoff,
+                                                      const int *__restrict__ keoff, const float *__restrict__ sx,
+                                                      int ldx, float *__restrict__ fs, int ldf, int nhalf, int nhp,
+                                                      int nlat, int ntrunc, int ntj, int ncol,
+                                                      const int *__restrict__ nfdyn) {
+    // tiles in the order of k_leg_synth
+    const int ntc = gridDim.x / (2 * (ntrunc + 1) * ntj);
+    const int L = xcd_tile(blockIdx.x, gridDim.x);
+    const int tc = L % ntc, g = L / ntc, tj = g % ntj, ip = g / ntj, par = ip & 1, im = ip >> 1;
+    const int m = (im & 1) ? ntrunc - (im >> 1) : (im >> 1);
+    const int K = ntrunc + 2 - m, Ke = (K + 1) >> 1, Kp = par ? (K >> 1) : Ke, Kw = round_up_d(Ke, GEMM_BM);
+    const int j0 = tj * GEMM_BM, c0 = tc * GEMM_BN;
+    if (nfdyn) ncol = min(ncol, 2 * *nfdyn);
+    if (c0 >= ncol) return;
+    // the slab of each wave's output is restaged here after the k-loop (as k_leg_synth)
+    constexpr int STG_P = GEMM_BN / 2 + 4;
+    __shared__ __attribute__((aligned(16))) union {
+        B3Lds o;
+        float st[4][16 * STG_P];
+    } lds;
+    b3f4 E[2][4];
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+        for (int y = 0; y < 4; y++) E[x][y] = b3f4{0.f, 0.f, 0.f, 0.f};
+    const float *A = plmt + tpoff[m] + ((long)par * nhp + j0) * Kw;  // rows of Kw degrees, zero past the last
+    const float *B = sx + (long)keoff[m] * ldx + (long)par * ldx + c0;
+    b3_loop(
+        lds.o, [&](int i, int k) { return A + (long)i * Kw + k; }, [&](int k) { return B + (long)(2 * k) * ldx; },
+        GEMM_BM, Kp, E);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
+    float *st = lds.st[wave];
+    const int c = c0 + wn + 4 * (lane & 15);
+#pragma unroll
+    for (int bi = 0; bi < 2; bi++) {
+#pragma unroll
+        for (int bj = 0; bj < 4; bj++) {
+            const b3f4 e = E[bi][bj];
+            *(float4 *)(st + (lane & 15) * STG_P + bj * 16 + 4 * (lane >> 4)) = float4{e[0], e[1], e[2], e[3]};
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int r = 4 * q + (lane >> 4), j = j0 + wm + bi * 16 + r;
+            const float4 v = *(const float4 *)(st + r * STG_P + 4 * (lane & 15));
+            if (j < nhalf && c < ncol) *(float4 *)(fs + fs_index(par ? nlat - 1 - j : j, m, c, ldf, ntrunc + 1)) = v;
+        }
+    }
 }
 
 __global__ __launch_bounds__(256) void k_leg_anal_b3(const float *__restrict__ plm, const long *__restrict__ poff,
                                                      const int *__restrict__ keoff, const int *__restrict__ mtile_m,
                                                      const int *__restrict__ mtile_i, const float *__restrict__ fa,
-                                                     int ldf, float *__restrict__ sx, int ldx, int nhalf, int nhp, int ntrunc) {
-    const int tc = blockIdx.x;
-    const int m = mtile_m[blockIdx.y], i0 = mtile_i[blockIdx.y];
-    const int K = ntrunc + 2 - m, Ke = (K + 1) >> 1, Ko = K >> 1;
-    const float *P0 = plm + poff[m], *P1 = P0 + (long)Ke * nhp;
-    const float *F0 = fa + (long)(2 * m) * nhp * ldf, *F1 = F0 + (long)nhp * ldf;
-    const int c0 = tc * GEMM_BN;
-    __shared__ __attribute__((aligned(16))) unsigned short Ah[2][GEMM_BM][B3P], Al[2][GEMM_BM][B3P];
-    __shared__ __attribute__((aligned(16))) unsigned short Bh[2][GEMM_BN][B3P], Bl[2][GEMM_BN][B3P];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
-    b3f4 E[2][4], O[2][4];
+                                                     int ldf, float *__restrict__ sx, int ldx, int nhalf, int nhp,
+                                                     int ntrunc, int ncol, int nmt, const int *__restrict__ nfdyn) {
+    // tiles in the order of k_leg_anal
+    const int ntc = gridDim.x / (2 * nmt);
+    const int L = xcd_tile(blockIdx.x, gridDim.x), tc = L % ntc, g = L / ntc, par = g & 1, mt = g >> 1;
+    const int m = mtile_m[mt], i0 = mtile_i[mt];
+    const int K = ntrunc + 2 - m, Ke = (K + 1) >> 1, Kp = par ? (K >> 1) : Ke, c0 = tc * GEMM_BN;
+    if (i0 >= Kp) return;  // an odd-parity tile past the last odd degree
+    if (nfdyn) ncol = min(ncol, 2 * *nfdyn);
+    if (c0 >= ncol) return;
+    __shared__ __attribute__((aligned(16))) B3Lds lds;
+    b3f4 E[2][4];
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int x = 0; x < 2; x++)
 #pragma unroll
-        for (int b = 0; b < 4; b++) E[a][b] = O[a][b] = b3f4{0.f, 0.f, 0.f, 0.f};
-    for (int j0 = 0; j0 < nhalf; j0 += B3K) {
-#pragma unroll
-        for (int par = 0; par < 2; par++) {
-            const float *Pp = par ? P1 : P0;
-            const int Kpp = par ? Ko : Ke;
-#pragma unroll
-            for (int u = 0; u < 2; u++) {  // P: 64 degrees x 32 latitudes (k-contiguous already)
-                const int v = tid + 256 * u, ii = v >> 3, jj = (v & 7) * 4, i = i0 + ii;
-                float4 x = *(const float4 *)(Pp + (long)min(i, Kpp - 1) * nhp + j0 + jj);
-                x = vkeep(x, i < Kpp);
-                b3_split(x.x, Ah[par][ii][jj], Al[par][ii][jj]);
-                b3_split(x.y, Ah[par][ii][jj + 1], Al[par][ii][jj + 1]);
-                b3_split(x.z, Ah[par][ii][jj + 2], Al[par][ii][jj + 2]);
-                b3_split(x.w, Ah[par][ii][jj + 3], Al[par][ii][jj + 3]);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {  // F: 32 latitudes x 128 columns
-                const int v = tid + 256 * u, kk = v >> 5, cc = (v & 31) * 4;
-                const float4 x = *(const float4 *)((par ? F1 : F0) + (long)(j0 + kk) * ldf + c0 + cc);
-                b3_split(x.x, Bh[par][cc][kk], Bl[par][cc][kk]);
-                b3_split(x.y, Bh[par][cc + 1][kk], Bl[par][cc + 1][kk]);
-                b3_split(x.z, Bh[par][cc + 2][kk], Bl[par][cc + 2][kk]);
-                b3_split(x.w, Bh[par][cc + 3][kk], Bl[par][cc + 3][kk]);
-            }
-        }
-        __syncthreads();
-        const int r = lane & 15, kq = 8 * (lane >> 4);
-#pragma unroll
-        for (int bi = 0; bi < 2; bi++)
-#pragma unroll
-            for (int bj = 0; bj < 4; bj++) {
-                const int ir = wm + bi * 16 + r, cr = wn + bj * 16 + r;
-                E[bi][bj] = b3_mma3(&Bh[0][cr][kq], &Bl[0][cr][kq], &Ah[0][ir][kq], &Al[0][ir][kq], E[bi][bj]);
-                O[bi][bj] = b3_mma3(&Bh[1][cr][kq], &Bl[1][cr][kq], &Ah[1][ir][kq], &Al[1][ir][kq], O[bi][bj]);
-            }
-        __syncthreads();
-    }
+        for (int y = 0; y < 4; y++) E[x][y] = b3f4{0.f, 0.f, 0.f, 0.f};
+    const float *A = plm + poff[m] + (par ? (long)Ke * nhp : 0L);  // rows of nhp latitude pairs, zero past the last
+    const float *B = fa + (long)(2 * m + par) * nhp * ldf + c0;
+    // rows of nhp >= 64 latitude pairs: a k past nhalf but inside them is zero in both operands
+    b3_loop(
+        lds, [&](int i, int k) { return A + (long)min(i0 + i, Kp - 1) * nhp + k; },
+        [&](int k) { return B + (long)k * ldf; }, Kp - i0, (nhalf + B3K - 1) / B3K * B3K, E);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
     float *X = sx + (long)keoff[m] * ldx;
 #pragma unroll
     for (int bi = 0; bi < 2; bi++)
 #pragma unroll
         for (int bj = 0; bj < 4; bj++) {
             const int i = i0 + wm + bi * 16 + (lane & 15), c = c0 + wn + bj * 16 + 4 * (lane >> 4);
-            const b3f4 e = E[bi][bj], o = O[bi][bj];
-            if (i < Ke) *(float4 *)(X + (long)(2 * i) * ldx + c) = float4{e[0], e[1], e[2], e[3]};
-            if (i < Ko) *(float4 *)(X + (long)(2 * i + 1) * ldx + c) = float4{o[0], o[1], o[2], o[3]};
+            const b3f4 e = E[bi][bj];
+            if (i < Kp) *(float4 *)(X + (long)(2 * i + par) * ldx + c) = float4{e[0], e[1], e[2], e[3]};
         }
 }
 
@@ -1920,16 +1939,14 @@ void launch_scatter_ref_vec(const Plan<T> &p, const T *sx, int ldx, cplx<T> *qv,
                        p.eoff, p.ntrunc, p.nlm, p.nlme, (T)(1.0 / rsphere), inv);
 }
 
-// The BF16x3 Legendre kernels take no device field count: they transform every
-// column of the launch (the columns past it hold earlier data and are not read).
 template <typename T>
 void launch_leg_synth(const Plan<T> &p, const T *sx, int ldx, T *fs, int ldf, int ncol, hipStream_t s,
                       const int *nfdyn) {
     int ntj = p.nhp / GEMM_BM, ntc = (ncol + GT<T>::BN - 1) / GT<T>::BN;
     if constexpr (sizeof(T) == 4) {
         if (p.leg_bf16x3) {
-            hipLaunchKernelGGL(k_leg_synth_b3, dim3((ncol + GEMM_BN - 1) / GEMM_BN, (p.ntrunc + 1) * ntj), dim3(256), 0,
-                               s, p.plm, p.poff, p.keoff, sx, ldx, fs, ldf, p.nhalf, p.nhp, p.nlat, p.ntrunc, ntj);
+            hipLaunchKernelGGL(k_leg_synth_b3, dim3(ntc * 2 * (p.ntrunc + 1) * ntj), dim3(256), 0, s, p.plmt, p.tpoff,
+                               p.keoff, sx, ldx, fs, ldf, p.nhalf, p.nhp, p.nlat, p.ntrunc, ntj, ncol, nfdyn);
             return;
         }
     }
@@ -1943,8 +1960,8 @@ void launch_leg_anal(const Plan<T> &p, const T *fa, int ldf, T *sx, int ldx, int
     int ntc = (ncol + GT<T>::BN - 1) / GT<T>::BN;
     if constexpr (sizeof(T) == 4) {
         if (p.leg_bf16x3) {
-            hipLaunchKernelGGL(k_leg_anal_b3, dim3((ncol + GEMM_BN - 1) / GEMM_BN, p.n_mtiles), dim3(256), 0, s, p.plm,
-                               p.poff, p.keoff, p.mtile_m, p.mtile_i, fa, ldf, sx, ldx, p.nhalf, p.nhp, p.ntrunc);
+            hipLaunchKernelGGL(k_leg_anal_b3, dim3(ntc * p.n_mtiles * 2), dim3(256), 0, s, p.plm, p.poff, p.keoff,
+                               p.mtile_m, p.mtile_i, fa, ldf, sx, ldx, p.nhalf, p.nhp, p.ntrunc, ncol, p.n_mtiles, nfdyn);
             return;
         }
     }

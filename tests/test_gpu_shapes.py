@@ -189,3 +189,19 @@ def test_state_packing(grid, nlev, ntrac, nmem, prec):
     finally:
         for q in d:
             H.hipFree(q)
+
+
+# partial latitude, degree and column tiles (64 x 64 x 128 values), partial k chunks of 32, several column tiles
+@pytest.mark.parametrize("grid,nf", [((64, 32, 21), 1), ((72, 36, 23), 65), ((192, 94, 62), 33), ((288, 144, 95), 64),
+                                     ((384, 190, 126), 5)])
+def test_bf16x3_tiles(grid, nf):
+    """BF16X3 transforms against the oracle at the bounds of test_gpu_transforms (3e-5)."""
+    import gfsdc
+    nlon, nlat, T = grid
+    o, g = O.Sht(nlon, nlat, T), gfsdc.Context(nlon, nlat, T, gfsdc.BF16X3)
+    rng = np.random.default_rng(nf)
+    q = np.maximum(o.degree, 1) ** -1.5 * np.exp(2j * np.pi * rng.random((nf, o.nlm)))
+    q[:, o.order == 0] = q[:, o.order == 0].real
+    ref = o.spectogrd(q)
+    assert rel(g.spectogrd(q.astype(np.complex64), dtype=1), ref) < 3e-5
+    assert rel(g.grdtospec(ref.astype(np.float32), dtype=1), o.grdtospec(ref)) < 3e-5
