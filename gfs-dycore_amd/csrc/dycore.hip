@@ -85,7 +85,6 @@ struct DycoreBuffers {
     double *pwsum = nullptr;                     // FP64 area sum of pwat per member
     void *colq = nullptr;                        // T per member ng: column tracer mass sum(dpk q)
     void *pwat = nullptr, *precip = nullptr;     // T per member ng (simple physics)
-    void *pblscr = nullptr;                      // T per member 2 nlev ng: PBL sweep coefficients
     double *latd = nullptr;                      // FP64 latitude (radians), nlat
     // AR(1) temperature pattern (patterngenerator.f90), per member
     void *tpat = nullptr;                        // cplx<T> nm * nlm
@@ -1276,22 +1275,37 @@ __device__ __forceinline__ double simple_sst(int mode, double lat) {
     return 302.15;
 }
 
+// Simple physics, SP_C columns a workgroup: everything that belongs to a level
+// (layer pressure, condensation, Exner factors, diffusivities, the changes at the
+// end) over SP_C x 16 threads, up to four levels each, and the two tridiagonal
+// sweeps of the boundary layer over one wavefront, a lane for each of u, v, T and
+// q of a column. The profiles stay in LDS in FP64 (49 KB: three workgroups a CU);
+// one thread per column, with the sweeps' coefficients through memory, ran
+// 1100 long FP64 wavefronts at T126. Bound by FP64 arithmetic (the powers and
+// exponentials) and the sweeps' chain of divisions: FP32, T126 64 levels, 150 us
+// a step (one thread per column 370; with 57 KB, two workgroups a CU, 194).
+constexpr int SP_C = 16, SP_L = MAXLEV / 16;
 template <typename T>
 __global__ __launch_bounds__(256) void k_simple_columns(
-    const T *__restrict__ gsyn, const T *__restrict__ psg, T *__restrict__ gan, T *__restrict__ pbl,
-    T *__restrict__ pwat_out, T *__restrict__ precip_out, const T *__restrict__ ak_, const T *__restrict__ bk_,
-    const double *__restrict__ latd, int nl, int ntr, int nsyn, int nsp, long ng, int nlon, T kappa, SimpleCfg sc,
-    ColSel cs) {
+    const T *__restrict__ gsyn, const T *__restrict__ psg, T *__restrict__ gan, T *__restrict__ pwat_out,
+    T *__restrict__ precip_out, const T *__restrict__ ak_, const T *__restrict__ bk_, const double *__restrict__ latd,
+    int nl, int ntr, int nsyn, int nsp, long ng, int nlon, T kappa, SimpleCfg sc, ColSel cs) {
     if (cs.gate && cs.gate[0] == 0) return;
     __shared__ T ak[MAXLEV + 1], bk[MAXLEV + 1];
-    for (int i = threadIdx.x; i <= nl; i += blockDim.x) {
+    // profiles [position c - 1, top -> bottom][column]: T (then T / Exner), q, u, v; Y, then
+    // the momentum sweep's CE; layer pressure, then 1 / dp, then the heat sweep's CE
+    __shared__ double st[MAXLEV][SP_C], sq[MAXLEV][SP_C], su[MAXLEV][SP_C], sv[MAXLEV][SP_C];
+    __shared__ double sy[MAXLEV][SP_C], srp[MAXLEV][SP_C], skm[SP_C], ske[SP_C];
+    const int tid = threadIdx.x, cl = tid % SP_C, lg = tid / SP_C;
+    for (int i = tid; i <= nl; i += 256) {
         ak[i] = ak_[i];
         bk[i] = bk_[i];
     }
     __syncthreads();
-    const long col = sel_col(cs, (long)blockIdx.x * blockDim.x + threadIdx.x, ng);
+    const long col_ = sel_col(cs, (long)xcd_tile(blockIdx.x, gridDim.x) * SP_C + cl, ng);
+    const bool valid = col_ >= 0;
+    const long col = valid ? col_ : 0;  // a column past the last repeats the first and stores nothing
     const int mem = blockIdx.y;
-    if (col < 0) return;
     // simple_physics_v5_1.f90:175-222
     const double gravit = 9.80616, rair = 287.0, cpair = 1.0045e3, latvap = 2.5e6, rh2o = 461.5;
     const double epsilo = rair / rh2o, zvir = (rh2o / rair) - 1.0, Csfc = 0.0011, T0 = 273.16;
@@ -1302,24 +1316,31 @@ __global__ __launch_bounds__(256) void k_simple_columns(
     const T *U = G, *V = G + (long)nl * ng, *TV = G + 4L * nl * ng, *Q = G + 7L * nl * ng;
     T *A = gan + (long)mem * nsp * ng + col;
     T *DT = A, *DU = A + (long)nl * ng, *DV = A + 2L * nl * ng, *DQ = A + 3L * nl * ng;
-    T *CE = pbl + (long)mem * 2 * nl * ng + col, *CEM = CE + (long)nl * ng;
     const T ps = psg[(long)mem * ng + col];
     const T fvT = (T)sc.fv, qminT = (T)sc.qmin;
-    // column accessors, c = 1..nl top -> bottom
-    auto lvl = [&](int c) { return (long)(nl - c) * ng; };  // grid offset of column position c
+    // column positions c = 1..nl top -> bottom; this thread's are lg + 1 + 16 i
+    auto lvl = [&](int c) { return (long)(nl - c) * ng; };
     auto pint = [&](int c) { return (double)(ak[c - 1] + bk[c - 1] * ps); };
-    auto pmid = [&](int c) {
+    T tv0[SP_L], q0[SP_L], u0[SP_L], v0[SP_L];
+#pragma unroll
+    for (int i = 0; i < SP_L; i++) {
+        const long o = lvl(min(lg + 1 + 16 * i, nl));
+        tv0[i] = TV[o];
+        q0[i] = Q[o];
+        u0[i] = U[o];
+        v0[i] = V[o];
+    }
+    double precl = 0.0, pw = 0.0, ex[SP_L];
+#pragma unroll
+    for (int i = 0; i < SP_L; i++) {
+        const int c = lg + 1 + 16 * i;
+        if (c > nl) break;
         // Phillips layer pressure of pressure_data.f90:87-88 in the grid precision
-        return (double)phillips_prs(ak[c - 1] + bk[c - 1] * ps, ak[c] + bk[c] * ps, kappa);
-    };
-    auto tin = [&](int c) {  // T = Tv / (1 + fv max(qmin, q)) (phy_run_simple.f90:56)
-        const long o = lvl(c);
-        return (double)(TV[o] / (T(1) + fvT * fmax(qminT, Q[o])));
-    };
-    // large-scale condensation at one level: (t, q) -> (t, q), precipitation added
-    double precl = 0.0;
-    auto condense = [&](int c, double &t, double &q) {
-        const double pm = pmid(c);
+        const double pm = (double)phillips_prs(ak[c - 1] + bk[c - 1] * ps, ak[c] + bk[c] * ps, kappa);
+        // T = Tv / (1 + fv max(qmin, q)) (phy_run_simple.f90:56)
+        const double tin = (double)(tv0[i] / (T(1) + fvT * fmax(qminT, q0[i])));
+        double t = tin, q = (double)q0[i], u = (double)u0[i], v = (double)v0[i];
+        // large-scale condensation
         const double qsat = epsilo * e0 / pm * exp(-latvap / rh2o * ((1.0 / t) - 1.0 / T0));
         if (q > qsat) {
             const double tmp = 1.0 / dt * (q - qsat) / (1.0 + (latvap / cpair) * (epsilo * latvap * qsat / (rair * (t * t))));
@@ -1327,124 +1348,128 @@ __global__ __launch_bounds__(256) void k_simple_columns(
             q = q + (-tmp) * dt;
             precl = precl + tmp * (pint(c + 1) - pint(c)) / (gravit * rhow);
         }
-    };
-    const double lat = latd[col / nlon];
-    // za from the lowest level before any update (225-229)
-    const double zab = rair / gravit * tin(nl) * (1.0 + zvir * (double)Q[lvl(nl)]) * 0.5 * (log((double)ps) - log(pint(nl)));
-    double pw = 0.0;
-    auto finish = [&](int c, double t, double q, double u, double v) {
-        // Tv, changes and column water (phy_run_simple.f90:92-107)
-        const long o = lvl(c);
-        const double tv = t * (1.0 + sc.fv * fmax(sc.qmin, q));
-        DT[o] = (T)(tv - (double)TV[o]);
-        const T dq = (T)(q - (double)Q[o]);
-        DQ[o] = dq;
-        DU[o] = (T)(u - (double)U[o]);
-        DV[o] = (T)(v - (double)V[o]);
-        pw += (pint(c + 1) - pint(c)) * (double)(dq + Q[o]);
-    };
-    if (!sc.turbflux) {
-        for (int c = 1; c <= nl; c++) {
-            double t = tin(c), q = (double)Q[lvl(c)];
-            condense(c, t, q);
-            finish(c, t, q, (double)U[lvl(c)], (double)V[lvl(c)]);
+        if (sc.turbflux && c == nl) {
+            // za from the lowest level before any update (225-229); drag and eddy
+            // diffusivities (300-335); surface fluxes (344-366)
+            const double zab = rair / gravit * tin * (1.0 + zvir * (double)q0[i]) * 0.5 * (log((double)ps) - log(pint(nl)));
+            const double wind = sqrt(u * u + v * v), lat = latd[col / nlon];
+            const double cd = wind < v20 ? Cd0 + Cd1 * wind : Cm;
+            skm[cl] = cd * wind * zab;
+            ske[cl] = Csfc * wind * zab;
+            const double tsurf = simple_sst(sc.sst_mode, lat);
+            const double qsats = epsilo * e0 / (double)ps * exp(-latvap / rh2o * ((1.0 / tsurf) - 1.0 / T0));
+            u = u / (1.0 + cd * wind * dt / zab);
+            v = v / (1.0 + cd * wind * dt / zab);
+            t = (t + Csfc * wind * tsurf * dt / zab) / (1.0 + Csfc * wind * dt / zab);
+            q = (q + Csfc * wind * qsats * dt / zab) / (1.0 + Csfc * wind * dt / zab);
         }
-    } else {
-        // drag and eddy diffusivities from the lowest-level wind (300-335)
-        const double ub = (double)U[lvl(nl)], vb = (double)V[lvl(nl)];
-        const double wind = sqrt(ub * ub + vb * vb);
-        const double kes = Csfc * wind * zab;
-        double cd, kms;
-        if (wind < v20) {
-            cd = Cd0 + Cd1 * wind;
-            kms = cd * wind * zab;
-        } else {
-            cd = Cm;
-            kms = Cm * wind * zab;
-        }
-        auto prof = [&](int c) {  // taper above pbltop; c = nl + 1 is the surface
-            if (c == nl + 1) return 1.0;
-            const double pi_ = pint(c);
-            if (pi_ >= pbltop) return 1.0;
-            return exp(-((pbltop - pi_) * (pbltop - pi_)) / (pblconst * pblconst));
-        };
-        const double tsurf = simple_sst(sc.sst_mode, lat);
-        const double qsats = epsilo * e0 / (double)ps * exp(-latvap / rh2o * ((1.0 / tsurf) - 1.0 / T0));
-        // state after condensation (and, on the lowest level, the surface fluxes)
-        auto state = [&](int c, double &t, double &q, double &u, double &v) {
-            t = tin(c);
-            q = (double)Q[lvl(c)];
-            u = (double)U[lvl(c)];
-            v = (double)V[lvl(c)];
-            condense(c, t, q);
-            if (c == nl) {  // 344-366
-                u = u / (1.0 + cd * wind * dt / zab);
-                v = v / (1.0 + cd * wind * dt / zab);
-                t = (t + Csfc * wind * tsurf * dt / zab) / (1.0 + Csfc * wind * dt / zab);
-                q = (q + Csfc * wind * qsats * dt / zab) / (1.0 + Csfc * wind * dt / zab);
-            }
-        };
-        // upward elimination sweep c = nl..1 (407-431)
-        double tc, qc, uc, vc, ta, qa, ua, va;  // level c and level c-1 (above)
-        state(nl, tc, qc, uc, vc);
-        double ce1 = 0.0, cem1 = 0.0, cfu1 = 0.0, cfv1 = 0.0, cft1 = 0.0, cfq1 = 0.0;  // values at c + 1
-        double ca_c = 0.0, cam_c = 0.0;  // CA(c), CAm(c) from the interface below (0 at c = nl)
-        for (int c = nl; c >= 1; c--) {
-            // interface c (between c-1 and c): CC(c), CCm(c) and CA(c-1), CAm(c-1)
-            double cc_c = 0.0, ccm_c = 0.0, ca_up = 0.0, cam_up = 0.0;
+        st[c - 1][cl] = t;
+        sq[c - 1][cl] = q;
+        su[c - 1][cl] = u;
+        sv[c - 1][cl] = v;
+        srp[c - 1][cl] = pm;
+        ex[i] = 1.0;
+    }
+    if (sc.turbflux) {
+        __syncthreads();
+        // interface c (between c - 1 and c): the sweeps' coefficients are 1 / dp of the
+        // layer above or below times the diffusivity times Y (407-431)
+        double th[SP_L], rp[SP_L];
+#pragma unroll
+        for (int i = 0; i < SP_L; i++) {
+            const int c = lg + 1 + 16 * i;
+            if (c > nl) break;
+            const double pi_ = pint(c), pm = srp[c - 1][cl], t = st[c - 1][cl];
+            double y = 0.0;
             if (c >= 2) {
-                state(c - 1, ta, qa, ua, va);
-                const double rho = (pint(c) / (rair * (tc + ta) / 2.0));
-                const double dpm = pmid(c) - pmid(c - 1);
-                const double km = kms * prof(c), ke = kes * prof(c);
-                const double rpu = 1.0 / (pint(c) - pint(c - 1)), rpc = 1.0 / (pint(c + 1) - pint(c));
-                cam_up = rpu * dt * gravit * gravit * km * rho * rho / dpm;
-                ccm_c = rpc * dt * gravit * gravit * km * rho * rho / dpm;
-                ca_up = rpu * dt * gravit * gravit * ke * rho * rho / dpm;
-                cc_c = rpc * dt * gravit * gravit * ke * rho * rho / dpm;
+                const double rho = pi_ / (rair * (t + st[c - 2][cl]) / 2.0);
+                double prof = 1.0;  // taper above pbltop
+                if (pi_ < pbltop) prof = exp(-((pbltop - pi_) * (pbltop - pi_)) / (pblconst * pblconst));
+                y = dt * gravit * gravit * rho * rho / (pm - srp[c - 2][cl]) * prof;
             }
-            const double dh = 1.0 + ca_c + cc_c - ca_c * ce1;
-            const double dm = 1.0 + cam_c + ccm_c - cam_c * cem1;
-            const double ce = cc_c / dh, cem = ccm_c / dm;
-            const double cfu = (uc + cam_c * cfu1) / dm, cfv = (vc + cam_c * cfv1) / dm;
-            const double cft = (pow(p0 / pmid(c), rk) * tc + ca_c * cft1) / dh;
-            const double cfq = (qc + ca_c * cfq1) / dh;
-            const long o = lvl(c);
-            CE[o] = (T)ce;
-            CEM[o] = (T)cem;
-            DU[o] = (T)cfu;
-            DV[o] = (T)cfv;
-            DT[o] = (T)cft;
-            DQ[o] = (T)cfq;
-            ce1 = ce; cem1 = cem; cfu1 = cfu; cfv1 = cfv; cft1 = cft; cfq1 = cfq;
-            ca_c = ca_up; cam_c = cam_up;
-            tc = ta; qc = qa; uc = ua; vc = va;
+            sy[c - 1][cl] = y;
+            rp[i] = 1.0 / (pint(c + 1) - pi_);
+            const double pf = pow(p0 / pm, rk);
+            th[i] = pf * t;
+            ex[i] = 1.0 / pf;
         }
-        // downward back-substitution c = 1..nl (432-447)
-        double tp = 0.0, qp = 0.0, up = 0.0, vp = 0.0, pmp = 0.0;
-        for (int c = 1; c <= nl; c++) {
-            const long o = lvl(c);
-            const double cfu = (double)DU[o], cfv = (double)DV[o], cft = (double)DT[o], cfq = (double)DQ[o];
-            const double pm = pmid(c);
-            double u, v, t, q;
-            if (c == 1) {
-                u = cfu;
-                v = cfv;
-                t = cft * pow(pm / p0, rk);
-                q = cfq;
-            } else {
-                const double ce = (double)CE[o], cem = (double)CEM[o];
-                u = cem * up + cfu;
-                v = cem * vp + cfv;
-                t = (ce * tp * pow(p0 / pmp, rk) + cft) * pow(pm / p0, rk);
-                q = ce * qp + cfq;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < SP_L; i++)
+            if (lg + 1 + 16 * i <= nl) {
+                st[lg + 16 * i][cl] = th[i];
+                srp[lg + 16 * i][cl] = rp[i];
             }
-            finish(c, t, q, u, v);
-            tp = t; qp = q; up = u; vp = v; pmp = pm;
+        __syncthreads();
+        if (tid < 4 * SP_C) {
+            // lanes of one wavefront in step: u, v (momentum), T, q (heat) of each column
+            const int f = tid / SP_C;
+            double(*x)[SP_C] = f == 0 ? su : f == 1 ? sv : f == 2 ? st : sq;
+            double(*e)[SP_C] = f < 2 ? sy : srp;  // where this sweep's CE goes
+            const double k = f < 2 ? skm[cl] : ske[cl];
+            // lanes that share a row write the same CE, one step after all have read it;
+            // a step's values are loaded a step ahead, above what it stores
+            double ce1 = 0.0, cf1 = 0.0, ca = 0.0;  // CE, CF at c + 1; CA(c), zero at c = nl
+            double rp = srp[nl - 1][cl], y = sy[nl - 1][cl], rhs = x[nl - 1][cl];
+            for (int c = nl; c >= 1; c--) {  // upward elimination
+                const int up = max(c - 2, 0);
+                const double rpn = srp[up][cl], yn = sy[up][cl], rhsn = x[up][cl];
+                const double cc = rp * (k * y);
+                const double r = 1.0 / (1.0 + ca + cc - ca * ce1);
+                ce1 = cc * r;
+                cf1 = (rhs + ca * cf1) * r;
+                ca = rpn * (k * y);  // unused above the top
+                e[c - 1][cl] = ce1;
+                x[c - 1][cl] = cf1;
+                rp = rpn;
+                y = yn;
+                rhs = rhsn;
+            }
+            double xp = 0.0;
+            int c = 0;
+            for (; c + 8 <= nl; c += 8) {  // downward back-substitution (432-447)
+                double ev[8], xv[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    ev[j] = e[c + j][cl];
+                    xv[j] = x[c + j][cl];
+                }
+#pragma unroll
+                for (int j = 0; j < 8; j++) x[c + j][cl] = xp = ev[j] * xp + xv[j];
+            }
+            for (; c < nl; c++) x[c][cl] = xp = e[c][cl] * xp + x[c][cl];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < SP_L; i++) {
+        const int c = lg + 1 + 16 * i;
+        if (c > nl) break;
+        // Tv, changes and column water (phy_run_simple.f90:92-107)
+        const double t = st[c - 1][cl] * ex[i], q = sq[c - 1][cl];
+        const long o = lvl(c);
+        const T dq = (T)(q - (double)q0[i]);
+        pw += (pint(c + 1) - pint(c)) * (double)(dq + q0[i]);
+        if (valid) {
+            const double tv = t * (1.0 + sc.fv * fmax(sc.qmin, q));
+            DT[o] = (T)(tv - (double)tv0[i]);
+            DQ[o] = dq;
+            DU[o] = (T)(su[c - 1][cl] - (double)u0[i]);
+            DV[o] = (T)(sv[c - 1][cl] - (double)v0[i]);
         }
     }
-    pwat_out[(long)mem * ng + col] = (T)(pw / sc.grav);
-    precip_out[(long)mem * ng + col] = (T)(precl * 1000.0);
+    __syncthreads();
+    srp[lg][cl] = pw;
+    sy[lg][cl] = precl;
+    __syncthreads();
+    if (lg == 0 && valid) {
+        for (int g = 1; g < 16; g++) {
+            pw += srp[g][cl];
+            precl += sy[g][cl];
+        }
+        pwat_out[(long)mem * ng + col] = (T)(pw / sc.grav);
+        precip_out[(long)mem * ng + col] = (T)(precl * 1000.0);
+    }
 }
 
 // ---- learned column physics: features, targets, application, judge --------
@@ -2885,12 +2910,11 @@ template <typename T> int Engine<T>::dyn_init() {
     B->colq = dalloc<T>((size_t)nm * ng);
     B->pwat = dalloc<T>((size_t)nm * ng);
     B->precip = dalloc<T>((size_t)nm * ng);
-    B->pblscr = dalloc<T>(cfg.physics == GFSDC_PHYS_SIMPLE ? (size_t)nm * 2 * nl * ng : 1);
     B->hsdyn = dalloc<int>(8);
     void *ptrs[] = {B->spec, B->spec0, B->ten[0], B->ten[1], B->ten[2], B->lin[0], B->lin[1], B->lin[2],
                     B->tphys, B->topo, B->gsyn, B->gan, B->etadot, B->dlnpdt, B->psg, B->dlnpsdt, B->dphisdx,
                     B->dphisdy, B->pdryini, B->pmean, B->diag, B->pspart, B->pwsum, B->colq, B->pwat,
-                    B->precip, B->pblscr, B->gmean, B->clock, B->hsdyn};
+                    B->precip, B->gmean, B->clock, B->hsdyn};
     for (void *p : ptrs)
         if (!p) {
             set_error("device allocation failed for the dycore state");
@@ -3153,7 +3177,7 @@ template <typename T> void Engine<T>::dyn_destroy() {
                     B->ak, B->bk, B->ck, B->dbk, B->sinlat, B->coslat, B->areaw, B->kbydeg, B->degree, B->si_tiles,
                     B->pdryini, B->pmean, B->pspart, B->diag, B->sdesc, B->adesc_dyn, B->adesc_hs, B->adesc_hsu,
                     B->rflag_syn,
-                    B->rflag_an, B->rflag_hs, B->pwsum, B->colq, B->pwat, B->precip, B->pblscr, B->latd,
+                    B->rflag_an, B->rflag_hs, B->pwsum, B->colq, B->pwat, B->precip, B->latd,
                     B->adesc_sp, B->rflag_sp, B->tpat, B->tpat_var, B->tpat_vf, B->tpat_ctr, B->ds_x, B->ds_y,
                     B->nrm, B->xin, B->yout, B->tbx, B->tby, B->ganj, B->pwatj, B->precipj, B->jpart, B->jstat,
                     B->jflag, B->jctr, B->gmean, B->dak, B->sdesc_ph, B->rflag_ph, B->slot_ph, B->sdesc_hl,
@@ -3440,13 +3464,10 @@ template <typename T> struct Step {
     void simple_columns(ColSel cs = ColSel{0, nullptr, nullptr}, void *gan = nullptr, void *pwat = nullptr,
                         void *precip = nullptr, const char *name = "simple_columns") {
         const gfsdc_cfg &c = E.cfg;
-        long nthreads = cs.stride > 0 ? B.ng / cs.stride : B.ng;
-        // a column is a long serial computation: the few judged columns are spread
-        // over as many CUs as possible (one wave per workgroup)
-        const int bs = cs.stride > 0 ? 64 : 256;
-        dim3 g((unsigned)((nthreads + bs - 1) / bs), B.nm);
-        hipLaunchKernelGGL(k_simple_columns<T>, g, dim3(bs), 0, s, (const T *)B.gsyn, (const T *)B.psg,
-                           (T *)(gan ? gan : B.gan), (T *)B.pblscr, (T *)(pwat ? pwat : B.pwat),
+        const long ncol = cs.stride > 0 ? B.ng / cs.stride : B.ng;
+        dim3 g((unsigned)((ncol + SP_C - 1) / SP_C), B.nm);
+        hipLaunchKernelGGL(k_simple_columns<T>, g, dim3(256), 0, s, (const T *)B.gsyn, (const T *)B.psg,
+                           (T *)(gan ? gan : B.gan), (T *)(pwat ? pwat : B.pwat),
                            (T *)(precip ? precip : B.precip), (const T *)B.ak, (const T *)B.bk,
                            (const double *)B.latd, B.nl, B.ntr, B.nsyn, B.nsp, B.ng, E.plan.nlon, (T)(c.rd / c.cp),
                            simple_cfg(), cs);

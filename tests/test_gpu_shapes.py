@@ -205,3 +205,42 @@ def test_bf16x3_tiles(grid, nf):
     ref = o.spectogrd(q)
     assert rel(g.spectogrd(q.astype(np.complex64), dtype=1), ref) < 3e-5
     assert rel(g.grdtospec(ref.astype(np.float32), dtype=1), o.grdtospec(ref)) < 3e-5
+
+
+# levels below, on and past the 16 of a round; a member's columns on and off the 16 of a workgroup
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("grid,nlev,turb", [((64, 32, 21), 2, 1), ((36, 18, 11), 15, 1), ((72, 36, 23), 16, 0),
+                                            ((36, 18, 11), 17, 1), ((64, 32, 21), 33, 1), ((36, 18, 11), 64, 1),
+                                            ((64, 32, 21), 64, 0)])
+def test_simple_columns_every_round(grid, nlev, turb, prec):
+    """Simple physics of two members against the oracle at the bounds of test_gpu_moist (FP64 1e-9 of the largest
+    value, FP32 2e-3 in the 2-norm: a point at saturation may condense on one side alone)."""
+    import cases
+    import gfsdc
+    nlon, nlat, T = grid
+    ak, bk = levels.hybrid_levels(nlev)
+    kw = dict(ntrac=1, physics=2, simple_test=2, turbflux=turb)
+    o = O.Model(nlon, nlat, T, nlev, ak, bk, 600.0, **kw)
+    p = gfsdc.FP64 if prec == "fp64" else gfsdc.FP32
+    g = gfsdc.Context(nlon, nlat, T, p, nlev=nlev, ak=ak, bk=bk, dt=600.0, nmem=2, **kw)
+    st = []
+    for mem in range(2):
+        vrt, div, tv, lnps = cases.perturbed_state(o.sht.degree, o.sht.order, nlev, seed=3 + mem, amp=0.5)
+        q = o.sht.grdtospec(cases.moist_grid(o.sht.lats, nlon, ak, bk, seed=5 + mem))
+        st.append((vrt[0], div[0], tv[0], lnps[0], q[None]))
+    a = [np.stack(x) for x in zip(*st)]
+    g.set_state(a[0], a[1], a[2], a[3], trac=a[4])
+    g.getdyntend(3, inverse_only=True)
+    tg = g.simple_phytend()
+    far, tol = (rel, 1e-9) if prec == "fp64" else (lambda x, y: np.linalg.norm(x - y) / max(np.linalg.norm(y), 1e-300), 2e-3)
+    for mem in range(2):
+        o.set_state(st[mem][0], st[mem][1], st[mem][2], st[mem][3], st[mem][4])
+        o.getdyntend(3, inverse_only=True)
+        to = o.simple_phytend()
+        pairs = {k: (tg[k][mem], to[k]) for k in ("dvrt", "ddiv", "dtv", "dtrac")}
+        pairs |= {k: (g.grid(k)[mem].ravel(), o.grid(k).ravel()) for k in ("precip", "pwat")}
+        for k, (x, y) in pairs.items():
+            if np.abs(y).max() > 0:
+                assert far(x, y) < tol, (k, mem, far(x, y))
+            else:  # two layers do not condense; without the boundary layer the wind is untouched
+                assert np.abs(x).max() == 0, (k, mem)
