@@ -81,7 +81,8 @@ struct DycoreBuffers {
     int n_si_tiles = 0;
     int *degree = nullptr;                       // degree of coefficient k
     double *pdryini = nullptr, *pmean = nullptr; // FP64 per member
-    double *pspart = nullptr;                    // FP64 partial sums (2 x PS_BLOCKS per member)
+    double *pspart = nullptr;                    // FP64 partial sums and ranges (4 x PS_BLOCKS per member)
+    unsigned *psdone = nullptr;                  // workgroups and members that have arrived (k_area), zero between calls
     double *pwsum = nullptr;                     // FP64 area sum of pwat per member
     void *colq = nullptr;                        // T per member ng: column tracer mass sum(dpk q)
     void *pwat = nullptr, *precip = nullptr;     // T per member ng (simple physics)
@@ -162,7 +163,7 @@ struct DycoreBuffers {
     SynthDesc *sdesc_hl = nullptr;
     unsigned char *rflag_hl = nullptr;
     int *slot_hl = nullptr;
-    // device counts of the lean pass, written by k_area_final: [0] fields of
+    // device counts of the lean pass, written by k_area: [0] fields of
     // the vorticity / divergence synthesis that follows the drag's count (0
     // where the first synthesis already held every level with drag), [1]
     // Held-Suarez forcing fields to analyse, [2] nact, the levels counted from
@@ -199,6 +200,11 @@ static void drop_graph(DycoreBuffers *B) {
 
 // ---------------------------------------------------------------------------
 // kernels
+
+// ps = exp(q_00 / sqrt(4 pi) + ln ps'), rounded alike in every kernel that forms it
+template <typename T> __device__ __forceinline__ T full_ps(T q00, T lnps) {
+    return (T)exp(fma((double)q00, 0.28209479177387814, (double)lnps));
+}
 
 // Layer coefficients of calc_pressdata / getpresgrad for K >= 2 (pressure_data.f90:
 // 76-82, dyn_run.f90:393-410): rlnp = ln(p2/p1), alfa = 1 - p1/dp rlnp,
@@ -371,8 +377,8 @@ __global__ __launch_bounds__(ColCfg<T>::NC * ColCfg<T>::CH, sizeof(T) * LPC <= 1
             }
         }
     const T dpx = ld(LNPS, 1), dpy = ld(LNPS, 2);
-    const double c0 = (double)spec[(long)mem * nfs + 3L * nl + (long)ntr * nl].x * 0.28209479177387814;  // 1/sqrt(4 pi)
-    const T ps = (T)exp(c0 + (double)ld(LNPS, 0));
+    const T c00 = spec[(long)mem * nfs + 3L * nl + (long)ntr * nl].x;
+    const T ps = full_ps(c00, ld(LNPS, 0));
     const T gpx = ps * dpx, gpy = ps * dpy;
     const T alfa1 = T(SGLF(0.69314718055994530942)), rlnp1 = T(SGLF(99999.99));
     __syncthreads();  // the level tables
@@ -702,8 +708,8 @@ __global__ __launch_bounds__(256) void k_columns_serial(
     const T *QX = Q + (long)ntr * nl * ng, *QY = QX + (long)ntr * nl * ng;
     const T *LNPS = G + (7L + 3L * ntr) * nl * ng;
     const T dpx = LNPS[ng], dpy = LNPS[2 * ng];
-    const double c0 = (double)spec[(long)mem * nfs + 3L * nl + (long)ntr * nl].x * 0.28209479177387814;  // 1/sqrt(4 pi)
-    const T ps = (T)exp(c0 + (double)LNPS[0]);
+    const T c00 = spec[(long)mem * nfs + 3L * nl + (long)ntr * nl].x;
+    const T ps = full_ps(c00, LNPS[0]);
     T *ET = etadot + (long)mem * (nl + 1) * ng + col;
     T *WD = dlnpdt + (long)mem * nl * ng + col;
     const T alfa1 = T(SGLF(0.69314718055994530942)), rlnp1 = T(SGLF(99999.99));
@@ -979,19 +985,6 @@ __host__ __device__ inline int hs_field(int nl, int nm, int mem, int kind, int k
     return kind == HS_T ? mem * (nl + 1) + k : nm * (nl + 1) + 2 * (k * nm + mem) + (kind - HS_VRT);
 }
 
-// Surface pressure of the lean Held-Suarez pass: ps = exp(mean + ln ps'), the
-// mean from the spectral state in FP64, as the column kernel forms it.
-template <typename T>
-__global__ __launch_bounds__(256) void k_psg(const T *__restrict__ gsyn, const cplx<T> *__restrict__ spec,
-                                             T *__restrict__ psg, int nl, int ntr, int nsyn, int nfs, long ng) {
-    const long col = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int mem = blockIdx.y;
-    if (col >= ng) return;
-    const T *LNPS = gsyn + (long)mem * nsyn * ng + (7L + 3L * ntr) * nl * ng + col;
-    const double c0 = (double)spec[(long)mem * nfs + 3L * nl + (long)ntr * nl].x * 0.28209479177387814;  // 1/sqrt(4 pi)
-    psg[(long)mem * ng + col] = (T)exp(c0 + (double)LNPS[0]);
-}
-
 // The levels on which the Held-Suarez drag can act, for the lean pass.
 // phy_run_hs.f90:52-58 sets the drag profile max(0, (p_k / ps - sigbot) /
 // (1 - sigbot)): where p_k / ps stays below sigbot in every column, a level's
@@ -1001,7 +994,7 @@ __global__ __launch_bounds__(256) void k_psg(const T *__restrict__ gsyn, const c
 // so over all columns it is largest at the least or the greatest ps (1 / ps =
 // rmin, rmax). A level where it stays below 0.999 sigbot at both (a margin far
 // above the rounding of p_k) has no drag. The lean pass takes the levels up
-// to the highest other one (nact, which k_area_final turns into the counts the
+// to the highest other one (nact, which k_area turns into the counts the
 // pass's kernels read).
 template <typename T>
 __device__ inline bool hs_level_drags(int k, double rmin, double rmax, const T *__restrict__ ak,
@@ -1108,110 +1101,138 @@ __global__ __launch_bounds__(256) void k_hs_columns(const T *__restrict__ gsyn, 
 
 // Area-weighted global sums per member in FP64 (areawts sum to 1, so these are
 // global means): S_a of field a (ps) and, when b is given, S_b of field b (the
-// column tracer mass, or pwat). Two deterministic stages: PS_BLOCKS partial
-// sums per member, then a fixed-order final sum. The final stage optionally
-// sets pdryini = S_a - S_b where it is still 0 (dyn_run.f90:135-149).
+// column tracer mass, or pwat); pdryini = S_a - S_b where it is still 0
+// (dyn_run.f90:135-149). PS_BLOCKS workgroups per member write partial sums, and
+// the last of them to arrive adds these up in the order of the workgroups, so the
+// result does not depend on which one it is. part holds four values per (member,
+// workgroup): S_a, S_b and the least and the greatest a of its columns; done
+// counts the workgroups that have arrived, per member, and after those the
+// members, and is left at zero.
+// With PSG (the lean pass) a is formed here from ln ps, as the column kernel
+// forms it: ps = exp(mean + ln ps'), the mean from the spectral state in FP64; and
+// the last member's last workgroup takes the range of ps over all members, finds
+// the levels with drag from it (hs_level_drags) and writes the lean pass's counts
+// (cnt[0..4], as DycoreBuffers::hsdyn describes them).
+// Bound by latency: the lean pass's ps, sums, range and counts take 8.8 us at T42
+// FP64 and 12.8 us at T254 FP32 as one launch (13.5 and 17 us as three, without
+// the gaps between them); the dynamics' call, once the dry mass is set, ends at once.
 constexpr int PS_BLOCKS = 128;
-static_assert(MAXLEV <= PS_BLOCKS, "k_area_final tests one level per thread");
+static_assert(MAXLEV <= PS_BLOCKS, "k_area tests one level per thread");
 
-// part holds four values per (member, block): S_a, S_b and the least and the
-// greatest a of the block's columns
-template <typename T>
-__global__ __launch_bounds__(256) void k_area_partial(const T *__restrict__ a, const T *__restrict__ b,
-                                                      const double *__restrict__ areaw, double *__restrict__ part,
-                                                      long ng, int nlon) {
-    const int mem = blockIdx.y;
-    const T *pa = a + (long)mem * ng;
+template <typename T, bool PSG>
+__global__ __launch_bounds__(256) void k_area(T *__restrict__ a, const T *__restrict__ b,
+                                              const double *__restrict__ areaw, double *__restrict__ part,
+                                              unsigned *__restrict__ done, long ng, int nlon,
+                                              double *__restrict__ out_a, double *__restrict__ out_b,
+                                              double *__restrict__ pdryini, const T *__restrict__ ak,
+                                              const T *__restrict__ bk, int nl, int *__restrict__ cnt,
+                                              const T *__restrict__ gsyn, const cplx<T> *__restrict__ spec, int ntr,
+                                              int nsyn, int nfs) {
+    const int mem = blockIdx.y, nm = gridDim.y, tid = threadIdx.x;
+    // nothing to find out about a member whose dry mass is set
+    if (!PSG && !out_a && !out_b && (!pdryini || pdryini[mem] != 0.0)) return;
+    T *pa = a + (long)mem * ng;
     const T *pb = b ? b + (long)mem * ng : nullptr;
+    const T *in = PSG ? gsyn + (long)mem * nsyn * ng + (7L + 3L * ntr) * nl * ng : pa;
+    const T c00 = PSG ? spec[(long)mem * nfs + 3L * nl + (long)ntr * nl].x : T(0);
     double sa = 0.0, sb = 0.0, lo = INFINITY, hi = -INFINITY;
-    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < ng; i += (long)PS_BLOCKS * 256) {
-        const double w = areaw[i / nlon], v = (double)pa[i];
-        sa += w * v;
-        lo = fmin(lo, v);
-        hi = fmax(hi, v);
-        if (pb) sb += w * (double)pb[i];
+    constexpr int AB = 4;  // columns whose loads are in flight together
+    const long step = (long)PS_BLOCKS * 256;
+    for (long i0 = (long)blockIdx.x * 256 + tid; i0 < ng; i0 += AB * step) {
+        T x[AB], y[AB];
+        double w[AB];
+#pragma unroll
+        for (int u = 0; u < AB; u++) {
+            const long i = min(i0 + u * step, ng - 1);
+            x[u] = in[i];
+            y[u] = pb ? pb[i] : T(0);
+            w[u] = areaw[(unsigned)i / (unsigned)nlon];  // a member has less than 2^31 columns
+        }
+#pragma unroll
+        for (int u = 0; u < AB; u++) {
+            const long i = i0 + u * step;
+            if (i >= ng) break;
+            if constexpr (PSG) pa[i] = x[u] = full_ps(c00, x[u]);
+            const double v = (double)x[u];
+            sa += w[u] * v;
+            lo = fmin(lo, v);
+            hi = fmax(hi, v);
+            if (pb) sb += w[u] * (double)y[u];
+        }
     }
     __shared__ double ra[256], rb[256], rl[256], rh[256];
-    ra[threadIdx.x] = sa;
-    rb[threadIdx.x] = sb;
-    rl[threadIdx.x] = lo;
-    rh[threadIdx.x] = hi;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            ra[threadIdx.x] += ra[threadIdx.x + w];
-            rb[threadIdx.x] += rb[threadIdx.x + w];
-            rl[threadIdx.x] = fmin(rl[threadIdx.x], rl[threadIdx.x + w]);
-            rh[threadIdx.x] = fmax(rh[threadIdx.x], rh[threadIdx.x + w]);
+    __shared__ int last;
+    auto reduce = [&](int n) {
+        for (int w = n / 2; w > 0; w >>= 1) {
+            __syncthreads();
+            if (tid < w) {
+                ra[tid] += ra[tid + w];
+                rb[tid] += rb[tid + w];
+                rl[tid] = fmin(rl[tid], rl[tid + w]);
+                rh[tid] = fmax(rh[tid], rh[tid + w]);
+            }
         }
         __syncthreads();
-    }
-    if (threadIdx.x == 0) {
+    };
+    // counts this workgroup in (thread 0) and says whether it was the n-th. Thread 0 has
+    // stored the workgroup's part with device-scope (write-through) stores and waits
+    // for them here, and they are read with device-scope loads: a release fence would
+    // write back the L2 of the XCD for each workgroup (16 members at T126: 60 us)
+    auto arrive = [&](unsigned *at, int n) {
+        if (tid == 0) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            last = __hip_atomic_fetch_add(at, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)n - 1u;
+            asm volatile("" ::: "memory");
+            if (last) __hip_atomic_store(at, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        return last != 0;
+    };
+    auto get = [&](long i) { return __hip_atomic_load(part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    ra[tid] = sa;
+    rb[tid] = sb;
+    rl[tid] = lo;
+    rh[tid] = hi;
+    reduce(256);
+    if (tid == 0) {
         double *q = part + 4 * (mem * PS_BLOCKS + blockIdx.x);
-        q[0] = ra[0];
-        q[1] = rb[0];
-        q[2] = rl[0];
-        q[3] = rh[0];
+        const double r[4] = {ra[0], rb[0], rl[0], rh[0]};
+#pragma unroll
+        for (int u = 0; u < 4; u++) __hip_atomic_store(q + u, r[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-}
-
-// One workgroup per member sums its partials; with cnt, workgroup 0 also
-// takes the least and greatest a (ps) over every member and block, finds the
-// levels with drag from them (hs_level_drags) and writes the lean Held-Suarez
-// pass's counts (cnt[0..4], as DycoreBuffers::hsdyn describes them).
-template <typename T>
-__global__ __launch_bounds__(PS_BLOCKS) void k_area_final(const double *__restrict__ part, double *__restrict__ out_a,
-                                                           double *__restrict__ out_b, double *__restrict__ pdryini,
-                                                           const T *__restrict__ ak, const T *__restrict__ bk, int nl,
-                                                           int *__restrict__ cnt) {
-    const int mem = blockIdx.x, nm = gridDim.x;
-    __shared__ double ra[PS_BLOCKS], rb[PS_BLOCKS];
-    ra[threadIdx.x] = part[4 * (mem * PS_BLOCKS + threadIdx.x)];
-    rb[threadIdx.x] = part[4 * (mem * PS_BLOCKS + threadIdx.x) + 1];
-    __syncthreads();
-    for (int w = PS_BLOCKS / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            ra[threadIdx.x] += ra[threadIdx.x + w];
-            rb[threadIdx.x] += rb[threadIdx.x + w];
-        }
-        __syncthreads();
+    if (!arrive(done + mem, PS_BLOCKS)) return;
+    if (tid < PS_BLOCKS) {
+        ra[tid] = get(4 * (mem * PS_BLOCKS + tid));
+        rb[tid] = get(4 * (mem * PS_BLOCKS + tid) + 1);
     }
-    if (threadIdx.x == 0) {
+    reduce(PS_BLOCKS);
+    if (tid == 0) {
         if (out_a) out_a[mem] = ra[0];
         if (out_b) out_b[mem] = rb[0];
         if (pdryini && pdryini[mem] == 0.0) pdryini[mem] = ra[0] - rb[0];
     }
-    if (cnt && mem == 0) {
-        double lo = INFINITY, hi = -INFINITY;
-        for (int i = threadIdx.x; i < nm * PS_BLOCKS; i += PS_BLOCKS) {
-            lo = fmin(lo, part[4 * i + 2]);
-            hi = fmax(hi, part[4 * i + 3]);
+    if constexpr (PSG) {
+        __syncthreads();  // last, ra and rb are read
+        if (!arrive(done + nm, nm)) return;
+        lo = INFINITY;
+        hi = -INFINITY;
+        for (int i = tid; i < nm * PS_BLOCKS; i += 256) {
+            lo = fmin(lo, get(4 * i + 2));
+            hi = fmax(hi, get(4 * i + 3));
         }
-        __syncthreads();  // ra, rb reused
-        ra[threadIdx.x] = lo;
-        rb[threadIdx.x] = hi;
-        __syncthreads();
-        for (int w = PS_BLOCKS / 2; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) {
-                ra[threadIdx.x] = fmin(ra[threadIdx.x], ra[threadIdx.x + w]);
-                rb[threadIdx.x] = fmax(rb[threadIdx.x], rb[threadIdx.x + w]);
-            }
-            __syncthreads();
-        }
-        // one level per thread (nl <= MAXLEV <= PS_BLOCKS); every level for a
-        // state without a finite positive ps
-        const double pmin = ra[0], pmax = rb[0];
+        rl[tid] = lo;
+        rh[tid] = hi;
+        reduce(256);
+        // one level per thread; every level for a state without a finite positive ps
+        const double pmin = rl[0], pmax = rh[0];
         const bool ok = pmin > 0.0 && pmax < INFINITY;
-        const int k = threadIdx.x;
-        __shared__ int top[PS_BLOCKS];
-        top[k] = k < nl && (!ok || hs_level_drags(k, 1.0 / pmin, 1.0 / pmax, ak, bk, nl)) ? k + 1 : 0;
+        __shared__ int top;
+        if (tid == 0) top = 0;
         __syncthreads();
-        for (int w = PS_BLOCKS / 2; w > 0; w >>= 1) {
-            if (k < w) top[k] = max(top[k], top[k + w]);
-            __syncthreads();
-        }
-        if (k == 0) {
-            const int nact = top[0], took = cnt[4], next = min(nl, nact + 1);
+        if (tid < nl && (!ok || hs_level_drags(tid, 1.0 / pmin, 1.0 / pmax, ak, bk, nl))) atomicMax(&top, tid + 1);
+        __syncthreads();
+        if (tid == 0) {
+            const int nact = top, took = cnt[4], next = min(nl, nact + 1);
             cnt[0] = nact > took ? 2 * nm * nact : 0;
             cnt[1] = nm * (nl + 1) + 2 * nm * nact;
             cnt[2] = nact;
@@ -2904,6 +2925,7 @@ template <typename T> int Engine<T>::dyn_init() {
     B->pdryini = dalloc<double>(nm);
     B->pmean = dalloc<double>(nm);
     B->pspart = dalloc<double>((size_t)nm * PS_BLOCKS * 4);
+    B->psdone = dalloc<unsigned>(nm + 1);
     B->pwsum = dalloc<double>(nm);
     B->diag = dalloc<double>(4 * nm);
     B->clock = dalloc<double>(1);
@@ -2913,7 +2935,7 @@ template <typename T> int Engine<T>::dyn_init() {
     B->hsdyn = dalloc<int>(8);
     void *ptrs[] = {B->spec, B->spec0, B->ten[0], B->ten[1], B->ten[2], B->lin[0], B->lin[1], B->lin[2],
                     B->tphys, B->topo, B->gsyn, B->gan, B->etadot, B->dlnpdt, B->psg, B->dlnpsdt, B->dphisdx,
-                    B->dphisdy, B->pdryini, B->pmean, B->diag, B->pspart, B->pwsum, B->colq, B->pwat,
+                    B->dphisdy, B->pdryini, B->pmean, B->diag, B->pspart, B->psdone, B->pwsum, B->colq, B->pwat,
                     B->precip, B->gmean, B->clock, B->hsdyn};
     for (void *p : ptrs)
         if (!p) {
@@ -2931,6 +2953,7 @@ template <typename T> int Engine<T>::dyn_init() {
     GFSDC_CHECK(hipMemsetAsync(B->pwsum, 0, sizeof(double) * nm, stream));
     GFSDC_CHECK(hipMemsetAsync(B->gmean, 0, sizeof(T) * nm * B->nsyn, stream));
     GFSDC_CHECK(hipMemsetAsync(B->hsdyn, 0, sizeof(int) * 8, stream));
+    GFSDC_CHECK(hipMemsetAsync(B->psdone, 0, sizeof(unsigned) * (nm + 1), stream));
     Work<T> *W = new Work<T>();
     B->Work = W;
     if ((rc = work_alloc(*W, plan, nm * std::max(B->nsyn, B->nan)))) return rc;
@@ -3175,7 +3198,7 @@ template <typename T> void Engine<T>::dyn_destroy() {
                     B->tphys, B->gsyn, B->gan, B->etadot, B->dlnpdt, B->psg, B->dlnpsdt, B->dphisdx,
                     B->dphisdy, B->topo, B->at, B->bt, B->dt3, B->sv, B->tor, B->disspec, B->diffp, B->dmpp,
                     B->ak, B->bk, B->ck, B->dbk, B->sinlat, B->coslat, B->areaw, B->kbydeg, B->degree, B->si_tiles,
-                    B->pdryini, B->pmean, B->pspart, B->diag, B->sdesc, B->adesc_dyn, B->adesc_hs, B->adesc_hsu,
+                    B->pdryini, B->pmean, B->pspart, B->psdone, B->diag, B->sdesc, B->adesc_dyn, B->adesc_hs, B->adesc_hsu,
                     B->rflag_syn,
                     B->rflag_an, B->rflag_hs, B->pwsum, B->colq, B->pwat, B->precip, B->latd,
                     B->adesc_sp, B->rflag_sp, B->tpat, B->tpat_var, B->tpat_vf, B->tpat_ctr, B->ds_x, B->ds_y,
@@ -3259,12 +3282,9 @@ template <typename T> struct Step {
         launch_fft_synth(p, W.fs, W.ldc, (T *)B.gsyn, B.ng, nf, B.rflag_hl, s, (const T *)B.gmean, B.slot_hl, 0,
                          B.hsdyn + 3);
         mark("fft_synth");
-        dim3 g((unsigned)((B.ng + 255) / 256), B.nm);
-        hipLaunchKernelGGL(k_psg<T>, g, dim3(256), 0, s, (const T *)B.gsyn, spec, (T *)B.psg, B.nl, B.ntr, B.nsyn,
-                           B.nfs, B.ng);
+        // ps, the global means of the forcing's mass fixer, and the drag's levels
+        area<true>(nullptr, E.cfg.massfix ? B.pmean : (double *)nullptr, nullptr, nullptr);
         mark("psg");
-        // the global means of the forcing's mass fixer, and the drag's levels
-        area_sums(nullptr, E.cfg.massfix ? B.pmean : (double *)nullptr, nullptr, false, true);
         launch_synth_gather(p, spec, 1, sk, B.sdesc_hl + na, B.nhlb, W.sx, W.ldc, 1.0, s, (T *)nullptr, B.hsdyn);
         mark("synth_gather_more");
         launch_leg_synth(p, W.sx, W.ldc, W.fs, W.ldc, 2 * B.nhlb, s, B.hsdyn);
@@ -3321,14 +3341,15 @@ template <typename T> struct Step {
         launch(B.ntr > 0 ? mode(std::true_type()) : mode(std::false_type()), (unsigned)((B.ng + NC - 1) / NC), NC * CH);
         mark(inverse_only ? "columns_inverse" : "columns");
     }
-    // FP64 area sums: S(psg) -> pmean, S(b) -> bsum; pdryini = S(psg) - S(b) where 0;
-    // with drag_count also the lean Held-Suarez pass's counts (hsdyn) from psg's range
-    void area_sums(const void *b, double *pmean, double *bsum, bool set_pdry, bool drag_count = false) {
-        hipLaunchKernelGGL(k_area_partial<T>, dim3(PS_BLOCKS, B.nm), dim3(256), 0, s, (const T *)B.psg,
-                           (const T *)b, (const double *)B.areaw, B.pspart, B.ng, E.plan.nlon);
-        hipLaunchKernelGGL(k_area_final<T>, dim3(B.nm), dim3(PS_BLOCKS), 0, s, (const double *)B.pspart, pmean,
-                           bsum, set_pdry ? B.pdryini : (double *)nullptr, (const T *)B.ak, (const T *)B.bk, B.nl,
-                           drag_count ? B.hsdyn : (int *)nullptr);
+    template <bool PSG> void area(const void *b, double *pmean, double *bsum, double *pdryini) {
+        hipLaunchKernelGGL((k_area<T, PSG>), dim3(PS_BLOCKS, B.nm), dim3(256), 0, s, (T *)B.psg, (const T *)b,
+                           (const double *)B.areaw, B.pspart, B.psdone, B.ng, E.plan.nlon, pmean, bsum, pdryini,
+                           (const T *)B.ak, (const T *)B.bk, B.nl, B.hsdyn, (const T *)B.gsyn,
+                           (const cplx<T> *)B.spec, B.ntr, B.nsyn, B.nfs);
+    }
+    // FP64 area sums: S(psg) -> pmean, S(b) -> bsum; pdryini = S(psg) - S(b) where 0
+    void area_sums(const void *b, double *pmean, double *bsum, bool set_pdry) {
+        area<false>(b, pmean, bsum, set_pdry ? B.pdryini : (double *)nullptr);
         mark("ps_mean");
     }
     // ngf grid fields of gan -> spectral fields of dst; with nfdyn only the

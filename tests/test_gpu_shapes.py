@@ -244,3 +244,39 @@ def test_simple_columns_every_round(grid, nlev, turb, prec):
                 assert far(x, y) < tol, (k, mem, far(x, y))
             else:  # two layers do not condense; without the boundary layer the wind is untouched
                 assert np.abs(x).max() == 0, (k, mem)
+
+
+# columns of a member: fewer than a round of the 128 workgroups, a little over one, over four; one member to seven
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("grid,nlev,nmem", [((36, 18, 11), 5, 7), ((256, 130, 84), 20, 2), ((576, 288, 190), 3, 1),
+                                            ((64, 32, 21), 64, 3)])
+def test_area_sums(grid, nlev, nmem, prec):
+    """Dry mass of each member against the oracle at the bounds of test_gpu_moist (FP64 1e-9, FP32 2e-6), again after
+    the next state, and lean steps (ps, its range and its mean in one launch) equal to full ones bit for bit."""
+    import cases
+    import gfsdc
+    nlon, nlat, T = grid
+    ak, bk = levels.hybrid_levels(nlev)
+    o = O.Model(nlon, nlat, T, nlev, ak, bk, 300.0, physics=1, massfix=1)
+    p = gfsdc.FP64 if prec == "fp64" else gfsdc.FP32
+    a, b = (gfsdc.Context(nlon, nlat, T, p, nlev=nlev, ak=ak, bk=bk, dt=300.0, nmem=nmem, physics=1, massfix=1)
+            for _ in range(2))
+    for turn in range(2):
+        st = [cases.perturbed_state(o.sht.degree, o.sht.order, nlev, seed=3 + m + nmem * turn, amp=0.2)
+              for m in range(nmem)]
+        x = [np.concatenate(v) for v in zip(*st)]
+        for g in (a, b):
+            g.set_state(*x)
+            g.pdryini = np.zeros(nmem)
+        a.advance(3, use_graph=turn == 0)
+        for _ in range(3):
+            b.advance(1, use_graph=turn == 0)
+        sa, sb = a.get_state(), b.get_state()
+        for k in ("vrt", "div", "tv", "lnps"):
+            assert np.isfinite(sa[k]).all() and np.array_equal(sa[k], sb[k]), (turn, k)
+        for m in range(nmem):
+            o.pdryini = 0.0
+            o.set_state(*(v[m] for v in x))
+            o.getdyntend(1)
+            for g in (a, b):
+                assert abs(g.pdryini[m] - o.pdryini) < (1e-9 if prec == "fp64" else 2e-6) * o.pdryini, (turn, m)
