@@ -4140,7 +4140,7 @@ template <typename T> int Engine<T>::set_topo(const void *topo, int dtype, int l
         sd[mem] = SynthDesc{SK_UHAT, -1, mem, 0.0, g, 0, 0};
         sd[nm + mem] = SynthDesc{SK_VHAT, -1, mem, 0.0, g, 0, 0};
     }
-    if ((rc = upload_descs(sd, {}, std::vector<unsigned char>(2 * nm, 1)))) return rc;
+    if ((rc = upload_descs(sd, std::vector<unsigned char>(2 * nm, 1)))) return rc;
     GFSDC_CHECK(hipMemcpyAsync(B->topo, in, sizeof(cplx<T>) * nlm * nm, hipMemcpyDeviceToDevice, stream));
     launch_synth_gather(plan, (const cplx<T> *)B->topo, nlm, 1, d_sdesc, 2 * nm, W.sx, W.ldc, 1.0, stream);
     launch_leg_synth(plan, W.sx, W.ldc, W.fs, W.ldc, 4 * nm, stream);

@@ -30,22 +30,28 @@ template <typename T> struct Engine {
     // staging for caller buffers
     void *stage[4] = {nullptr, nullptr, nullptr, nullptr};
     size_t stage_sz[4] = {0, 0, 0, 0};
+    // small host fields of the transforms: HOST_SMALL bytes for each of two inputs and two
+    // outputs, in host memory that the kernels read and write themselves
+    char *pinned = nullptr;
     SynthDesc *d_sdesc = nullptr;
-    AnalDesc *d_adesc = nullptr;
     unsigned char *d_rflag = nullptr;
     int desc_cap = 0;
     std::vector<SynthDesc> h_sdesc;
-    std::vector<AnalDesc> h_adesc;
     std::vector<unsigned char> h_rflag;
     DycoreBuffers *dyn = nullptr;
 
     int init(const gfsdc_cfg &c);
     void destroy();
     int ensure_stage(int i, size_t bytes);
-    int upload_descs(const std::vector<SynthDesc> &sd, const std::vector<AnalDesc> &ad,
-                     const std::vector<unsigned char> &rf);
+    int upload_descs(const std::vector<SynthDesc> &sd, const std::vector<unsigned char> &rf);
     // caller buffer (n real values of dtype at loc) -> device T buffer
     int input(const void *p, size_t n, int dtype, int loc, int slot, const T **out);
+    // the transforms' inputs and outputs: as input() and output(), or through pinned where a
+    // field is small and in host memory. A transform with such a buffer ends with finish()
+    int field_in(const void *p, size_t n, int dtype, int loc, int i, const T **out);
+    T *field_out(void *p, size_t n, int dtype, int loc, int i, bool grid);
+    int finish(T *const *d, void *const *p, int np, size_t n, int dtype, int loc);
+    T *host_small(const void *p, size_t n, int dtype, int loc, int i);
     // device T buffer -> caller buffer
     int output(const T *d, void *p, size_t n, int dtype, int loc, int slot);
 

@@ -98,8 +98,8 @@ template <typename T> void Engine<T>::destroy() {
     plan_destroy(plan);
     for (int i = 0; i < 4; i++)
         if (stage[i]) (void)hipFree(stage[i]);
+    if (pinned) (void)hipHostFree(pinned);
     if (d_sdesc) (void)hipFree(d_sdesc);
-    if (d_adesc) (void)hipFree(d_adesc);
     if (d_rflag) (void)hipFree(d_rflag);
     if (stream) (void)hipStreamDestroy(stream);
     stream = nullptr;
@@ -117,26 +117,19 @@ template <typename T> int Engine<T>::ensure_stage(int i, size_t bytes) {
 }
 
 template <typename T>
-int Engine<T>::upload_descs(const std::vector<SynthDesc> &sd, const std::vector<AnalDesc> &ad,
-                            const std::vector<unsigned char> &rf) {
-    int need = (int)std::max(sd.size(), std::max(ad.size(), rf.size()));
+int Engine<T>::upload_descs(const std::vector<SynthDesc> &sd, const std::vector<unsigned char> &rf) {
+    const int need = (int)std::max(sd.size(), rf.size());
     if (need > desc_cap) {
         if (d_sdesc) GFSDC_CHECK(hipFree(d_sdesc));
-        if (d_adesc) GFSDC_CHECK(hipFree(d_adesc));
         if (d_rflag) GFSDC_CHECK(hipFree(d_rflag));
         GFSDC_CHECK(hipMalloc((void **)&d_sdesc, sizeof(SynthDesc) * need));
-        GFSDC_CHECK(hipMalloc((void **)&d_adesc, sizeof(AnalDesc) * need));
         GFSDC_CHECK(hipMalloc((void **)&d_rflag, need));
         desc_cap = need;
     }
     h_sdesc = sd;
-    h_adesc = ad;
     h_rflag = rf;
     if (!sd.empty())
         GFSDC_CHECK(hipMemcpyAsync(d_sdesc, h_sdesc.data(), sizeof(SynthDesc) * sd.size(), hipMemcpyHostToDevice,
-                                   stream));
-    if (!ad.empty())
-        GFSDC_CHECK(hipMemcpyAsync(d_adesc, h_adesc.data(), sizeof(AnalDesc) * ad.size(), hipMemcpyHostToDevice,
                                    stream));
     if (!rf.empty())
         GFSDC_CHECK(hipMemcpyAsync(d_rflag, h_rflag.data(), rf.size(), hipMemcpyHostToDevice, stream));
@@ -212,12 +205,65 @@ template <typename T> int Engine<T>::output(const T *d, void *p, size_t n, int d
     return 0;
 }
 
-// A caller's device buffer of the context's element type that the last kernel
-// of a transform can write itself, else null (it writes the workspace, and
-// output() converts or copies). Grids take 16-byte stores.
-template <typename T> static T *direct(void *p, int dtype, int loc, bool grid) {
-    if (!p || !is_direct<T>(dtype, loc)) return nullptr;
-    return grid && ((uintptr_t)p & 15) ? nullptr : (T *)p;
+// Host fields up to this size (in the context's element type) are copied by the host
+// into pinned memory that the first kernel reads and the last one writes over the bus,
+// instead of by two queued copies of a pageable buffer, each longer than such a kernel.
+// T42 FP64, synthesis and analysis: one field (64 KB) 42 and 40 -> 29 and 27 us, six
+// fields 56 and 48 -> 45 and 40 us. Past a megabyte (100 us) the 10 us no longer count,
+// and a context would hold more than 4 MB of such memory.
+constexpr size_t HOST_SMALL = 1 << 20;
+
+// pinned buffer i (0, 1: inputs, 2, 3: outputs) for n values of a caller's field, or null:
+// the field is not in host memory, of another type or larger, or there is no memory for it
+template <typename T> T *Engine<T>::host_small(const void *p, size_t n, int dtype, int loc, int i) {
+    if (!p || loc != GFSDC_HOST || dtype != (sizeof(T) == 8 ? GFSDC_DT_F64 : GFSDC_DT_F32) || n * sizeof(T) > HOST_SMALL)
+        return nullptr;
+    if (!pinned && hipHostMalloc((void **)&pinned, 4 * HOST_SMALL, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+        (void)hipGetLastError();
+        pinned = nullptr;
+        return nullptr;
+    }
+    return (T *)(pinned + i * HOST_SMALL);
+}
+
+// The last transform that read or wrote pinned memory has ended (finish), so the host
+// may write it.
+template <typename T>
+int Engine<T>::field_in(const void *p, size_t n, int dtype, int loc, int i, const T **out) {
+    T *h = host_small(p, n, dtype, loc, i);
+    if (!h) return input(p, n, dtype, loc, 2 * i, out);
+    std::memcpy(h, p, n * sizeof(T));
+    *out = h;
+    return 0;
+}
+
+// Where the last kernel of a transform writes a caller's field itself: a device buffer of
+// the context's element type, or pinned memory for a small host field; else null (it
+// writes the workspace, and output() converts or copies). Grids take 16-byte stores.
+template <typename T> T *Engine<T>::field_out(void *p, size_t n, int dtype, int loc, int i, bool grid) {
+    if (!p) return nullptr;
+    if (is_direct<T>(dtype, loc)) return grid && ((uintptr_t)p & 15) ? nullptr : (T *)p;
+    return host_small(p, n, dtype, loc, 2 + i);
+}
+
+// The end of a transform whose np fields went to d: to the caller's buffers p where they
+// are not there yet.
+template <typename T>
+int Engine<T>::finish(T *const *d, void *const *p, int np, size_t n, int dtype, int loc) {
+    GFSDC_CHECK(hipGetLastError());
+    bool waited = false;
+    for (int i = 0; i < np; i++) {
+        if ((void *)d[i] == p[i]) continue;
+        if (pinned && (char *)d[i] == pinned + (2 + i) * HOST_SMALL) {
+            if (!waited) GFSDC_CHECK(hipStreamSynchronize(stream));
+            waited = true;
+            std::memcpy(p[i], d[i], n * sizeof(T));
+            continue;
+        }
+        const int rc = output(d[i], p[i], n, dtype, loc, 1);
+        if (rc) return rc;
+    }
+    return 0;
 }
 
 template <typename T> int Engine<T>::spectogrd(const void *spec, void *grid, int nf, int dtype, int loc) {
@@ -225,13 +271,14 @@ template <typename T> int Engine<T>::spectogrd(const void *spec, void *grid, int
     int rc = work_alloc(work, plan, nf);
     if (rc) return rc;
     const T *in;
-    if ((rc = input(spec, (size_t)nf * plan.nlm * 2, dtype, loc, 0, &in))) return rc;
-    T *out = direct<T>(grid, dtype, loc, true);
+    const size_t n = (size_t)nf * plan.nlat * plan.nlon;
+    if ((rc = field_in(spec, (size_t)nf * plan.nlm * 2, dtype, loc, 0, &in))) return rc;
+    T *out = field_out(grid, n, dtype, loc, 0, true);
+    if (!out) out = work.grid;
     launch_gather_ref(plan, (const cplx<T> *)in, nf, work.sx, work.ldc, stream);
     launch_leg_synth(plan, work.sx, work.ldc, work.fs, work.ldc, 2 * nf, stream);
-    launch_fft_synth(plan, work.fs, work.ldc, out ? out : work.grid, (long)plan.nlat * plan.nlon, nf, nullptr, stream);
-    GFSDC_CHECK(hipGetLastError());
-    return out ? 0 : output(work.grid, grid, (size_t)nf * plan.nlat * plan.nlon, dtype, loc, 1);
+    launch_fft_synth(plan, work.fs, work.ldc, out, (long)plan.nlat * plan.nlon, nf, nullptr, stream);
+    return finish(&out, &grid, 1, n, dtype, loc);
 }
 
 // spectogrd on device buffers of the context's element type with every
@@ -272,15 +319,14 @@ template <typename T> int Engine<T>::grdtospec(const void *grid, void *spec, int
     int rc = work_alloc(work, plan, nf);
     if (rc) return rc;
     const T *in;
-    size_t ng = (size_t)plan.nlat * plan.nlon;
-    if ((rc = input(grid, (size_t)nf * ng, dtype, loc, 0, &in))) return rc;
+    const size_t ng = (size_t)plan.nlat * plan.nlon, n = (size_t)nf * plan.nlm * 2;
+    if ((rc = field_in(grid, (size_t)nf * ng, dtype, loc, 0, &in))) return rc;
     launch_fft_anal(plan, in, (long)ng, nf, nullptr, work.fa, work.ldc, stream);
     launch_leg_anal(plan, work.fa, work.ldc, work.sx, work.ldc, 2 * nf, stream);
-    T *dir = direct<T>(spec, dtype, loc, false);
-    T *out = dir ? dir : work.grid;  // reuse as spectral output buffer (nf * nlm complex <= nf * ng)
+    T *out = field_out(spec, n, dtype, loc, 0, false);
+    if (!out) out = work.grid;  // reuse as spectral output buffer (nf * nlm complex <= nf * ng)
     launch_scatter_ref(plan, work.sx, work.ldc, (cplx<T> *)out, nf, stream);
-    GFSDC_CHECK(hipGetLastError());
-    return dir ? 0 : output(out, spec, (size_t)nf * plan.nlm * 2, dtype, loc, 1);
+    return finish(&out, &spec, 1, n, dtype, loc);
 }
 
 // Transform microbenchmark with device-resident buffers: per iteration a
@@ -388,24 +434,21 @@ int Engine<T>::sphtor_to_spat(const void *s, const void *t, void *u, void *v, in
     if (rc) return rc;
     const size_t ns = (size_t)nf * plan.nlm * 2, ng = (size_t)plan.nlat * plan.nlon;
     const T *is = nullptr, *it;
-    if (s && (rc = input(s, ns, dtype, loc, 0, &is))) return rc;
-    if ((rc = input(t, ns, dtype, loc, 2, &it))) return rc;
+    if (s && (rc = field_in(s, ns, dtype, loc, 0, &is))) return rc;
+    if ((rc = field_in(t, ns, dtype, loc, 1, &it))) return rc;
     // the Fourier synthesis writes the caller's two grids, or both into the workspace
-    T *du = direct<T>(u, dtype, loc, true), *dv = direct<T>(v, dtype, loc, true);
-    const bool dir = du && dv;
-    if (!dir) {
-        du = work.grid;
-        dv = work.grid + nf * ng;
+    T *d[2] = {field_out(u, nf * ng, dtype, loc, 0, true), field_out(v, nf * ng, dtype, loc, 1, true)};
+    if (!d[0] || !d[1]) {
+        d[0] = work.grid;
+        d[1] = work.grid + nf * ng;
     }
     launch_gather_ref_vec(plan, (const cplx<T> *)is, (const cplx<T> *)it, nf, work.sx, work.ldc, sscale, sinv, tscale,
                           tinv, stream);
     launch_leg_synth(plan, work.sx, work.ldc, work.fs, work.ldc, 4 * nf, stream);
-    launch_fft_synth(plan, work.fs, work.ldc, du, (long)ng, 2 * nf, nullptr, stream, (const T *)nullptr, nullptr, 0,
-                     nullptr, nullptr, 0.0, FftOpt<T>{dv, nf, 1});
-    GFSDC_CHECK(hipGetLastError());
-    if (dir) return 0;
-    if ((rc = output(du, u, nf * ng, dtype, loc, 1))) return rc;
-    return output(dv, v, nf * ng, dtype, loc, 1);
+    launch_fft_synth(plan, work.fs, work.ldc, d[0], (long)ng, 2 * nf, nullptr, stream, (const T *)nullptr, nullptr, 0,
+                     nullptr, nullptr, 0.0, FftOpt<T>{d[1], nf, 1});
+    void *const p[2] = {u, v};
+    return finish(d, p, 2, nf * ng, dtype, loc);
 }
 
 // (Vt, Vp) -> vorticity / divergence (lap/rsphere S, lap/rsphere T), or SHTns (S, T) when inv = 1.
@@ -417,22 +460,19 @@ int Engine<T>::spat_to_sphtor(const void *u, const void *v, void *s, void *t, in
     if (rc) return rc;
     const size_t ng = (size_t)plan.nlat * plan.nlon, ns = (size_t)nf * plan.nlm * 2;
     const T *iu, *iv;
-    if ((rc = input(u, nf * ng, dtype, loc, 0, &iu))) return rc;
-    if ((rc = input(v, nf * ng, dtype, loc, 2, &iv))) return rc;
+    if ((rc = field_in(u, nf * ng, dtype, loc, 0, &iu))) return rc;
+    if ((rc = field_in(v, nf * ng, dtype, loc, 1, &iv))) return rc;
     launch_fft_anal(plan, iu, (long)ng, 2 * nf, nullptr, work.fa, work.ldc, stream, nullptr,
                     FftOpt<const T>{iv, nf, 1});
     launch_leg_anal(plan, work.fa, work.ldc, work.sx, work.ldc, 4 * nf, stream);
-    T *os = direct<T>(s, dtype, loc, false), *ot = direct<T>(t, dtype, loc, false);
-    const bool dir = os && ot;
-    if (!dir) {
-        os = work.grid;
-        ot = work.grid + ns;
+    T *d[2] = {field_out(s, ns, dtype, loc, 0, false), field_out(t, ns, dtype, loc, 1, false)};
+    if (!d[0] || !d[1]) {
+        d[0] = work.grid;
+        d[1] = work.grid + ns;
     }
-    launch_scatter_ref_vec(plan, work.sx, work.ldc, (cplx<T> *)os, (cplx<T> *)ot, nf, rsphere, inv, stream);
-    GFSDC_CHECK(hipGetLastError());
-    if (dir) return 0;
-    if ((rc = output(os, s, ns, dtype, loc, 1))) return rc;
-    return output(ot, t, ns, dtype, loc, 1);
+    launch_scatter_ref_vec(plan, work.sx, work.ldc, (cplx<T> *)d[0], (cplx<T> *)d[1], nf, rsphere, inv, stream);
+    void *const p[2] = {s, t};
+    return finish(d, p, 2, ns, dtype, loc);
 }
 
 template struct Engine<float>;

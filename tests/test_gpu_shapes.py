@@ -280,3 +280,31 @@ def test_area_sums(grid, nlev, nmem, prec):
             o.getdyntend(1)
             for g in (a, b):
                 assert abs(g.pdryini[m] - o.pdryini) < (1e-9 if prec == "fp64" else 2e-6) * o.pdryini, (turn, m)
+
+
+# fields in host memory below, at and past the megabyte that goes through pinned memory: the grids alone past it, both
+@pytest.mark.parametrize("prec,nf", [("fp64", 1), ("fp64", 64), ("fp64", 65), ("fp64", 270), ("fp32", 128), ("fp32", 129)])
+def test_small_host_fields(prec, nf):
+    """Host calls equal the calls on device buffers bit for bit, two after each other with different fields, and with
+    the other element type they stay within its rounding of them."""
+    import gfsdc
+    nlon, nlat, T = 64, 32, 21
+    g = gfsdc.Context(nlon, nlat, T, gfsdc.FP64 if prec == "fp64" else gfsdc.FP32)
+    dt, ct, rt = (0, np.complex128, np.float64) if prec == "fp64" else (1, np.complex64, np.float32)
+    S, G = ((nf, g.nlm), ct), ((nf, nlat, nlon), rt)
+    rng = np.random.default_rng(nf)
+    x = rng.standard_normal((4, nf, g.nlm)) + 1j * rng.standard_normal((4, nf, g.nlm))
+    x[..., g.order == 0] = x[..., g.order == 0].real
+    y = rng.standard_normal((4, nf, nlat, nlon)).astype(rt)
+    a = x.astype(ct)
+    for i in (0, 1):
+        host = [[g.spectogrd(a[i], dt)], [g.grdtospec(y[i], dt)], g.getuv(a[i], a[i + 2], A, dt),
+                g.getvrtdivspec(y[i], y[i + 2], A, dt)]
+        dev = [device_call(g, "gfsdc_spectogrd", [a[i]], [G], nf), device_call(g, "gfsdc_grdtospec", [y[i]], [S], nf),
+               device_call(g, "gfsdc_getuv", [a[i], a[i + 2]], [G, G], nf, C.c_double(A)),
+               device_call(g, "gfsdc_getvrtdivspec", [y[i], y[i + 2]], [S, S], nf, C.c_double(A))]
+        for p, q in zip(host, dev):
+            for u, v in zip(p, q):
+                assert np.array_equal(u, v), i
+        other = g.spectogrd(a[i].astype(np.complex64 if dt == 0 else np.complex128), 1 - dt)
+        assert np.abs(other - host[0][0]).max() < 2e-6 * np.abs(host[0][0]).max()
