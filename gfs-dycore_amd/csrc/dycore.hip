@@ -2234,40 +2234,65 @@ template <> struct SiMma<double> {
     __device__ static int row(int lane, int r) { return (lane >> 4) + 4 * r; }
 };
 
-// Y[i][col] = sum_k M[i][k] X[k][col], M given transposed (Mt[k * nl + i] = M[i][k]),
-// zero beyond nl levels
-template <typename T>
-__device__ inline void si_gemm(const T *__restrict__ Mt, int nl, const T (*X)[SiCfg<T>::LD], T (*Y)[SiCfg<T>::LD],
-                               int wave, int lane) {
+// Rows that a product reads and writes: 32 of the 64 where the levels fit them
+__device__ __forceinline__ int si_rows(int nl) { return nl <= 32 ? 32 : 64; }
+
+// This lane's values of a level operator M, given transposed (Mt[k * nl + i] = M[i][k]),
+// zero beyond nl levels: all loaded at once, one wait for the (cached) operator
+template <typename T> struct SiOp {
+    T a[16];
+    template <int Q0, int Q1> __device__ __forceinline__ void part(const T *__restrict__ Mt, int nl, int i, int kq) {
+#pragma unroll
+        for (int q = Q0; q < Q1; q++) {
+            const int k = 4 * q + kq;
+            const T x = Mt[min(k, nl - 1) * nl + min(i, nl - 1)];
+            a[q] = i < nl && k < nl ? x : T(0);
+        }
+    }
+    __device__ __forceinline__ void load(const T *__restrict__ Mt, int nl, int wave, int lane) {
+        const int i = wave * 16 + (lane & 15), kq = lane >> 4, nr = si_rows(nl);
+        if (wave * 16 >= nr) return;
+        part<0, 8>(Mt, nl, i, kq);
+        if (nr > 32) part<8, 16>(Mt, nl, i, kq);
+    }
+};
+
+// Y[i][col] = sum_k M[i][k] X[k][col] over the first si_rows(nl) rows, zero in X past nl
+template <typename T, int NQ>
+__device__ __forceinline__ void si_gemm_n(const SiOp<T> &M, const T (*X)[SiCfg<T>::LD], T (*Y)[SiCfg<T>::LD], int wave,
+                                          int lane) {
     constexpr int NB = SiCfg<T>::W / 16;
     typename SiMma<T>::acc acc[NB];
 #pragma unroll
     for (int b = 0; b < NB; b++) acc[b] = typename SiMma<T>::acc{T(0), T(0), T(0), T(0)};
-    const int i = wave * 16 + (lane & 15), kq = lane >> 4;
-    // every operator value of this lane first: one wait for the (cached) operator, not one per k-step
-    T a[16];
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-        const int k = 4 * q + kq;
-        a[q] = (i < nl && k < nl) ? Mt[min(k, nl - 1) * nl + min(i, nl - 1)] : T(0);
-    }
+    for (int q = 0; q < NQ; q++)
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-        const int k = 4 * q + kq;
-#pragma unroll
-        for (int b = 0; b < NB; b++) acc[b] = SiMma<T>::mma(a[q], X[k][b * 16 + (lane & 15)], acc[b]);
-    }
+        for (int b = 0; b < NB; b++)
+            acc[b] = SiMma<T>::mma(M.a[q], X[4 * q + (lane >> 4)][b * 16 + (lane & 15)], acc[b]);
 #pragma unroll
     for (int b = 0; b < NB; b++)
 #pragma unroll
         for (int r = 0; r < 4; r++) Y[wave * 16 + SiMma<T>::row(lane, r)][b * 16 + (lane & 15)] = acc[b][r];
 }
-
 template <typename T>
-__device__ inline void si_colsum(const T *__restrict__ w, int nl, const T (*X)[SiCfg<T>::LD], T *out) {
-    const int col = threadIdx.x;
-    if (col < SiCfg<T>::W) {
+__device__ __forceinline__ void si_gemm(const SiOp<T> &M, int nl, const T (*X)[SiCfg<T>::LD], T (*Y)[SiCfg<T>::LD],
+                                        int wave, int lane) {
+    const int nr = si_rows(nl);
+    if (wave * 16 >= nr) return;
+    if (nr > 32)
+        si_gemm_n<T, 16>(M, X, Y, wave, lane);
+    else
+        si_gemm_n<T, 8>(M, X, Y, wave, lane);
+}
+
+// by the last wavefront, which has no product where the levels fit 32 rows
+template <typename T>
+__device__ inline void si_colsum(const T *w, int nl, const T (*X)[SiCfg<T>::LD], T *out) {
+    const int col = (int)threadIdx.x - 192;
+    if (col >= 0 && col < SiCfg<T>::W) {
         T s = T(0);
+#pragma unroll 8
         for (int l = 0; l < nl; l++) s += w[l] * X[l][col];
         out[col] = s;
     }
@@ -2278,6 +2303,12 @@ __device__ inline void si_colsum(const T *__restrict__ w, int nl, const T (*X)[S
 // stage that first reads it; the last stage keeps nothing. Per coefficient the
 // three stages move 3154 instead of 4121 values a member at 64 levels (dry),
 // the copy of the initial state included: T254L64 FP32 six steps 18.24 -> 17.96 ms.
+// Bound by its chain of waits and barriers at small sizes, by memory (two thirds of
+// the time of a copy of what it moves) at T254: T42 20 levels FP64 14.5 -> 11.0 us a stage
+// with 32-row products where the levels fit, the coefficient's index computed instead
+// of loaded, and the column sums on a wavefront of their own; T254 64 levels FP32 110 ->
+// 105 us, 16 members at T126 393 -> 378 us. The operators and the combination's values
+// loaded ahead of all else cost more in wavefronts (191 and 110 registers: T254 150 us).
 // the tableau's column of a stage: its own coefficients, the next stage's and the one after's
 struct SiNext {
     double a0, aa0, a1, aa1, a2, aa2;
@@ -2288,8 +2319,7 @@ __global__ __launch_bounds__(256) void k_si_mfma(
     const T *__restrict__ ten2, T *__restrict__ e1_, T *__restrict__ e2_,
     const T *__restrict__ At, const T *__restrict__ Bt, const T *__restrict__ Dt,
     const T *__restrict__ sv, const T *__restrict__ tor, const T *__restrict__ disspec,
-    const T *__restrict__ diffp, const T *__restrict__ dmpp, const int *__restrict__ kbydeg,
-    const int2 *__restrict__ tiles, int stage, Coeffs3 cf, SiNext cn, T cimp, int do_implicit, int damp, int nl, int ntr,
+    const T *__restrict__ diffp, const T *__restrict__ dmpp, const int2 *__restrict__ tiles, int stage, Coeffs3 cf, SiNext cn, T cimp, int do_implicit, int damp, int nl, int ntr,
     int nfs, int nm, int ntrunc, T dt, double *__restrict__ clock, double dtd) {
     constexpr int C = SiCfg<T>::C, W = SiCfg<T>::W, LD = SiCfg<T>::LD;
     typedef cplx<T> V2;
@@ -2297,7 +2327,12 @@ __global__ __launch_bounds__(256) void k_si_mfma(
     __shared__ T lpin[W], lpc[W], csum[W];
     __shared__ long sbase[C], slbase[C];
     __shared__ int sk[C];
+    __shared__ T svs[64], tors[64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid < nl) {
+        svs[tid] = sv[tid];
+        tors[tid] = tor[tid];
+    }
     // tiles run in degree order, each XCD a contiguous range of them, so that
     // the tiles of one degree share its operators in one L2
     const int2 tl = tiles[xcd_tile(blockIdx.x, gridDim.x)];
@@ -2309,7 +2344,7 @@ __global__ __launch_bounds__(256) void k_si_mfma(
         int k = 0;
         if (tid < cnt) {
             const int item = i0 + tid, mem = item / (n + 1), m = item - mem * (n + 1);
-            k = kbydeg[n * (n + 1) / 2 + m];
+            k = m * (2 * ntrunc + 3 - m) / 2 + n - m;
             b = (long)k * NFS + (long)mem * nfs;
             lb = (long)k * nlin * nm + (long)mem * nlin;
         }
@@ -2328,6 +2363,19 @@ __global__ __launch_bounds__(256) void k_si_mfma(
     V2 *E1 = (V2 *)e1_, *E2 = (V2 *)e2_;
     // element e = c * nl + lev: one complex value (re, im) per element
     const int nel = cnt * nl;
+    // the loads of the stage input (tv, div, ln ps) go out before those of the fields below
+    constexpr int NI = 64 * C / 256;
+    V2 tvi[NI], dvi[NI], lp0 = V2{T(0), T(0)};
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int c = min((tid >> 6) + 4 * i, cnt - 1);
+        const long b = sbase[c] + min(lane, nl - 1);
+        tvi[i] = sp[b + 2L * nl];
+        dvi[i] = sp[b + nl];
+    }
+    if (tid < cnt) lp0 = sp[sbase[tid] + 3L * nl + (long)ntr * nl];
+    const V2 *Tn = tn[stage];
+    const V2 *Ep = stage == 2 ? E2 : E1;
     // vorticity and tracers: always explicit (plus damping after the last stage)
     for (int e = tid; e < nel * (1 + ntr); e += 256) {
         const int fld = e / nel, r0 = e - fld * nel, c = r0 / nl, lev = r0 - c * nl;
@@ -2350,42 +2398,40 @@ __global__ __launch_bounds__(256) void k_si_mfma(
         sp[off] = v;
     }
     // stage input: tv -> S0, div -> S1 (zero padded), ln ps -> lpin
-    for (int e = tid; e < 64 * C; e += 256) {
-        const int c = e >> 6, lev = e & 63;
-        V2 tv = V2{T(0), T(0)}, dv = tv;
-        if (c < cnt && lev < nl) {
-            const long b = sbase[c] + lev;
-            tv = sp[b + 2L * nl];
-            dv = sp[b + nl];
-            if (stage == 0) {
-                ((V2 *)spec0)[b + 2L * nl] = tv;
-                ((V2 *)spec0)[b + nl] = dv;
-            }
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int c = (tid >> 6) + 4 * i;
+        const bool in = c < cnt && lane < nl;
+        const V2 tv = in ? tvi[i] : V2{T(0), T(0)}, dv = in ? dvi[i] : V2{T(0), T(0)};
+        if (stage == 0 && in) {
+            ((V2 *)spec0)[sbase[c] + lane + 2L * nl] = tv;
+            ((V2 *)spec0)[sbase[c] + lane + nl] = dv;
         }
-        S0[lev][2 * c] = tv.x;
-        S0[lev][2 * c + 1] = tv.y;
-        S1[lev][2 * c] = dv.x;
-        S1[lev][2 * c + 1] = dv.y;
+        S0[lane][2 * c] = tv.x;
+        S0[lane][2 * c + 1] = tv.y;
+        S1[lane][2 * c] = dv.x;
+        S1[lane][2 * c + 1] = dv.y;
     }
     if (tid < C) {
-        const long b = sbase[tid] + 3L * nl + (long)ntr * nl;
-        const V2 v = (tid < cnt) ? sp[b] : V2{T(0), T(0)};
-        if (stage == 0 && tid < cnt) ((V2 *)spec0)[b] = v;
-        lpin[2 * tid] = v.x;
-        lpin[2 * tid + 1] = v.y;
+        if (stage == 0 && tid < cnt) ((V2 *)spec0)[sbase[tid] + 3L * nl + (long)ntr * nl] = lp0;
+        lpin[2 * tid] = lp0.x;
+        lpin[2 * tid + 1] = lp0.y;
     }
     __syncthreads();
     // linear terms of the stage input (run.f90:329-335)
-    si_gemm<T>(At, nl, S0, S2, wave, lane);
-    si_gemm<T>(Bt, nl, S1, S3, wave, lane);
-    si_colsum<T>(sv, nl, S1, csum);
+    SiOp<T> op;
+    op.load(At, nl, wave, lane);
+    si_gemm<T>(op, nl, S0, S2, wave, lane);
+    op.load(Bt, nl, wave, lane);
+    si_gemm<T>(op, nl, S1, S3, wave, lane);
+    si_colsum<T>(svs, nl, S1, csum);
     __syncthreads();
     // take them from this stage's tendency; explicit combination. A later stage
     // needs this one's tendency d and linear term l only as a d + aa l, so that is
     // what is kept: E1 for stage 1, E2 for stage 2
-    const V2 *Tn = tn[stage];
-    // own contribution of (d, l), with the earlier stages' from E; updates E for the later ones
-    auto combine = [&](long lb, V2 d, V2 l) {
+    // own contribution of (d, l), with the earlier stages' (e) from E; updates E for the
+    // later ones (f: what E2 holds in stage 1)
+    auto combine = [&](long lb, V2 d, V2 l, V2 e, V2 f) {
         auto mix = [&](double ca, double cl) { return V2{(T)(ca * d.x + cl * l.x), (T)(ca * d.y + cl * l.y)}; };
         const V2 a = mix(cn.a0, cn.aa0);
         if (stage == 0) {
@@ -2393,9 +2439,8 @@ __global__ __launch_bounds__(256) void k_si_mfma(
             E2[lb] = mix(cn.a2, cn.aa2);
             return a;
         }
-        const V2 e = stage == 1 ? E1[lb] : E2[lb];
         if (stage == 1) {
-            const V2 f = E2[lb], m = mix(cn.a1, cn.aa1);
+            const V2 m = mix(cn.a1, cn.aa1);
             E2[lb] = V2{f.x + m.x, f.y + m.y};
         }
         return V2{a.x + e.x, a.y + e.y};
@@ -2403,15 +2448,23 @@ __global__ __launch_bounds__(256) void k_si_mfma(
     for (int e = tid; e < nel; e += 256) {
         const int c = e / nl, lev = e - c * nl;
         const long lb = slbase[c] + lev, b = sbase[c] + lev;
+        const V2 dd = Tn[b + nl], dT = Tn[b + 2L * nl], d0 = sp0[b + nl], t0 = sp0[b + 2L * nl];
+        V2 e1{T(0), T(0)}, e2 = e1, f1 = e1, f2 = e1;
+        if (stage > 0) {
+            e1 = Ep[lb];
+            e2 = Ep[lb + nl];
+        }
+        if (stage == 1) {
+            f1 = E2[lb];
+            f2 = E2[lb + nl];
+        }
         V2 ddl, dtl;
-        ddl.x = -lap * (S2[lev][2 * c] + tor[lev] * lpin[2 * c]);
-        ddl.y = -lap * (S2[lev][2 * c + 1] + tor[lev] * lpin[2 * c + 1]);
+        ddl.x = -lap * (S2[lev][2 * c] + tors[lev] * lpin[2 * c]);
+        ddl.y = -lap * (S2[lev][2 * c + 1] + tors[lev] * lpin[2 * c + 1]);
         dtl.x = -S3[lev][2 * c];
         dtl.y = -S3[lev][2 * c + 1];
-        const V2 dd = Tn[b + nl], dT = Tn[b + 2L * nl];
-        const V2 d0 = sp0[b + nl], t0 = sp0[b + 2L * nl];
-        const V2 a1 = combine(lb, V2{dd.x - ddl.x, dd.y - ddl.y}, ddl);
-        const V2 a2 = combine(lb + nl, V2{dT.x - dtl.x, dT.y - dtl.y}, dtl);
+        const V2 a1 = combine(lb, V2{dd.x - ddl.x, dd.y - ddl.y}, ddl, e1, f1);
+        const V2 a2 = combine(lb + nl, V2{dT.x - dtl.x, dT.y - dtl.y}, dtl, e2, f2);
         S1[lev][2 * c] = d0.x + dt * a1.x;  // dvc
         S1[lev][2 * c + 1] = d0.y + dt * a1.y;
         S0[lev][2 * c] = t0.x + dt * a2.x;  // tvc
@@ -2419,27 +2472,33 @@ __global__ __launch_bounds__(256) void k_si_mfma(
     }
     if (tid < cnt) {
         const long b = sbase[tid] + 3L * nl + (long)ntr * nl;
+        const long lb = slbase[tid] + 2L * nl;
         const V2 l{-csum[2 * tid], -csum[2 * tid + 1]}, d = Tn[b], p0 = sp0[b];
-        const V2 a3 = combine(slbase[tid] + 2L * nl, V2{d.x - l.x, d.y - l.y}, l);
+        const V2 zero{T(0), T(0)}, pe = stage > 0 ? Ep[lb] : zero, pf = stage == 1 ? E2[lb] : zero;
+        const V2 a3 = combine(lb, V2{d.x - l.x, d.y - l.y}, l, pe, pf);
         lpc[2 * tid] = p0.x + dt * a3.x;
         lpc[2 * tid + 1] = p0.y + dt * a3.y;
     }
     __syncthreads();
     if (do_implicit) {
         // rhs, solve with d_hyb_m(:,:,n+1,stage) and back-substitution (run.f90:344-349)
-        si_gemm<T>(At, nl, S0, S2, wave, lane);
+        op.load(At, nl, wave, lane);
+        si_gemm<T>(op, nl, S0, S2, wave, lane);
         __syncthreads();
-        for (int e = tid; e < 64 * W; e += 256) {
+        const int nrow = si_rows(nl);
+        for (int e = tid; e < nrow * W; e += 256) {
             const int lev = e / W, col = e - lev * W;
-            S3[lev][col] = (lev < nl) ? S1[lev][col] - cimp * lap * dt * (S2[lev][col] + tor[lev] * lpc[col]) : T(0);
+            S3[lev][col] = (lev < nl) ? S1[lev][col] - cimp * lap * dt * (S2[lev][col] + tors[lev] * lpc[col]) : T(0);
         }
         __syncthreads();
-        si_gemm<T>(Dt + ((long)stage * (ntrunc + 1) + n) * nl * nl, nl, S3, S2, wave, lane);
+        op.load(Dt + ((long)stage * (ntrunc + 1) + n) * nl * nl, nl, wave, lane);
+        si_gemm<T>(op, nl, S3, S2, wave, lane);
         __syncthreads();
-        si_gemm<T>(Bt, nl, S2, S3, wave, lane);
-        si_colsum<T>(sv, nl, S2, csum);
+        op.load(Bt, nl, wave, lane);
+        si_gemm<T>(op, nl, S2, S3, wave, lane);
+        si_colsum<T>(svs, nl, S2, csum);
         __syncthreads();
-        for (int e = tid; e < 64 * W; e += 256) {
+        for (int e = tid; e < nl * W; e += 256) {
             const int lev = e / W, col = e - lev * W;
             S0[lev][col] -= cimp * dt * S3[lev][col];
             S1[lev][col] = S2[lev][col];
@@ -3404,7 +3463,7 @@ template <typename T> struct Step {
                                (T *)B.spec0, (const T *)B.ten[0], (const T *)B.ten[1], (const T *)B.ten[2], (T *)B.lin[0],
                                (T *)B.lin[1], (const T *)B.at, (const T *)B.bt, (const T *)B.dt3,
                                (const T *)B.sv, (const T *)B.tor, (const T *)B.disspec, (const T *)B.diffp,
-                               (const T *)B.dmpp, B.kbydeg, (const int2 *)B.si_tiles, stage, cf, cn,
+                               (const T *)B.dmpp, (const int2 *)B.si_tiles, stage, cf, cn,
                                (T)TAB_IMP[stage], do_imp, damp ? 1 : 0, B.nl, B.ntr, B.nfs, B.nm, E.plan.ntrunc,
                                (T)c.dt, B.clock, c.dt);
             mark("si_stage");

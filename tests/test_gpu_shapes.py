@@ -308,3 +308,34 @@ def test_small_host_fields(prec, nf):
                 assert np.array_equal(u, v), i
         other = g.spectogrd(a[i].astype(np.complex64 if dt == 0 else np.complex128), 1 - dt)
         assert np.abs(other - host[0][0]).max() < 2e-6 * np.abs(host[0][0]).max()
+
+
+# levels on both sides of the solve's 32 and 64 rows and of its blocks of 16; coefficients of a degree off the 8 of a tile
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("nlev,ntrac,nmem", [(2, 0, 3), (16, 1, 1), (31, 0, 2), (32, 2, 1), (33, 0, 2), (47, 0, 1), (64, 1, 2)])
+def test_solve_every_size(nlev, ntrac, nmem, prec):
+    """One semi-implicit step of each member against the oracle at the bounds of test_gpu_moist (2-norm, FP64 1e-9,
+    FP32 1e-4)."""
+    import cases
+    import gfsdc
+    ak, bk = levels.hybrid_levels(nlev)
+    o = O.Model(64, 32, 21, nlev, ak, bk, 600.0, ntrac=ntrac)
+    p, tol = (gfsdc.FP64, 1e-9) if prec == "fp64" else (gfsdc.FP32, 1e-4)
+    g = gfsdc.Context(64, 32, 21, p, nlev=nlev, ak=ak, bk=bk, dt=600.0, ntrac=ntrac, nmem=nmem)
+    x = [np.concatenate(v) for v in zip(*(cases.perturbed_state(o.sht.degree, o.sht.order, nlev, seed=3 + m, amp=0.2)
+                                          for m in range(nmem)))]
+    q = np.zeros((nmem, ntrac, nlev, o.sht.nlm), complex)
+    for t in range(ntrac):
+        q[:, t] = 1e-4 * x[2]
+        q[:, t, :, 0] = 0.01 * np.linspace(1.0, 0.2, nlev) * np.sqrt(4 * np.pi)
+    g.set_state(*x, trac=q if ntrac else None)
+    g.advance(1)
+    sg = g.get_state()
+    for m in range(nmem):
+        o.pdryini = 0.0  # each member keeps its own dry mass
+        o.set_state(*(v[m] for v in x), *([q[m]] if ntrac else []))
+        o.advance(1)
+        so = o.get_state()
+        for k in ("vrt", "div", "tv", "lnps") + (("trac",) if ntrac else ()):
+            e = np.linalg.norm(sg[k][m] - so[k]) / np.linalg.norm(so[k])
+            assert e < tol, (k, m, e)
