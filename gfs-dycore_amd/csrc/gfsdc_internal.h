@@ -75,9 +75,7 @@ template <typename T> struct Plan {
     long *tpoff = nullptr;   // device, offset of order m in plmt
     long *poff = nullptr;    // device, per m (ntrunc+2 entries)
     int *keoff = nullptr;    // device, extended spectral offset of order m
-    int *koff = nullptr;     // device, spectral offset of order m
     T *eps = nullptr;        // device, eps_n^m at extended index (n = m..T+1) plus n=T+2 row
-    int *eoff = nullptr;     // device, offset of order m in eps (T+3-m entries)
     T *rcos = nullptr;       // device, 1/cos(lat), nlat
     T *wfac = nullptr;       // device, 2 pi w_j / nlon, nlat
     T *tw = nullptr;         // device, complex FFT twiddles in stage order (see plan_create), 2*nlon

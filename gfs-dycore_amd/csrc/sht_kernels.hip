@@ -1377,7 +1377,7 @@ template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void k_gather_ref(const cplx<T> *__restrict__ qa, const cplx<T> *__restrict__ qb,
                                                     int np, T *__restrict__ sx, int ldx,
                                                     const int2 *__restrict__ kemn, const T *__restrict__ eps,
-                                                    const int *__restrict__ eoff, int ntrunc, int nlm, int nke, T sa,
+                                                    int ntrunc, int nlm, int nke, T sa,
                                                     T sb, int inva, int invb) {
     constexpr int F = REF_F<T>, P = REF_P<T>, NA = VEC ? 2 : 1, R = REF_K + 2;
     __shared__ cplx<T> buf[NA][F][P];  // row r: ke0 - 1 + r, the first and the last for the recurrences only
@@ -1428,7 +1428,7 @@ __global__ __launch_bounds__(256) void k_gather_ref(const cplx<T> *__restrict__ 
         if (tid < 2 * nf) load(tid < nf ? 0 : R - 1, tid < nf ? tid : tid - nf, 1, std::integral_constant<int, 1>());
         if (tid < REF_K && ke0 + tid < nke) {
             const int2 mn = kemn[ke0 + tid];
-            const T *ep = eps + eoff[mn.x] + mn.y - mn.x;
+            const T *ep = eps + ke0 + tid + mn.x;
             nm[tid] = mn;
             cm[tid] = T(mn.y - 1) * ep[0];
             cp[tid] = T(mn.y + 2) * ep[1];
@@ -1464,7 +1464,7 @@ __global__ __launch_bounds__(256) void k_gather_ref(const cplx<T> *__restrict__ 
 template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void k_scatter_ref(const T *__restrict__ sx, int ldx, cplx<T> *__restrict__ qa,
                                                      cplx<T> *__restrict__ qb, int np, const int2 *__restrict__ kemn,
-                                                     const T *__restrict__ eps, const int *__restrict__ eoff,
+                                                     const T *__restrict__ eps,
                                                      int ntrunc, int nlm, int nke, T rrs, int inv) {
     constexpr int F = REF_F<T>, P = REF_P<T>, NA = VEC ? 2 : 1, R = REF_K + 2;
     __shared__ cplx<T> buf[NA][F][P];
@@ -1490,7 +1490,7 @@ __global__ __launch_bounds__(256) void k_scatter_ref(const T *__restrict__ sx, i
     if (n > ntrunc) return;
     T cp = T(0), cm = T(0), il = T(1);
     if constexpr (VEC) {
-        const T *ep = eps + eoff[m] + n - m;
+        const T *ep = eps + ke + m;
         cm = T(n + 1) * ep[0];
         cp = T(n) * ep[1];
         if (inv) il = (n == 0) ? T(0) : T(-1.0 / ((double)n * (n + 1.0)));
@@ -1515,8 +1515,15 @@ __global__ __launch_bounds__(256) void k_scatter_ref(const T *__restrict__ sx, i
 
 // ---------------------------------------------------------------------------
 // Gather into extended spectral columns and scatter out of them.
-constexpr int GATHER_KE = 8;
+// Rows a workgroup of the gather and of the scatter takes: 8 (one descriptor load for them
+// all), or 4 where that leaves at most 4 workgroups a CU; both are then one batch of loads.
+// Gather and scatter, T42 20 levels FP64: 6.9 and 5.1 us with 8 rows, 5.2 and 4.8 with 4;
+// T62 64 levels FP64 8.6 and 6.0, 7.6 and 5.2; T84 FP32 9.1 and 5.8, 8.2 and 5.4; T84 FP64,
+// at the line: 11.0 and 7.8, 11.3 and 7.6. Every offset follows from the row and its
+// order: loading them first cost T42 another 0.5 to 1 us.
 constexpr int GATHER_QB = 4;  // rows whose loads are issued together
+constexpr long ROW_BATCH_WGS = 1024;
+static int row_batch(long rows, int nblk) { return (rows + 7) / 8 * nblk <= ROW_BATCH_WGS ? 4 : 8; }
 
 // Each output element is a combination of at most three source coefficients
 // ("taps") of the row's order m: U-hat takes S at n - 1 and n + 1 and T at n,
@@ -1527,8 +1534,8 @@ constexpr int GATHER_QB = 4;  // rows whose loads are issued together
 template <typename T>
 __global__ void k_synth_gather(const cplx<T> *__restrict__ src, long sf, long sk, const SynthDesc *__restrict__ desc,
                                int nfo, T *__restrict__ sx, int ldx, const int2 *__restrict__ kemn,
-                               const int *__restrict__ koff, const T *__restrict__ eps, const int *__restrict__ eoff,
-                               int ntrunc, int nke, T *__restrict__ mean, const int *__restrict__ nfdyn) {
+                               const T *__restrict__ eps, int ntrunc, int nke, int rows, T *__restrict__ mean,
+                               const int *__restrict__ nfdyn) {
     const int fo = blockIdx.x * blockDim.x + threadIdx.x;
     if (nfdyn) nfo = min(nfo, *nfdyn);
     if (fo >= nfo) return;
@@ -1552,27 +1559,30 @@ __global__ void k_synth_gather(const cplx<T> *__restrict__ src, long sf, long sk
     const T sa = T(d.sa), sb = T(d.sb);
     const T s0 = sa, s1 = uh ? sa : sb, s2 = sb;
     const int i0 = d.inv_a, i1 = uh ? d.inv_a : d.inv_b, i2 = d.inv_b;
-    auto tap = [&](int f, int m, int n) {
-        const int nc = min(max(n, m), ntrunc);
-        return src[f * sf + (long)(koff[m] + nc - m) * sk];
+    // row ke = (m, n) of the extended columns (orders of T + 2 - m rows) is coefficient
+    // ke - m of the source (T + 1 - m) and entry ke + m of eps (T + 3 - m)
+    auto tap = [&](int f, int ke, int m, int n, int td) {
+        const int nc = min(max(n + td, m), ntrunc);
+        return src[f * sf + (long)(ke - m + nc - n) * sk];
     };
     auto fac = [&](bool ok, int m, int n, T sc, int inv) {
         if (!ok || n < m || n > ntrunc) return T(0);
         if (inv) sc *= (n == 0) ? T(0) : T(-1.0 / ((double)n * (n + 1.0)));
         return sc;
     };
-    const int kb0 = blockIdx.y * GATHER_KE, kb1 = min(nke, kb0 + GATHER_KE);
+    const int kb0 = blockIdx.y * rows, kb1 = min(nke, kb0 + rows);
     for (int kb = kb0; kb < kb1; kb += GATHER_QB) {
         int2 mn[GATHER_QB];
         cplx<T> v0[GATHER_QB], v1[GATHER_QB], v2[GATHER_QB];
 #pragma unroll
         for (int q = 0; q < GATHER_QB; q++) {
-            mn[q] = kemn[min(kb + q, kb1 - 1)];  // clamped: rows past kb1 are not stored
+            const int ke = min(kb + q, kb1 - 1);  // clamped: rows past kb1 are not stored
+            mn[q] = kemn[ke];
             const int m = mn[q].x, n = mn[q].y;
-            v0[q] = tap(tf0, m, n + td0);
+            v0[q] = tap(tf0, ke, m, n, td0);
             if (vec) {
-                v1[q] = tap(tf1, m, n + td1);
-                v2[q] = tap(tf2, m, n + td2);
+                v1[q] = tap(tf1, ke, m, n, td1);
+                v2[q] = tap(tf2, ke, m, n, td2);
             }
         }
 #pragma unroll
@@ -1582,8 +1592,7 @@ __global__ void k_synth_gather(const cplx<T> *__restrict__ src, long sf, long sk
             const int m = mn[q].x, n = mn[q].y;
             cplx<T> r{T(0), T(0)};
             if (vec) {
-                const T *ep = eps + eoff[m];
-                const T en = ep[n - m], en1 = ep[n + 1 - m];
+                const T en = eps[ke + m], en1 = eps[ke + m + 1];
                 const T cm1 = T(n - 1) * en, cp1 = T(n + 2) * en1, fm = T(m);
                 const T c0 = fac(ok0, m, n + td0, s0, i0), c1 = fac(ok1, m, n + td1, s1, i1);
                 const T c2 = fac(ok2, m, n + td2, s2, i2);
@@ -1607,21 +1616,19 @@ __global__ void k_synth_gather(const cplx<T> *__restrict__ src, long sf, long sk
     }
 }
 
-// SCATTER_KE coefficients per workgroup (one descriptor load, SCATTER_KE rows),
-// threads over the output fields.
-constexpr int SCATTER_KE = 8;
+// KE coefficients per workgroup (one descriptor load, KE rows), threads over the output
+// fields. Coefficient k = (m, n) is row k + m of the extended columns, entry k + 2 m of eps.
 
 // MFX: the descriptors may hold AK_MASSFIX (a separate instantiation keeps its
 // division out of the plain scatter)
-template <typename T, bool MFX>
+template <typename T, bool MFX, int KE>
 __global__ void k_anal_scatter(const T *__restrict__ sx, int ldx, const AnalDesc *__restrict__ desc, int nfo,
                                cplx<T> *__restrict__ dst, long df, long dk, const int2 *__restrict__ kmn,
-                               const int *__restrict__ keoff, const T *__restrict__ eps,
-                               const int *__restrict__ eoff, T rrs, int nlm, const int *__restrict__ nfdyn) {
+                               const T *__restrict__ eps, T rrs, int nlm, const int *__restrict__ nfdyn) {
     const int fo = blockIdx.x * blockDim.x + threadIdx.x;
     if (fo >= nfo) return;
     const AnalDesc d = desc[fo];
-    const int k0 = blockIdx.y * SCATTER_KE, kend = min(nlm, k0 + SCATTER_KE);
+    const int k0 = blockIdx.y * KE, kend = min(nlm, k0 + KE);
     // a source field past the device field count was not transformed (the
     // caller has established that it is zero on the grid): its output is zero
     const int lim = nfdyn ? *nfdyn : INT_MAX;
@@ -1631,8 +1638,8 @@ __global__ void k_anal_scatter(const T *__restrict__ sx, int ldx, const AnalDesc
         return;
     }
     // the inputs of QB rows first (loads all in flight together), then those rows;
-    // FP64 takes half the rows per batch to stay within the registers
-    constexpr int QB = sizeof(T) == 4 ? SCATTER_KE : SCATTER_KE / 2;
+    // FP64 takes at most four rows per batch to stay within the registers
+    constexpr int QB = sizeof(T) == 4 || KE < 4 ? KE : 4;
     const bool mfx = MFX && d.kind == AK_MASSFIX, copy = d.kind == AK_COPY || mfx, rd = d.accum || mfx;
     const int ca = (d.kind == AK_VRT) ? d.b : d.a;  // i m (V for vrt, U for div; the field for a copy)
     const int cb = (d.kind == AK_VRT) ? d.a : d.b;  // recurrence partner (U for vrt, V for div)
@@ -1645,7 +1652,7 @@ __global__ void k_anal_scatter(const T *__restrict__ sx, int ldx, const AnalDesc
             const int2 mn = kmn[k];
             const int m = mn.x, n = mn.y;
             mnq[q] = mn;
-            const T *X = sx + (long)(keoff[m] + n - m) * ldx;
+            const T *X = sx + (long)(k + m) * ldx;
             const T *C = copy ? X + 2 * d.a : X + 2 * ca;
             z0[q] = cplx<T>{C[0], C[1]};
             zp[q] = zm[q] = zc[q] = za[q] = cplx<T>{T(0), T(0)};
@@ -1663,8 +1670,7 @@ __global__ void k_anal_scatter(const T *__restrict__ sx, int ldx, const AnalDesc
             const int m = mnq[q].x, n = mnq[q].y;
             cplx<T> r = z0[q];
             if (!copy) {
-                const T *ep = eps + eoff[m];
-                T en = ep[n - m], en1 = ep[n + 1 - m];
+                T en = eps[k + 2 * m], en1 = eps[k + 2 * m + 1];
                 T cp = T(n) * en1, cm = T(n + 1) * en, fm = T(m);
                 T sgn = (d.kind == AK_VRT) ? T(-1) : T(1);
                 // vrt = (i m V_n - n eps_{n+1} U_{n+1} + (n+1) eps_n U_{n-1}) / a
@@ -1802,8 +1808,6 @@ template <typename T> int plan_create(Plan<T> &p, int nlon, int nlat, int ntrunc
     int rc;
     if ((rc = upload(&p.poff, p.poff_h.data(), sizeof(long) * (T_ + 2), s))) return rc;
     if ((rc = upload(&p.keoff, p.keoff_h.data(), sizeof(int) * (T_ + 2), s))) return rc;
-    if ((rc = upload(&p.koff, p.koff_h.data(), sizeof(int) * (T_ + 2), s))) return rc;
-    if ((rc = upload(&p.eoff, eoff_h.data(), sizeof(int) * (T_ + 2), s))) return rc;
     if ((rc = upload(&p.eps, epsv.data(), sizeof(T) * eo, s))) return rc;
     if ((rc = upload(&p.mtile_m, mt_m.data(), sizeof(int) * mt_m.size(), s))) return rc;
     if ((rc = upload(&p.mtile_i, mt_i.data(), sizeof(int) * mt_i.size(), s))) return rc;
@@ -1865,7 +1869,7 @@ template <typename T> int plan_create(Plan<T> &p, int nlon, int nlat, int ntrunc
 }
 
 template <typename T> void plan_destroy(Plan<T> &p) {
-    void *ptrs[] = {p.plm, p.poff, p.plmt, p.tpoff, p.keoff, p.koff, p.eps, p.eoff, p.rcos, p.wfac,
+    void *ptrs[] = {p.plm, p.poff, p.plmt, p.tpoff, p.keoff, p.eps, p.rcos, p.wfac,
                     p.tw, p.mtile_m, p.mtile_i, p.mu_d, p.w_d, p.kemn, p.kmn};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
@@ -1904,9 +1908,9 @@ template <typename T>
 void launch_synth_gather(const Plan<T> &p, const cplx<T> *src, long sf, long sk, const SynthDesc *desc, int nfo,
                          T *sx, int ldx, double rsphere, hipStream_t s, T *mean, const int *nfdyn) {
     (void)rsphere;
-    dim3 grid((nfo + 255) / 256, (p.nlme + GATHER_KE - 1) / GATHER_KE);
-    hipLaunchKernelGGL(k_synth_gather<T>, grid, dim3(256), 0, s, src, sf, sk, desc, nfo, sx, ldx, p.kemn, p.koff,
-                       p.eps, p.eoff, p.ntrunc, p.nlme, mean, nfdyn);
+    const int bs = nfo >= 256 ? 256 : 64 * ((nfo + 63) / 64), nb = (nfo + bs - 1) / bs, rows = row_batch(p.nlme, nb);
+    hipLaunchKernelGGL(k_synth_gather<T>, dim3(nb, (p.nlme + rows - 1) / rows), dim3(bs), 0, s, src, sf, sk, desc, nfo,
+                       sx, ldx, p.kemn, p.eps, p.ntrunc, p.nlme, rows, mean, nfdyn);
 }
 
 template <typename T> static dim3 ref_grid(const Plan<T> &p, int nf) {
@@ -1916,27 +1920,27 @@ template <typename T> static dim3 ref_grid(const Plan<T> &p, int nf) {
 template <typename T>
 void launch_gather_ref(const Plan<T> &p, const cplx<T> *q, int nf, T *sx, int ldx, hipStream_t s) {
     hipLaunchKernelGGL((k_gather_ref<T, false>), ref_grid(p, nf), dim3(256), 0, s, q, (const cplx<T> *)nullptr, nf, sx,
-                       ldx, p.kemn, p.eps, p.eoff, p.ntrunc, p.nlm, p.nlme, T(1), T(1), 0, 0);
+                       ldx, p.kemn, p.eps, p.ntrunc, p.nlm, p.nlme, T(1), T(1), 0, 0);
 }
 
 template <typename T>
 void launch_gather_ref_vec(const Plan<T> &p, const cplx<T> *qs, const cplx<T> *qt, int np, T *sx, int ldx, double sa,
                            int inva, double sb, int invb, hipStream_t s) {
     hipLaunchKernelGGL((k_gather_ref<T, true>), ref_grid(p, np), dim3(256), 0, s, qs, qt, np, sx, ldx, p.kemn, p.eps,
-                       p.eoff, p.ntrunc, p.nlm, p.nlme, (T)sa, (T)sb, inva, invb);
+                       p.ntrunc, p.nlm, p.nlme, (T)sa, (T)sb, inva, invb);
 }
 
 template <typename T>
 void launch_scatter_ref(const Plan<T> &p, const T *sx, int ldx, cplx<T> *q, int nf, hipStream_t s) {
     hipLaunchKernelGGL((k_scatter_ref<T, false>), ref_grid(p, nf), dim3(256), 0, s, sx, ldx, q, (cplx<T> *)nullptr, nf,
-                       p.kemn, p.eps, p.eoff, p.ntrunc, p.nlm, p.nlme, T(1), 0);
+                       p.kemn, p.eps, p.ntrunc, p.nlm, p.nlme, T(1), 0);
 }
 
 template <typename T>
 void launch_scatter_ref_vec(const Plan<T> &p, const T *sx, int ldx, cplx<T> *qv, cplx<T> *qd, int np, double rsphere,
                             int inv, hipStream_t s) {
     hipLaunchKernelGGL((k_scatter_ref<T, true>), ref_grid(p, np), dim3(256), 0, s, sx, ldx, qv, qd, np, p.kemn, p.eps,
-                       p.eoff, p.ntrunc, p.nlm, p.nlme, (T)(1.0 / rsphere), inv);
+                       p.ntrunc, p.nlm, p.nlme, (T)(1.0 / rsphere), inv);
 }
 
 template <typename T>
@@ -2067,11 +2071,11 @@ void launch_fft_anal(const Plan<T> &p, const T *grid, long gstride, int nf, cons
 template <typename T>
 void launch_anal_scatter(const Plan<T> &p, const T *sx, int ldx, const AnalDesc *desc, int nfo, cplx<T> *dst,
                          long df, long dk, double rsphere, hipStream_t s, const int *nfdyn, bool massfix) {
-    const int bs = nfo >= 256 ? 256 : 64 * ((nfo + 63) / 64);
-    dim3 grid((nfo + bs - 1) / bs, (p.nlm + SCATTER_KE - 1) / SCATTER_KE);
-    auto kern = massfix ? k_anal_scatter<T, true> : k_anal_scatter<T, false>;
-    hipLaunchKernelGGL(kern, grid, dim3(bs), 0, s, sx, ldx, desc, nfo, dst, df, dk, p.kmn, p.keoff, p.eps, p.eoff,
-                       (T)(1.0 / rsphere), p.nlm, nfdyn);
+    const int bs = nfo >= 256 ? 256 : 64 * ((nfo + 63) / 64), nb = (nfo + bs - 1) / bs, rows = row_batch(p.nlm, nb);
+    auto kern = rows == 4 ? (massfix ? k_anal_scatter<T, true, 4> : k_anal_scatter<T, false, 4>)
+                          : (massfix ? k_anal_scatter<T, true, 8> : k_anal_scatter<T, false, 8>);
+    hipLaunchKernelGGL(kern, dim3(nb, (p.nlm + rows - 1) / rows), dim3(bs), 0, s, sx, ldx, desc, nfo, dst, df, dk,
+                       p.kmn, p.eps, (T)(1.0 / rsphere), p.nlm, nfdyn);
 }
 
 #define INST(T)                                                                                                \
