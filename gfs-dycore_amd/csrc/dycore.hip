@@ -668,26 +668,33 @@ template <typename T> struct PairSum {
     }
 };
 
-// columns of a member from which a getdyntend call takes k_columns_serial (FP32)
-static bool columns_serial(long ng) { return ng >= 100000; }
+// Whether a dynamics pass takes k_columns_serial. FP32: a getdyntend call (it hands the
+// grids and the tendency itself out) of a member with 100 000 columns. FP64: any pass
+// without tracers of 50 000 columns in all, enough for a thread each. k_columns and this
+// kernel in us a launch, 64 levels: T84 (33 000 columns) 63 and 84, T126 149 and 134, T170
+// 252 and 183, T254 558 and 402, 8 members at T62 with 28 levels 104 and 89. With a tracer
+// a T126 moist step takes 1.30 and 1.41 ms: here it is advected in a pass of its own.
+template <typename T> static bool columns_serial(long ng, int nm, int ntr, bool grids) {
+    return sizeof(T) == 4 ? grids && ng >= 100000 : ntr == 0 && nm * ng >= 50000;
+}
 // The dynamics columns with one thread per column, every sum in the order of the
-// reference's recursions (FP32). The curl of the pressure gradient nearly
+// reference's recursions. FP32: the curl of the pressure gradient nearly
 // vanishes, so the vorticity tendency carries the rounding of getpresgrad's
 // terms and sums: 5e-5 of itself at T254, 3e-5 at T170, and k_columns' order of
 // them moves it by 3e-5 and 2e-5. Inside advance that is a few parts in 1e6 of
 // the state; a getdyntend call hands the tendency itself out, and takes this
-// kernel where the columns fill the chip with one thread each (columns_serial):
-// 232 us at T254L64, k_columns 193.
-template <bool VC>
-__global__ __launch_bounds__(256) void k_columns_serial(
-    const float *__restrict__ gsyn, float *__restrict__ gan, float *__restrict__ etadot, float *__restrict__ dlnpdt,
-    float *__restrict__ psg_out, float *__restrict__ dlnpsdt_out, const float *__restrict__ dphisdx,
-    const float *__restrict__ dphisdy, const float *__restrict__ ak_, const float *__restrict__ bk_,
-    const float *__restrict__ ck_, const float *__restrict__ dbk_, const float *__restrict__ dak_, const float *__restrict__ sinlat,
-    int nl, int ntr, int nsyn, int nan, long ng, int nlon, float rd, float kappa, float cvcp, float twoom,
-    const cplx<float> *__restrict__ spec, int nfs, float *__restrict__ colq, const float *__restrict__ vcg,
-    const float *__restrict__ svcg, const float *__restrict__ vfsvc, float vcamp, int) {
-    typedef float T;
+// kernel where the columns fill the chip with one thread each:
+// 232 us at T254L64, k_columns 193. FP64 (three wavefronts a SIMD) takes it for its fewer
+// operations: bound by them, where k_columns forms prefix sums over its threads besides.
+template <typename T, bool VC>
+__global__ __launch_bounds__(256, sizeof(T) == 8 ? 3 : 4) void k_columns_serial(
+    const T *__restrict__ gsyn, T *__restrict__ gan, T *__restrict__ etadot, T *__restrict__ dlnpdt,
+    T *__restrict__ psg_out, T *__restrict__ dlnpsdt_out, const T *__restrict__ dphisdx,
+    const T *__restrict__ dphisdy, const T *__restrict__ ak_, const T *__restrict__ bk_,
+    const T *__restrict__ ck_, const T *__restrict__ dbk_, const T *__restrict__ dak_, const T *__restrict__ sinlat,
+    int nl, int ntr, int nsyn, int nan, long ng, int nlon, T rd, T kappa, T cvcp, T twoom,
+    const cplx<T> *__restrict__ spec, int nfs, T *__restrict__ colq, const T *__restrict__ vcg,
+    const T *__restrict__ svcg, const T *__restrict__ vfsvc, T vcamp, int store) {
     __shared__ T ak[MAXLEV + 1], bk[MAXLEV + 1], ck[MAXLEV], dbk[MAXLEV], dak[MAXLEV];
     for (int i = threadIdx.x; i <= nl; i += blockDim.x) {
         ak[i] = ak_[i];
@@ -732,7 +739,8 @@ __global__ __launch_bounds__(256) void k_columns_serial(
     // pass 1 (top -> bottom): getomega's sums db, cb and their column totals
     T db = 0, cb = 0;
     PairSum<T> sdb, scb;
-    ET[(long)nl * ng] = T(0);
+    const bool st_et = store || ntr > 0;  // the tracers read etadot back
+    if (st_et) ET[(long)nl * ng] = T(0);
     constexpr int P1G = 4;  // levels whose loads are issued together
     for (int K0 = 1; K0 <= nl; K0 += P1G) {
         T gu[P1G], gv[P1G], gd[P1G];
@@ -781,6 +789,7 @@ __global__ __launch_bounds__(256) void k_columns_serial(
     T um = 0, vm = 0, tm = 0;                          // level L - 1
     T u = LV(U, 1), v = LV(V, 1), tv = LV(TV, 1);      // level L
     T eb = T(0);                                       // etadot at the layer's bottom interface
+    T rpb = recip(pk(nl + 1));                         // and the reciprocal of the pressure there
     PairSum<T> rdb, rcb;
     constexpr int P3G = 2;  // levels whose loads are issued together
     for (int K0 = nl; K0 >= 1; K0 -= P3G) {
@@ -815,9 +824,10 @@ __global__ __launch_bounds__(256) void k_columns_serial(
             const T dba = sdb.minus(rdb), cba = scb.minus(rcb);  // sums over the layers above K
             T ea = T(0);                                   // etadot at the top interface K - 1
             if (K > 1) ea = (-(ps * cba) - dba) - (ps * bk[K - 1]) * dlnpsdt;
-            ET[(long)(K - 1) * ng] = ea;
+            if (st_et) ET[(long)(K - 1) * ng] = ea;
             T rlnp = rlnp1, alfa = alfa1, cofa, dbp;
-            const T rp1 = recip(p1), rp2 = recip(p2);
+            const T rp1 = recip(p1), rp2 = rpb;
+            rpb = rp1;
             if (K == 1) {
                 cofa = -rdp * (bk[K] * p1 * rp2 - bk[K - 1] + rlnp * (bk[K - 1] - p1 * dbk[K - 1] * rdp));
                 dbp = bk[K] * rp2 - bk[K - 1] * rp1;
@@ -848,7 +858,7 @@ __global__ __launch_bounds__(256) void k_columns_serial(
                 vt = h * (eb * (tm - tv) + ea * (tv - tp));
             }
             const T om = omega_p(K, dba, cba, o, dv, dpk, rdp, rlnp, alfa);
-            LV(WD, L) = om;
+            if (store) LV(WD, L) = om;
             T vq = kappa * om * tv;
             if (ntr > 0) vq = vq / (T(1) + cvcp * LV(Q, L));
             vv -= prsgy;
@@ -3379,12 +3389,11 @@ template <typename T> struct Step {
                            B.st_on[0] ? (const T *)B.st_grd : (const T *)nullptr, (const T *)B.st_vf,
                            (T)B.sc.vcamp, store);
         };
-        if constexpr (sizeof(T) == 4)
-            if (grids && !inverse_only && columns_serial(B.ng)) {
-                launch(vc ? k_columns_serial<true> : k_columns_serial<false>, (unsigned)((B.ng + 255) / 256), 256);
-                mark("columns");
-                return;
-            }
+        if (!inverse_only && columns_serial<T>(B.ng, B.nm, B.ntr, grids)) {
+            launch(vc ? k_columns_serial<T, true> : k_columns_serial<T, false>, (unsigned)((B.ng + 255) / 256), 256);
+            mark("columns");
+            return;
+        }
         constexpr int NC = ColCfg<T>::NC, CH = ColCfg<T>::CH, LPC = MAXLEV / CH;
         const bool half = B.nl <= CH * LPC / 2;  // half the registers for the layers where they suffice
         auto pick = [&](auto mode, auto tr) {

@@ -113,10 +113,12 @@ def test_transforms_every_length(grid, nf, monkeypatch):
 
 
 # chunks of layers: one per thread, most empty, partial, full and half full ones; a member's columns on and off the
-# 64 (FP64: 32) of a workgroup; T170 has the columns for which a getdyntend call takes one thread per column in FP32
+# 64 (FP64: 32) of a workgroup; T170 has the columns for which a getdyntend call takes one thread per column in FP32,
+# T84 those (of two members) for which a pass without tracers does in FP64
 @pytest.mark.parametrize("grid,nlev,ntrac", [((64, 32, 21), 2, 1), ((64, 32, 21), 7, 0), ((72, 36, 23), 17, 2),
                                              ((72, 36, 23), 32, 1), ((64, 32, 21), 33, 1), ((72, 36, 23), 63, 0),
-                                             ((64, 32, 21), 64, 2), ((512, 256, 170), 5, 1)])
+                                             ((64, 32, 21), 64, 2), ((512, 256, 170), 5, 1),
+                                             ((256, 128, 84), 5, 0), ((256, 128, 84), 18, 0)])
 def test_columns_every_chunk(grid, nlev, ntrac):
     """Tendencies, omega/p and etadot grids of getdyntend and of its inverse-only form, two members, against the
     oracle at the bounds of test_gpu_dycore (FP64 1e-9, FP32 2e-4)."""
