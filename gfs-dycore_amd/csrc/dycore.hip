@@ -1253,16 +1253,13 @@ __global__ __launch_bounds__(256) void k_area(T *__restrict__ a, const T *__rest
 }
 
 // Simple moist physics on the post-dynamics grid (phy_run_simple.f90:50-107
-// around simple_physics_v5_1.f90), one thread per column and member, column
-// arithmetic in FP64 as the reference's r8 routine. The column runs top ->
-// bottom (c = 1 model top .. nl lowest level; grid level L = nl + 1 - c).
-// Large-scale condensation (265-292) is evaluated level by level inside the
-// upward (bottom -> top) elimination sweep of the implicit boundary-layer
-// solve (375-431); the sweep's coefficients CE/CEm go to pbl scratch and
-// CFu/CFv/CFt/CFq to the output slots, which the downward back-substitution
-// (432-447) overwrites with the final grid changes. Output per member
-// (nsp fields): dT(Tv), du, dv, dq (nlev each; changes over the step, the
-// 1/dt is applied in the analysis) and the mass-fixer slot.
+// around simple_physics_v5_1.f90), column arithmetic in FP64 as the reference's
+// r8 routine. The column runs top -> bottom (c = 1 model top .. nl lowest level;
+// grid level L = nl + 1 - c): large-scale condensation (265-292) and the surface
+// fluxes (344-366) level by level, then the upward (bottom -> top) elimination
+// and the downward back-substitution (375-447) of the implicit boundary layer.
+// Output per member (nsp fields): dT(Tv), du, dv, dq (nlev each; changes over the
+// step, the 1/dt is applied in the analysis) and the mass-fixer slot.
 struct SimpleCfg {
     double dt, fv, qmin, grav;
     int sst_mode, turbflux;
@@ -3335,7 +3332,7 @@ template <typename T> struct Step {
     }
     // the lean Held-Suarez pass: temperature, ln ps and the vorticity and
     // divergence of the levels where the last lean pass found drag (and one
-    // more) into their grid slots; ps as the column kernel forms it (k_psg);
+    // more) into their grid slots; ps as the column kernel forms it (k_area);
     // the levels where the drag can act now (with the area sums); and, only
     // where those reach past the first synthesis, the vorticity and divergence
     // of all of them

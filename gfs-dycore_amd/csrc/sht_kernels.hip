@@ -138,9 +138,8 @@ __global__ void k_legendre_table(T *plm, const long *poff, const double *mu, int
 // ---------------------------------------------------------------------------
 // Legendre GEMMs. One workgroup = one order m, a 64-row x 128-column output tile;
 // 4 waves in a 2x2 arrangement, each wave 32 x 64 via 2 x 4 MFMA 16x16x4 blocks.
-// The synthesis gives each parity of n - m its own workgroup (half the
-// accumulators: 7 waves per SIMD instead of 3); the analysis keeps both
-// parities in one workgroup, which measured faster there. Global loads are 16-byte vectors,
+// Each parity of n - m has its own workgroup (half the accumulators: 7 waves per
+// SIMD instead of 3). Global loads are 16-byte vectors,
 // prefetched into registers for chunk k+1 while chunk k is computed from LDS.
 // FP32 swaps the MFMA operands (C^T = B^T A^T) so the four accumulators of a lane
 // are four consecutive columns of one output row and the epilogue stores 16-byte
