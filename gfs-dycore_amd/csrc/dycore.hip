@@ -739,7 +739,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 3 : 4) void k_columns_serial(
     // pass 1 (top -> bottom): getomega's sums db, cb and their column totals
     T db = 0, cb = 0;
     PairSum<T> sdb, scb;
-    const bool st_et = store || ntr > 0;  // the tracers read etadot back
+    // FP32 always stores the grids (its calls hand them out), without a branch: one there
+    // changes how the interface pressures are fused, which the vorticity tendency shows
+    const bool st_om = sizeof(T) == 4 || store, st_et = st_om || ntr > 0;  // the tracers read etadot back
     if (st_et) ET[(long)nl * ng] = T(0);
     constexpr int P1G = 4;  // levels whose loads are issued together
     for (int K0 = 1; K0 <= nl; K0 += P1G) {
@@ -826,7 +828,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 3 : 4) void k_columns_serial(
             if (K > 1) ea = (-(ps * cba) - dba) - (ps * bk[K - 1]) * dlnpsdt;
             if (st_et) ET[(long)(K - 1) * ng] = ea;
             T rlnp = rlnp1, alfa = alfa1, cofa, dbp;
-            const T rp1 = recip(p1), rp2 = rpb;
+            // FP64, bound by its operations, takes the reciprocal from the layer below
+            const T rp1 = recip(p1), rp2 = sizeof(T) == 4 ? recip(p2) : rpb;
             rpb = rp1;
             if (K == 1) {
                 cofa = -rdp * (bk[K] * p1 * rp2 - bk[K - 1] + rlnp * (bk[K - 1] - p1 * dbk[K - 1] * rdp));
@@ -858,7 +861,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 3 : 4) void k_columns_serial(
                 vt = h * (eb * (tm - tv) + ea * (tv - tp));
             }
             const T om = omega_p(K, dba, cba, o, dv, dpk, rdp, rlnp, alfa);
-            if (store) LV(WD, L) = om;
+            if (st_om) LV(WD, L) = om;
             T vq = kappa * om * tv;
             if (ntr > 0) vq = vq / (T(1) + cvcp * LV(Q, L));
             vv -= prsgy;
