@@ -354,31 +354,45 @@ __global__ __launch_bounds__(ColCfg<T>::NC * ColCfg<T>::CH, sizeof(T) * LPC <= 1
     const T *U = G, *V = G + (long)nl * ng, *VRT = G + 2L * nl * ng, *DIV = G + 3L * nl * ng;
     const T *TV = G + 4L * nl * ng, *TX = G + 5L * nl * ng, *TY = G + 6L * nl * ng, *Q = G + 7L * nl * ng;
     const T *LNPS = G + (7L + 3L * ntr) * nl * ng;
-    // this column's value at level lev = L - 1 = nl - K of a field of nl (+ 1) levels:
-    // a descriptor in scalar registers, the level's offset in one and the column's
-    // in a vector register, so that no access takes vector arithmetic
+    // This column's value at layer K = K0 + 1 + i (clamped to the column) of a field of
+    // nl levels, level nl - K: the descriptor starts at the wavefront's lowest level, so
+    // that a field may be of any size, the layer's offset is in a scalar register and the
+    // column's in a vector register, where FP64 also has the distance between the
+    // wavefront's two chunks (a layer's offset that differed between them would make
+    // every access a loop over the two).
+    constexpr bool TWO = NC < 64;
     const unsigned lb = (unsigned)(ng * sizeof(T));
-    auto ld = [&](const T *P, int lev) { return buf_load(P, cb, (unsigned)lev * lb); };
-    auto st = [&](T *P, int lev, T x) { buf_store(P, cb, (unsigned)lev * lb, x); };
+    const int w0 = __builtin_amdgcn_readfirstlane(tid / NC);  // the wavefront's first chunk
+    const int Kw = TWO ? (w0 + 1) * lpc : K0;                 // layers above its last one
+    auto level = [&](int K, int i) { return min(max(nl - 1 - K - i, 0), nl - 1); };
+    const int low = level(Kw, lpc + 1);  // tracers reach two layers past the chunk
+    auto voff = [&](int i) { return TWO ? cb + (unsigned)(level(K0, i) - level(Kw, i)) * lb : cb; };
+    auto soff = [&](int i) { return (unsigned)(level(Kw, i) - low) * lb; };
+    auto ld = [&](const T *P, int i) { return buf_load(P + (long)low * ng, voff(i), soff(i)); };
+    auto st = [&](T *P, int i, T x) { buf_store(P + (long)low * ng, voff(i), soff(i), x); };
+    // etadot at interface K0 + i, counted from the top
+    const int top = w0 * lpc;
+    const unsigned ve = TWO ? cb + (unsigned)(K0 - top) * lb : cb;
+    T *ET = etadot + (long)mem * (nl + 1) * ng;
+    auto ste = [&](int i, T x) { buf_store(ET + (long)top * ng, ve, (unsigned)i * lb, x); };
     T u[LPC], v[LPC], dv[LPC], tv[LPC], tx[LPC], ty[LPC], vr[LPC], q1[LPC];
 #pragma unroll
     for (int i = 0; i < LPC; i++)
         if (i < lpc) {
-            const int lev = max(nl - (K0 + 1 + i), 0);  // clamped: past the lowest layer nothing is used
-            u[i] = ld(U, lev);
-            v[i] = ld(V, lev);
-            dv[i] = ld(DIV, lev);
+            u[i] = ld(U, i);  // past the lowest layer nothing is used
+            v[i] = ld(V, i);
+            dv[i] = ld(DIV, i);
             if constexpr (DYN) {
-                tv[i] = ld(TV, lev);
-                tx[i] = ld(TX, lev);
-                ty[i] = ld(TY, lev);
-                vr[i] = ld(VRT, lev);
-                if constexpr (TR) q1[i] = ld(Q, lev);
+                tv[i] = ld(TV, i);
+                tx[i] = ld(TX, i);
+                ty[i] = ld(TY, i);
+                vr[i] = ld(VRT, i);
+                if constexpr (TR) q1[i] = ld(Q, i);
             }
         }
-    const T dpx = ld(LNPS, 1), dpy = ld(LNPS, 2);
+    const T dpx = LNPS[ng + col], dpy = LNPS[2 * ng + col];
     const T c00 = spec[(long)mem * nfs + 3L * nl + (long)ntr * nl].x;
-    const T ps = full_ps(c00, ld(LNPS, 0));
+    const T ps = full_ps(c00, LNPS[col]);
     const T gpx = ps * dpx, gpy = ps * dpy;
     const T alfa1 = T(SGLF(0.69314718055994530942)), rlnp1 = T(SGLF(99999.99));
     __syncthreads();  // the level tables
@@ -461,7 +475,7 @@ __global__ __launch_bounds__(ColCfg<T>::NC * ColCfg<T>::CH, sizeof(T) * LPC <= 1
         T s = T(0);
         for (int i = 0; i < cnt; i++) {
             T qs = T(0);
-            for (int nt = 0; nt < ntr; nt++) qs += ld(Q + (long)nt * nl * ng, nl - (K0 + 1 + i));
+            for (int nt = 0; nt < ntr; nt++) qs += ld(Q + (long)nt * nl * ng, i);
             s += dp(K0 + 1 + i) * qs;
         }
         sh[S_CQ][w][ln] = s;
@@ -493,16 +507,16 @@ __global__ __launch_bounds__(ColCfg<T>::NC * ColCfg<T>::CH, sizeof(T) * LPC <= 1
         const int K = K0 + i;
         return (K > 0 && K < nl) ? -s - (ps * bk[K]) * dlnpsdt : T(0);
     };
-    T *ET = etadot + (long)mem * (nl + 1) * ng, *WD = dlnpdt + (long)mem * nl * ng;
+    T *WD = dlnpdt + (long)mem * nl * ng;
     if constexpr (!DYN) {
 #pragma unroll
         for (int i = 0; i < LPC; i++)
             if (i < cnt) {
                 const int K = K0 + 1 + i;
                 const T s = above(i);
-                st(WD, nl - K, w2[i] - w1[i] * s);
-                st(ET, K - 1, eta(i, s));
-                if (K == nl) st(ET, nl, T(0));
+                st(WD, i, w2[i] - w1[i] * s);
+                ste(i, eta(i, s));
+                if (K == nl) ste(i + 1, T(0));
             }
     } else {
         cof = px = py = T(0);
@@ -533,14 +547,14 @@ __global__ __launch_bounds__(ColCfg<T>::NC * ColCfg<T>::CH, sizeof(T) * LPC <= 1
 #pragma unroll
         for (int i = LPC - 1; i >= 0; i--)
             if (i < cnt) {
-                const int K = K0 + 1 + i, lev = nl - K;
+                const int K = K0 + 1 + i;
                 const T up = i > 0 ? u[i > 0 ? i - 1 : 0] : ua, vp = i > 0 ? v[i > 0 ? i - 1 : 0] : va;
                 const T tp = i > 0 ? tv[i > 0 ? i - 1 : 0] : ta;
                 const T s = above(i), ea = eta(i, s), om = w2[i] - w1[i] * s;
                 if (store) {
-                    st(WD, lev, om);
-                    st(ET, K - 1, ea);
-                    if (K == nl) st(ET, nl, T(0));
+                    st(WD, i, om);
+                    ste(i, ea);
+                    if (K == nl) ste(i + 1, T(0));
                 }
                 // getvadv for u, v, tv
                 const T h = T(0.5) * recip(dp(K)), hb = h * eb, ha = h * ea;
@@ -549,23 +563,23 @@ __global__ __launch_bounds__(ColCfg<T>::NC * ColCfg<T>::CH, sizeof(T) * LPC <= 1
                 const T vt = hb * (tm - tv[i]) + ha * (tv[i] - tp);
                 T vq = kappa * om * tv[i];
                 if constexpr (TR) vq = vq / (T(1) + cvcp * q1[i]);
-                st(TT, lev, adv[i] - vt + vq);
+                st(TT, i, adv[i] - vt + vq);
                 T fx = fx0[i] + vv - by, fy = fy0[i] - vu + bx;
                 if constexpr (VC) {
                     // up-gradient vorticity flux vc |vrt| grad(vrt) / |grad(vrt)|
                     const T *VCX = vcg + (long)mem * 2 * nl * ng, *VCY = VCX + (long)nl * ng;
-                    const T gx = ld(VCX, lev), gy = ld(VCY, lev), ag = sqrt(gx * gx + gy * gy);
+                    const T gx = ld(VCX, i), gy = ld(VCY, i), ag = sqrt(gx * gx + gy * gy);
                     T vcl = vcamp;
-                    if (svcg) vcl = (T(1) + vfsvc[lev] * svcg[(long)mem * ng + col]) * vcl;
+                    if (svcg) vcl = (T(1) + vfsvc[nl - K] * svcg[(long)mem * ng + col]) * vcl;
                     if (ag > T(FLT_MIN)) {
-                        const T av = fabs(ld(VRT, lev));
+                        const T av = fabs(ld(VRT, i));
                         fx += vcl * (gx / ag) * av;
                         fy += vcl * (gy / ag) * av;
                     }
                 }
-                st(FX, lev, fx);
-                st(FY, lev, fy);
-                st(KE, lev, T(0.5) * (u[i] * u[i] + v[i] * v[i]));
+                st(FX, i, fx);
+                st(FY, i, fy);
+                st(KE, i, T(0.5) * (u[i] * u[i] + v[i] * v[i]));
                 um = u[i];
                 vm = v[i];
                 tm = tv[i];
@@ -585,13 +599,12 @@ __global__ __launch_bounds__(ColCfg<T>::NC * ColCfg<T>::CH, sizeof(T) * LPC <= 1
             T D[LPC + 4], gx[LPC], gy[LPC];  // D[i] = D_{K0 - 1 + i}, clamped to the column
 #pragma unroll
             for (int i = 0; i < LPC + 4; i++)
-                if (i < lpc + 4) D[i] = ld(Qn, nl - min(max(K0 - 1 + i, 1), nl));
+                if (i < lpc + 4) D[i] = ld(Qn, i - 2);
 #pragma unroll
             for (int i = 0; i < LPC; i++)
                 if (i < lpc) {
-                    const int lev = max(nl - (K0 + 1 + i), 0);
-                    gx[i] = ld(QXn, lev);
-                    gy[i] = ld(QYn, lev);
+                    gx[i] = ld(QXn, i);
+                    gy[i] = ld(QYn, i);
                 }
             // dd_K, K = K0 - 1 + i: D_{K+1} - D_K, guarded; at the top and the surface from two layers
             auto dd = [&](int i) {
@@ -624,7 +637,7 @@ __global__ __launch_bounds__(ColCfg<T>::NC * ColCfg<T>::CH, sizeof(T) * LPC <= 1
                     const T eb2 = eta(i + 1, above(i + 1));
                     const T hk = half(i + 1, eb2), Dk = D[i + 2];
                     const T vadv = recip(dp(K)) * ((hk * eb2 - hp * et) + (Dk * (et - eb2)));
-                    st(DQ, nl - K, -u[i] * gx[i] - v[i] * gy[i] - vadv);
+                    st(DQ, i, -u[i] * gx[i] - v[i] * gy[i] - vadv);
                     hp = hk;
                     et = eb2;
                 }
