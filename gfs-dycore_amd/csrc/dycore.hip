@@ -683,12 +683,18 @@ template <typename T> struct PairSum {
 
 // Whether a dynamics pass takes k_columns_serial. FP32: a getdyntend call (it hands the
 // grids and the tendency itself out) of a member with 100 000 columns. FP64: any pass
-// without tracers of 50 000 columns in all, enough for a thread each. k_columns and this
-// kernel in us a launch, 64 levels: T84 (33 000 columns) 63 and 84, T126 149 and 134, T170
-// 252 and 183, T254 558 and 402, 8 members at T62 with 28 levels 104 and 89. With a tracer
-// a T126 moist step takes 1.30 and 1.41 ms: here it is advected in a pass of its own.
-template <typename T> static bool columns_serial(long ng, int nm, int ntr, bool grids) {
-    return sizeof(T) == 4 ? grids && ng >= 100000 : ntr == 0 && nm * ng >= 50000;
+// without tracers that has columns enough for a thread each. k_columns and this kernel in
+// us a launch, FP64: 64 levels T84 (33 000 columns) 58 and 90, T126 (73 000) 128 and 142,
+// two members at T95 (83 000) 148 and 142, T170 218 and 189, T254 444 and 446; 28 levels,
+// where k_columns takes half the registers, two members at T84 (66 000) 44 and 50, T126 49
+// and 62, eight at T62 (144 000) 86 and 98, but T170 (131 000) 91 and 73, T254 185 and 186.
+// With 33 to 43 levels its 16 threads a column have three layers each and up to a third of
+// them few or none: 36 levels two members at T84 77 and 67, 44 levels 85 and 84, T126 95 and
+// 102. With a tracer a T126 moist step takes 1.30 and 1.41 ms: here it is advected in a pass
+// of its own.
+template <typename T> static bool columns_serial(long ng, int nm, int ntr, int nl, bool grids) {
+    if (sizeof(T) == 4) return grids && ng >= 100000;
+    return ntr == 0 && nm * ng >= (nl <= 32 ? 100000 : nl < 44 ? 50000 : 80000);
 }
 // The dynamics columns with one thread per column, every sum in the order of the
 // reference's recursions. FP32: the curl of the pressure gradient nearly
@@ -3402,7 +3408,7 @@ template <typename T> struct Step {
                            B.st_on[0] ? (const T *)B.st_grd : (const T *)nullptr, (const T *)B.st_vf,
                            (T)B.sc.vcamp, store);
         };
-        if (!inverse_only && columns_serial<T>(B.ng, B.nm, B.ntr, grids)) {
+        if (!inverse_only && columns_serial<T>(B.ng, B.nm, B.ntr, B.nl, grids)) {
             launch(vc ? k_columns_serial<T, true> : k_columns_serial<T, false>, (unsigned)((B.ng + 255) / 256), 256);
             mark("columns");
             return;

@@ -35,3 +35,27 @@ def test_fields_past_4gib():
         g.close()
     for k, tol in (("dvrt", 1e-9), ("ddiv", 1e-9), ("dtv", 1e-9), ("dlnps", 1e-9), ("dtrac", 1e-3)):
         assert rel(tg[k][0], to[k]) < tol, (k, rel(tg[k][0], to[k]))
+
+
+# on both sides of the column counts from which a pass takes one thread per column: FP64 without tracers 50 000 in all
+# at 33 to 43 levels, 80 000 at more and 100 000 at fewer; FP32, a getdyntend call, 100 000 a member
+@pytest.mark.parametrize("prec,grid,nlev,nmem", [("fp64", (128, 194, 31), 34, 2), ("fp64", (128, 196, 31), 34, 2),
+                                                 ("fp64", (256, 156, 21), 44, 2), ("fp64", (256, 160, 21), 44, 2),
+                                                 ("fp64", (256, 194, 42), 5, 2), ("fp64", (256, 196, 42), 5, 2),
+                                                 ("fp32", (512, 194, 42), 5, 2), ("fp32", (512, 196, 42), 5, 2)])
+def test_columns_by_size(prec, grid, nlev, nmem):
+    """Tendencies of each member against the oracle at the bounds of test_gpu_dycore (FP64 1e-9, FP32 2e-4)."""
+    import gfsdc
+    nlon, nlat, T = grid
+    ak, bk = levels.hybrid_levels(nlev)
+    p, tol = (gfsdc.FP64, 1e-9) if prec == "fp64" else (gfsdc.FP32, 2e-4)
+    g = gfsdc.Context(nlon, nlat, T, p, nlev=nlev, ak=ak, bk=bk, dt=600.0, nmem=nmem)
+    st = [cases.perturbed_state(g.degree, g.order, nlev, seed=5 + m, amp=0.3) for m in range(nmem)]
+    g.set_state(*[np.concatenate(x) for x in zip(*st)])
+    tg = g.getdyntend(1)
+    for m in range(nmem):
+        o = O.Model(nlon, nlat, T, nlev, ak, bk, 600.0)
+        o.set_state(*[x[0] for x in st[m]])
+        to = o.getdyntend(1)
+        for k in ("dvrt", "ddiv", "dtv", "dlnps"):
+            assert rel(tg[k][m], to[k]) < tol, (k, m, rel(tg[k][m], to[k]))
