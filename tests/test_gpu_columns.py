@@ -39,22 +39,30 @@ def test_fields_past_4gib():
 
 # on both sides of the column counts from which a pass takes one thread per column: FP64 without tracers 50 000 in all
 # at 33 to 43 levels, 80 000 at more and 100 000 at fewer; FP32, a getdyntend call, 100 000 a member
+@pytest.mark.parametrize("vc", ["plain", "vc", "vc_svc"])
 @pytest.mark.parametrize("prec,grid,nlev,nmem", [("fp64", (128, 194, 31), 34, 2), ("fp64", (128, 196, 31), 34, 2),
                                                  ("fp64", (256, 156, 21), 44, 2), ("fp64", (256, 160, 21), 44, 2),
                                                  ("fp64", (256, 194, 42), 5, 2), ("fp64", (256, 196, 42), 5, 2),
                                                  ("fp32", (512, 194, 42), 5, 2), ("fp32", (512, 196, 42), 5, 2)])
-def test_columns_by_size(prec, grid, nlev, nmem):
-    """Tendencies of each member against the oracle at the bounds of test_gpu_dycore (FP64 1e-9, FP32 2e-4)."""
+def test_columns_by_size(prec, grid, nlev, nmem, vc):
+    """Tendencies of each member without and with vorticity confinement, and with its svc pattern, against the oracle at
+    the bounds of test_gpu_stoch (FP64 1e-9, FP32 2e-4)."""
     import gfsdc
     nlon, nlat, T = grid
+    stoch = {"plain": None, "vc": dict(vcamp=8.0),
+             "vc_svc": dict(vcamp=8.0, svc=0.7, svc_tau=3 * 3600.0, svc_lscale=5.0e5, iseed_svc=9)}[vc]
     ak, bk = levels.hybrid_levels(nlev)
     p, tol = (gfsdc.FP64, 1e-9) if prec == "fp64" else (gfsdc.FP32, 2e-4)
     g = gfsdc.Context(nlon, nlat, T, p, nlev=nlev, ak=ak, bk=bk, dt=600.0, nmem=nmem)
     st = [cases.perturbed_state(g.degree, g.order, nlev, seed=5 + m, amp=0.3) for m in range(nmem)]
+    if stoch:
+        g.stoch_init(**stoch)
     g.set_state(*[np.concatenate(x) for x in zip(*st)])
     tg = g.getdyntend(1)
     for m in range(nmem):
         o = O.Model(nlon, nlat, T, nlev, ak, bk, 600.0)
+        if stoch:
+            o.stoch_init(**{k: v + m if k == "iseed_svc" else v for k, v in stoch.items()})
         o.set_state(*[x[0] for x in st[m]])
         to = o.getdyntend(1)
         for k in ("dvrt", "ddiv", "dtv", "dlnps"):
