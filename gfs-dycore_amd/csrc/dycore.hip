@@ -681,9 +681,9 @@ template <typename T> struct PairSum {
     }
 };
 
-// Whether a dynamics pass takes k_columns_serial. FP32: a getdyntend call (it hands the
-// grids and the tendency itself out) of a member with 100 000 columns. FP64: any pass
-// without tracers that has columns enough for a thread each. k_columns and this kernel in
+// Whether a dynamics pass takes k_columns_serial. FP32: a getdyntend call of a member with
+// 100 000 columns, which so keeps its order of sums (see there). FP64: any pass without
+// tracers that has columns enough for a thread each. k_columns and this kernel in
 // us a launch, FP64: 64 levels T84 (33 000 columns) 58 and 90, T126 (73 000) 128 and 142,
 // two members at T95 (83 000) 148 and 142, T170 218 and 189, T254 444 and 446; 28 levels,
 // where k_columns takes half the registers, two members at T84 (66 000) 44 and 50, T126 49
@@ -697,14 +697,17 @@ template <typename T> static bool columns_serial(long ng, int nm, int ntr, int n
     return ntr == 0 && nm * ng >= (nl <= 32 ? 100000 : nl < 44 ? 50000 : 80000);
 }
 // The dynamics columns with one thread per column, every sum in the order of the
-// reference's recursions. FP32: the curl of the pressure gradient nearly
-// vanishes, so the vorticity tendency carries the rounding of getpresgrad's
-// terms and sums: 5e-5 of itself at T254, 3e-5 at T170, and k_columns' order of
-// them moves it by 3e-5 and 2e-5. Inside advance that is a few parts in 1e6 of
-// the state; a getdyntend call hands the tendency itself out, and takes this
-// kernel where the columns fill the chip with one thread each:
-// 232 us at T254L64, k_columns 193. FP64 (three wavefronts a SIMD) takes it for its fewer
-// operations: bound by them, where k_columns forms prefix sums over its threads besides.
+// reference's recursions. In FP64 (three wavefronts a SIMD) the faster kernel where the
+// columns are enough, for its fewer operations: bound by them, where k_columns forms prefix
+// sums over its threads besides.
+// In FP32 it is the slower one (232 us at T254L64, k_columns 193) and no closer to 64
+// bits. The vorticity tendency shows the rounding most, as the curl of the pressure gradient
+// nearly vanishes; its error in the 2-norm here and in k_columns, rough states of 64
+// levels: T84 6.69e-6 and 6.68e-6, T126 9.12e-6 and 9.01e-6, T170 1.207e-5 and 1.213e-5,
+// T254 1.780e-5 and 1.778e-5; after a day of Held-Suarez T126 1.10e-6 and 1.09e-6, T254
+// 9.9e-7 and 9.9e-7; the other tendencies alike (2 %). What the FP32 rule keeps is the order
+// of sums itself, by which a large getdyntend call's single coefficients differ by up to
+// 3e-5 of the largest, and k_columns' passes inside advance by a few parts in 1e6 of the state.
 template <typename T, bool VC>
 __global__ __launch_bounds__(256, sizeof(T) == 8 ? 3 : 4) void k_columns_serial(
     const T *__restrict__ gsyn, T *__restrict__ gan, T *__restrict__ etadot, T *__restrict__ dlnpdt,
