@@ -49,7 +49,7 @@ __host__ __device__ inline uint64_t rng_mix(uint64_t seed, uint64_t stream, uint
 }
 
 struct Coeffs3 {
-    double a[3], aa[3];
+    double a[3];
 };
 
 struct DycoreBuffers {
@@ -61,7 +61,9 @@ struct DycoreBuffers {
     int nsp = 0;    // simple-physics grid fields per member: dT, du, dv, dq (nlev each), mass fixer
     long ng = 0;
     void *spec = nullptr, *spec0 = nullptr, *ten[3] = {nullptr, nullptr, nullptr};
-    void *lin[3] = {nullptr, nullptr, nullptr};  // linear terms: div[nl], tv[nl], lnps per member
+    // what the second and the third stage need of the earlier ones' tendencies and linear
+    // terms (k_si_mfma's E1, E2; none in the explicit scheme): div[nl], tv[nl], lnps per member
+    void *mix[2] = {nullptr, nullptr};
     void *tphys = nullptr;                       // physics tendencies
     void *gsyn = nullptr, *gan = nullptr;        // grid fields (T)
     void *gmean = nullptr;                       // global means added back by the Fourier synthesis (nm * nsyn)
@@ -76,7 +78,6 @@ struct DycoreBuffers {
     void *disspec = nullptr, *diffp = nullptr, *dmpp = nullptr;
     void *ak = nullptr, *bk = nullptr, *ck = nullptr, *dbk = nullptr, *dak = nullptr;  // T
     void *sinlat = nullptr, *coslat = nullptr, *areaw = nullptr;      // T, nlat; areaw FP64 nlat
-    int *kbydeg = nullptr;                       // coefficients sorted by degree
     int2 *si_tiles = nullptr;                    // (degree, first item) tiles of the matrix-core solve
     int n_si_tiles = 0;
     int *degree = nullptr;                       // degree of coefficient k
@@ -2047,195 +2048,47 @@ __global__ __launch_bounds__(1024) void k_diag(const T *__restrict__ gsyn, const
     }
 }
 
-// matvec over levels inside one wavefront: lane i returns sum_j M^T[j][i] x_j,
-// x_j taken from lane j through LDS (x holds re/im of this lane's level)
+// One stage of the explicit scheme for every spectral coefficient (run.f90:313-350,
+// 374-417, 440-489 without the linear terms) and, after the last stage, the
+// implicit damping (run.f90:493-502). One wavefront per (coefficient, member),
+// lane = model level (bottom -> top).
 template <typename T>
-__device__ inline cplx<T> wave_matvec(const T *__restrict__ Mt, cplx<T> x, cplx<T> *sh, int nl, int lane) {
-    sh[lane] = x;
-    __syncthreads();
-    cplx<T> acc{T(0), T(0)};
-    if (lane < nl) {
-        for (int j = 0; j < nl; j++) {
-            T a = Mt[j * nl + lane];
-            cplx<T> xj = sh[j];
-            acc.x += a * xj.x;
-            acc.y += a * xj.y;
-        }
-    }
-    __syncthreads();
-    return acc;
-}
-
-template <typename T>
-__device__ inline T wave_sum(T v, T *sh, int lane) {
-    sh[lane] = v;
-    __syncthreads();
-    T s = T(0);
-    for (int j = 0; j < 64; j++) s += sh[j];
-    __syncthreads();
-    return s;
-}
-
-// One IMEX RK stage for every spectral coefficient (run.f90:313-350, 374-417,
-// 440-489) and, after the last stage, the implicit damping (run.f90:493-502).
-// One wavefront per (coefficient, member), lane = model level (bottom -> top).
-// Workgroup = 4 wavefronts with the same total wavenumber (shared d_hyb_m in cache).
-template <typename T>
-__global__ __launch_bounds__(256) void k_si_stage(
-    cplx<T> *__restrict__ spec, const cplx<T> *__restrict__ spec0, cplx<T> *__restrict__ ten0,
-    cplx<T> *__restrict__ ten1, cplx<T> *__restrict__ ten2, cplx<T> *__restrict__ lin0,
-    cplx<T> *__restrict__ lin1, cplx<T> *__restrict__ lin2, const T *__restrict__ At, const T *__restrict__ Bt,
-    const T *__restrict__ Dt, const T *__restrict__ sv, const T *__restrict__ tor, const T *__restrict__ disspec,
-    const T *__restrict__ diffp, const T *__restrict__ dmpp, const int *__restrict__ kbydeg,
-    const int *__restrict__ degree, int stage, Coeffs3 cf, T cimp, int do_implicit, int explicit_, int damp,
-    int nl, int ntr, int nfs, int nm, int nlm, int ntrunc, T dt) {
-    __shared__ cplx<T> shc[4][64];
-    __shared__ T shr[4][64];
+__global__ __launch_bounds__(256) void k_explicit_stage(
+    cplx<T> *__restrict__ spec, const cplx<T> *__restrict__ spec0, const cplx<T> *__restrict__ ten0,
+    const cplx<T> *__restrict__ ten1, const cplx<T> *__restrict__ ten2, const T *__restrict__ disspec,
+    const T *__restrict__ diffp, const T *__restrict__ dmpp, int stage, Coeffs3 cf, int damp, int nl, int ntr, int nfs,
+    int nm, int nlm, T dt) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long item = (long)blockIdx.x * 4 + wave;  // (member, coefficient in degree order)
-    const bool active = item < (long)nlm * nm;
-    const int mem = active ? (int)(item / nlm) : 0;
-    const int k = active ? kbydeg[item % nlm] : 0;
-    const int n = degree[k];
-    const long NFS = (long)nfs * nm;
-    const long base = (long)k * NFS + (long)mem * nfs;
-    const long nlin = 2L * nl + 1;
-    const long lbase = (long)k * nlin * nm + (long)mem * nlin;
-    const T lap = -T(n) * T(n + 1);
-    const bool lv = active && lane < nl;
-    cplx<T> *tn[3] = {ten0, ten1, ten2};
-    cplx<T> *ln[3] = {lin0, lin1, lin2};
-    const cplx<T> z{T(0), T(0)};
-    // vorticity and tracers: always explicit
-    if (lv) {
-        cplx<T> acc = z;
+    const long item = (long)blockIdx.x * 4 + wave;  // (coefficient, member)
+    if (item >= (long)nlm * nm) return;
+    const int mem = (int)(item / nlm), k = (int)(item % nlm);
+    const long base = (long)k * nfs * nm + (long)mem * nfs;
+    const cplx<T> *tn[3] = {ten0, ten1, ten2};
+    auto stepped = [&](long off) {
+        cplx<T> acc{T(0), T(0)};
         for (int r = 0; r <= stage; r++) {
-            cplx<T> t = tn[r][base + lane];
+            const cplx<T> t = tn[r][off];
             acc.x += T(cf.a[r]) * t.x;
             acc.y += T(cf.a[r]) * t.y;
         }
-        cplx<T> o = spec0[base + lane];
-        spec[base + lane] = cplx<T>{o.x + dt * acc.x, o.y + dt * acc.y};
-        for (int q = 0; q < ntr; q++) {
-            long off = base + 3L * nl + (long)q * nl + lane;
-            cplx<T> a2 = z;
-            for (int r = 0; r <= stage; r++) {
-                cplx<T> t = tn[r][off];
-                a2.x += T(cf.a[r]) * t.x;
-                a2.y += T(cf.a[r]) * t.y;
-            }
-            cplx<T> o2 = spec0[off];
-            spec[off] = cplx<T>{o2.x + dt * a2.x, o2.y + dt * a2.y};
+        const cplx<T> o = spec0[off];
+        return cplx<T>{o.x + dt * acc.x, o.y + dt * acc.y};
+    };
+    const T ds = disspec[k];
+    for (int q = 0; q < 3 + ntr && lane < nl; q++) {  // vorticity, divergence, temperature, tracers
+        const long off = base + (long)q * nl + lane;
+        cplx<T> v = stepped(off);
+        if (damp) {
+            const T f = q < 2 ? T(1) - (ds * diffp[lane] - dmpp[lane]) * dt : T(1) - ds * diffp[lane] * dt;
+            v = cplx<T>{v.x / f, v.y / f};
         }
+        spec[off] = v;
     }
-    const long idv = base + nl + lane, itv = base + 2L * nl + lane, ilp = base + 3L * nl + (long)ntr * nl;
-    if (explicit_) {
-        if (lv) {
-            cplx<T> a1 = z, a2 = z;
-            for (int r = 0; r <= stage; r++) {
-                cplx<T> d = tn[r][idv], t = tn[r][itv];
-                a1.x += T(cf.a[r]) * d.x; a1.y += T(cf.a[r]) * d.y;
-                a2.x += T(cf.a[r]) * t.x; a2.y += T(cf.a[r]) * t.y;
-            }
-            cplx<T> d0 = spec0[idv], t0 = spec0[itv];
-            spec[idv] = cplx<T>{d0.x + dt * a1.x, d0.y + dt * a1.y};
-            spec[itv] = cplx<T>{t0.x + dt * a2.x, t0.y + dt * a2.y};
-        }
-        if (active && lane == 0) {
-            cplx<T> a = z;
-            for (int r = 0; r <= stage; r++) {
-                cplx<T> p = tn[r][ilp];
-                a.x += T(cf.a[r]) * p.x; a.y += T(cf.a[r]) * p.y;
-            }
-            cplx<T> p0 = spec0[ilp];
-            spec[ilp] = cplx<T>{p0.x + dt * a.x, p0.y + dt * a.y};
-        }
-    } else {
-        // linear terms of this stage's input state (run.f90:329-335)
-        const cplx<T> *sin_ = (stage == 0) ? spec0 : spec;
-        cplx<T> tvin = lv ? sin_[itv] : z, dvin = lv ? sin_[idv] : z;
-        cplx<T> lpin = active ? sin_[ilp] : z;
-        cplx<T> Atv = wave_matvec(At, tvin, shc[wave], nl, lane);
-        cplx<T> Bdv = wave_matvec(Bt, dvin, shc[wave], nl, lane);
-        T svl = lv ? sv[lane] : T(0), torl = lv ? tor[lane] : T(0);
-        T sdr = wave_sum(svl * dvin.x, shr[wave], lane), sdi = wave_sum(svl * dvin.y, shr[wave], lane);
-        cplx<T> ddl{-lap * (Atv.x + torl * lpin.x), -lap * (Atv.y + torl * lpin.y)};
-        cplx<T> dtl{-Bdv.x, -Bdv.y};
-        cplx<T> dpl{-sdr, -sdi};
-        cplx<T> *L = ln[stage];
-        if (lv) {
-            L[lbase + lane] = ddl;
-            L[lbase + nl + lane] = dtl;
-            tn[stage][idv] = cplx<T>{tn[stage][idv].x - ddl.x, tn[stage][idv].y - ddl.y};
-            tn[stage][itv] = cplx<T>{tn[stage][itv].x - dtl.x, tn[stage][itv].y - dtl.y};
-        }
-        if (active && lane == 0) {
-            L[lbase + 2L * nl] = dpl;
-            tn[stage][ilp] = cplx<T>{tn[stage][ilp].x - dpl.x, tn[stage][ilp].y - dpl.y};
-        }
-        __syncthreads();
-        // explicit part (run.f90:337-342 and the later-stage forms)
-        cplx<T> dvc = z, tvc = z, lpc = z;
-        if (lv) {
-            cplx<T> a1 = z, a2 = z;
-            for (int r = 0; r <= stage; r++) {
-                cplx<T> d = tn[r][idv], t = tn[r][itv];
-                cplx<T> ld = ln[r][lbase + lane], lt = ln[r][lbase + nl + lane];
-                a1.x += T(cf.a[r]) * d.x + T(cf.aa[r]) * ld.x; a1.y += T(cf.a[r]) * d.y + T(cf.aa[r]) * ld.y;
-                a2.x += T(cf.a[r]) * t.x + T(cf.aa[r]) * lt.x; a2.y += T(cf.a[r]) * t.y + T(cf.aa[r]) * lt.y;
-            }
-            cplx<T> d0 = spec0[idv], t0 = spec0[itv];
-            dvc = cplx<T>{d0.x + dt * a1.x, d0.y + dt * a1.y};
-            tvc = cplx<T>{t0.x + dt * a2.x, t0.y + dt * a2.y};
-        }
-        if (active) {
-            cplx<T> a = z;
-            for (int r = 0; r <= stage; r++) {
-                cplx<T> p = tn[r][ilp], lp = ln[r][lbase + 2L * nl];
-                a.x += T(cf.a[r]) * p.x + T(cf.aa[r]) * lp.x; a.y += T(cf.a[r]) * p.y + T(cf.aa[r]) * lp.y;
-            }
-            cplx<T> p0 = spec0[ilp];
-            lpc = cplx<T>{p0.x + dt * a.x, p0.y + dt * a.y};
-        }
-        if (do_implicit) {
-            // rhs, solve and back-substitution (run.f90:344-349)
-            cplx<T> At2 = wave_matvec(At, tvc, shc[wave], nl, lane);
-            cplx<T> rhs{dvc.x - cimp * lap * dt * (At2.x + torl * lpc.x),
-                        dvc.y - cimp * lap * dt * (At2.y + torl * lpc.y)};
-            const T *D = Dt + ((long)stage * (ntrunc + 1) + n) * nl * nl;
-            cplx<T> dn = wave_matvec(D, rhs, shc[wave], nl, lane);
-            cplx<T> Bd = wave_matvec(Bt, dn, shc[wave], nl, lane);
-            T s2r = wave_sum(svl * dn.x, shr[wave], lane), s2i = wave_sum(svl * dn.y, shr[wave], lane);
-            tvc.x -= cimp * dt * Bd.x;
-            tvc.y -= cimp * dt * Bd.y;
-            lpc.x -= cimp * dt * s2r;
-            lpc.y -= cimp * dt * s2i;
-            dvc = dn;
-        }
-        if (lv) {
-            spec[idv] = dvc;
-            spec[itv] = tvc;
-        }
-        if (active && lane == 0) spec[ilp] = lpc;
-    }
-    if (damp && lv) {
-        // run.f90:493-502
-        T ds = disspec[k];
-        T fv = T(1) - (ds * diffp[lane] - dmpp[lane]) * dt;
-        T ft = T(1) - ds * diffp[lane] * dt;
-        cplx<T> a = spec[base + lane], d = spec[idv], t = spec[itv];
-        spec[base + lane] = cplx<T>{a.x / fv, a.y / fv};
-        spec[idv] = cplx<T>{d.x / fv, d.y / fv};
-        spec[itv] = cplx<T>{t.x / ft, t.y / ft};
-        for (int q = 0; q < ntr; q++) {
-            long off = base + 3L * nl + (long)q * nl + lane;
-            cplx<T> c = spec[off];
-            spec[off] = cplx<T>{c.x / ft, c.y / ft};
-        }
-    }
+    const long ilp = base + (3L + ntr) * nl;
+    if (lane == 0) spec[ilp] = stepped(ilp);
 }
 
-// The same IMEX stage (run.f90:313-350, 374-417, 440-489, damping 493-502) as
+// One stage of the IMEX scheme (run.f90:313-350, 374-417, 440-489, damping 493-502) as
 // batched matrix products on the matrix cores: a workgroup takes up to
 // C = SiCfg<T>::C spectral coefficients of one total wavenumber n (each member's m = 0..n),
 // i.e. 2 C real columns of level vectors, and every level operator
@@ -2976,17 +2829,13 @@ template <typename T> int Engine<T>::dyn_init() {
         B->latd = (double *)p;
     }
     {
-        std::vector<int> deg(nlm), byd;
+        std::vector<int> deg(nlm);
         int k = 0;
         for (int m = 0; m <= T_; m++)
             for (int n = m; n <= T_; n++) deg[k++] = n;
-        for (int n = 0; n <= T_; n++)
-            for (int m = 0; m <= n; m++) byd.push_back(plan.koff_h[m] + n - m);
         void *p;
         if ((rc = dupload<int>(&p, deg, stream))) return rc;
         B->degree = (int *)p;
-        if ((rc = dupload<int>(&p, byd, stream))) return rc;
-        B->kbydeg = (int *)p;
         std::vector<int2> tiles;
         for (int n = 0; n <= T_; n++)
             for (int i0 = 0; i0 < (n + 1) * nm; i0 += SiCfg<T>::C) tiles.push_back(make_int2(n, i0));
@@ -2995,13 +2844,12 @@ template <typename T> int Engine<T>::dyn_init() {
         B->n_si_tiles = (int)tiles.size();
     }
     // ---- state and work buffers
-    size_t nspec = (size_t)nlm * NFS, nlin = (size_t)nlm * nm * (2 * nl + 1);
+    size_t nspec = (size_t)nlm * NFS;
     B->spec = dalloc<cplx<T>>(nspec);
     B->spec0 = dalloc<cplx<T>>(nspec);
-    for (int s = 0; s < 3; s++) {
-        B->ten[s] = dalloc<cplx<T>>(nspec);
-        B->lin[s] = dalloc<cplx<T>>(nlin);
-    }
+    for (int s = 0; s < 3; s++) B->ten[s] = dalloc<cplx<T>>(nspec);
+    if (!cfg.explicit_)
+        for (int s = 0; s < 2; s++) B->mix[s] = dalloc<cplx<T>>((size_t)nlm * nm * (2 * nl + 1));
     B->tphys = dalloc<cplx<T>>(nspec);
     B->topo = dalloc<cplx<T>>((size_t)nlm * nm);
     B->gsyn = dalloc<T>((size_t)nm * B->nsyn * ng);
@@ -3024,7 +2872,11 @@ template <typename T> int Engine<T>::dyn_init() {
     B->pwat = dalloc<T>((size_t)nm * ng);
     B->precip = dalloc<T>((size_t)nm * ng);
     B->hsdyn = dalloc<int>(8);
-    void *ptrs[] = {B->spec, B->spec0, B->ten[0], B->ten[1], B->ten[2], B->lin[0], B->lin[1], B->lin[2],
+    if (!cfg.explicit_ && (!B->mix[0] || !B->mix[1])) {
+        set_error("device allocation failed for the dycore state");
+        return GFSDC_ENOMEM;
+    }
+    void *ptrs[] = {B->spec, B->spec0, B->ten[0], B->ten[1], B->ten[2],
                     B->tphys, B->topo, B->gsyn, B->gan, B->etadot, B->dlnpdt, B->psg, B->dlnpsdt, B->dphisdx,
                     B->dphisdy, B->pdryini, B->pmean, B->diag, B->pspart, B->psdone, B->pwsum, B->colq, B->pwat,
                     B->precip, B->gmean, B->clock, B->hsdyn};
@@ -3285,10 +3137,10 @@ template <typename T> void Engine<T>::dyn_destroy() {
     if (!B) return;
     drop_graph(B);
     for (auto e : B->ev) (void)hipEventDestroy(e);
-    void *ptrs[] = {B->spec, B->spec0, B->ten[0], B->ten[1], B->ten[2], B->lin[0], B->lin[1], B->lin[2],
+    void *ptrs[] = {B->spec, B->spec0, B->ten[0], B->ten[1], B->ten[2], B->mix[0], B->mix[1],
                     B->tphys, B->gsyn, B->gan, B->etadot, B->dlnpdt, B->psg, B->dlnpsdt, B->dphisdx,
                     B->dphisdy, B->topo, B->at, B->bt, B->dt3, B->sv, B->tor, B->disspec, B->diffp, B->dmpp,
-                    B->ak, B->bk, B->ck, B->dbk, B->sinlat, B->coslat, B->areaw, B->kbydeg, B->degree, B->si_tiles,
+                    B->ak, B->bk, B->ck, B->dbk, B->sinlat, B->coslat, B->areaw, B->degree, B->si_tiles,
                     B->pdryini, B->pmean, B->pspart, B->psdone, B->diag, B->sdesc, B->adesc_dyn, B->adesc_hs, B->adesc_hsu,
                     B->rflag_syn,
                     B->rflag_an, B->rflag_hs, B->pwsum, B->colq, B->pwat, B->precip, B->latd,
@@ -3481,18 +3333,15 @@ template <typename T> struct Step {
     void si_stage(int stage, bool damp) {
         const gfsdc_cfg &c = E.cfg;
         Coeffs3 cf;
-        for (int r = 0; r < 3; r++) {
-            cf.a[r] = TAB_A[stage][r];
-            cf.aa[r] = TAB_AA[stage][r];
-        }
-        int do_imp = (stage < 2 || std::fabs(TAB_IMP[stage]) > 1.e-5) ? 1 : 0;
+        for (int r = 0; r < 3; r++) cf.a[r] = TAB_A[stage][r];
         if (si_mfma()) {
+            const int do_imp = (stage < 2 || std::fabs(TAB_IMP[stage]) > 1.e-5) ? 1 : 0;
             auto ta = [&](int r) { return r < 3 ? TAB_A[r][stage] : 0.0; };
             auto taa = [&](int r) { return r < 3 ? TAB_AA[r][stage] : 0.0; };
             const SiNext cn{ta(stage), taa(stage), ta(stage + 1), taa(stage + 1), ta(stage + 2), taa(stage + 2)};
             hipLaunchKernelGGL(k_si_mfma<T>, dim3((unsigned)B.n_si_tiles), dim3(256), 0, s, (T *)B.spec,
-                               (T *)B.spec0, (const T *)B.ten[0], (const T *)B.ten[1], (const T *)B.ten[2], (T *)B.lin[0],
-                               (T *)B.lin[1], (const T *)B.at, (const T *)B.bt, (const T *)B.dt3,
+                               (T *)B.spec0, (const T *)B.ten[0], (const T *)B.ten[1], (const T *)B.ten[2], (T *)B.mix[0],
+                               (T *)B.mix[1], (const T *)B.at, (const T *)B.bt, (const T *)B.dt3,
                                (const T *)B.sv, (const T *)B.tor, (const T *)B.disspec, (const T *)B.diffp,
                                (const T *)B.dmpp, (const int2 *)B.si_tiles, stage, cf, cn,
                                (T)TAB_IMP[stage], do_imp, damp ? 1 : 0, B.nl, B.ntr, B.nfs, B.nm, E.plan.ntrunc,
@@ -3501,13 +3350,10 @@ template <typename T> struct Step {
             return;
         }
         long items = (long)E.plan.nlm * B.nm;
-        hipLaunchKernelGGL(k_si_stage<T>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, (cplx<T> *)B.spec,
-                           (const cplx<T> *)B.spec0, (cplx<T> *)B.ten[0], (cplx<T> *)B.ten[1],
-                           (cplx<T> *)B.ten[2], (cplx<T> *)B.lin[0], (cplx<T> *)B.lin[1], (cplx<T> *)B.lin[2],
-                           (const T *)B.at, (const T *)B.bt, (const T *)B.dt3, (const T *)B.sv, (const T *)B.tor,
-                           (const T *)B.disspec, (const T *)B.diffp, (const T *)B.dmpp, B.kbydeg, B.degree, stage,
-                           cf, (T)TAB_IMP[stage], do_imp, c.explicit_, damp ? 1 : 0, B.nl, B.ntr, B.nfs, B.nm,
-                           E.plan.nlm, E.plan.ntrunc, (T)c.dt);
+        hipLaunchKernelGGL(k_explicit_stage<T>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, (cplx<T> *)B.spec,
+                           (const cplx<T> *)B.spec0, (const cplx<T> *)B.ten[0], (const cplx<T> *)B.ten[1],
+                           (const cplx<T> *)B.ten[2], (const T *)B.disspec, (const T *)B.diffp, (const T *)B.dmpp,
+                           stage, cf, damp ? 1 : 0, B.nl, B.ntr, B.nfs, B.nm, E.plan.nlm, (T)c.dt);
         mark("si_stage");
     }
     void physics() {

@@ -86,7 +86,7 @@ template <typename T> struct Plan {
     int2 *kmn = nullptr;     // device, spectral index -> (m, n)
     double *mu_d = nullptr, *w_d = nullptr;  // FP64 nodes / weights (device)
     std::vector<double> mu, w;               // host copies
-    std::vector<int> keoff_h, koff_h;
+    std::vector<int> keoff_h;
     std::vector<long> poff_h;
 };
 

@@ -1764,19 +1764,16 @@ template <typename T> int plan_create(Plan<T> &p, int nlon, int nlat, int ntrunc
     // offsets
     p.poff_h.resize(T_ + 2);
     p.keoff_h.resize(T_ + 2);
-    p.koff_h.resize(T_ + 2);
     std::vector<int> eoff_h(T_ + 2);
     long po = 0;
-    int ke = 0, k = 0, eo = 0;
+    int ke = 0, eo = 0;
     for (int m = 0; m <= T_ + 1; m++) {
         p.poff_h[m] = po;
         p.keoff_h[m] = ke;
-        p.koff_h[m] = k;
         eoff_h[m] = eo;
         if (m <= T_) {
             po += (long)(T_ + 2 - m) * p.nhp;
             ke += T_ + 2 - m;
-            k += T_ + 1 - m;
             eo += T_ + 3 - m;
         }
     }
@@ -1788,7 +1785,7 @@ template <typename T> int plan_create(Plan<T> &p, int nlon, int nlat, int ntrunc
         }
     std::vector<int2> kemn(p.nlme), kmn(p.nlm);
     ke = 0;
-    k = 0;
+    int k = 0;
     for (int m = 0; m <= T_; m++)
         for (int n = m; n <= T_ + 1; n++) {
             kemn[ke++] = int2{m, n};
