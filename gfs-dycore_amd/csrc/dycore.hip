@@ -705,8 +705,8 @@ template <typename T> static bool columns_serial(long ng, int nm, int ntr, int n
 // bits. The vorticity tendency shows the rounding most, as the curl of the pressure gradient
 // nearly vanishes; its error in the 2-norm here and in k_columns, rough states of 64
 // levels: T84 6.69e-6 and 6.68e-6, T126 9.12e-6 and 9.01e-6, T170 1.207e-5 and 1.213e-5,
-// T254 1.780e-5 and 1.778e-5; after a day of Held-Suarez T126 1.10e-6 and 1.09e-6, T254
-// 9.9e-7 and 9.9e-7; the other tendencies alike (2 %). What the FP32 rule keeps is the order
+// T254 1.780e-5 and 1.778e-5; states of a Held-Suarez run T126 1.10e-6 and 1.09e-6, T254
+// 9.9e-7 and 9.9e-7; the other tendencies' alike, ln ps' up to 8 % smaller in k_columns. What the FP32 rule keeps is the order
 // of sums itself, by which a large getdyntend call's single coefficients differ by up to
 // 3e-5 of the largest, and k_columns' passes inside advance by a few parts in 1e6 of the state.
 template <typename T, bool VC>
@@ -715,9 +715,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 3 : 4) void k_columns_serial(
     T *__restrict__ psg_out, T *__restrict__ dlnpsdt_out, const T *__restrict__ dphisdx,
     const T *__restrict__ dphisdy, const T *__restrict__ ak_, const T *__restrict__ bk_,
     const T *__restrict__ ck_, const T *__restrict__ dbk_, const T *__restrict__ dak_, const T *__restrict__ sinlat,
-    int nl, int ntr, int nsyn, int nan, long ng, int nlon, T rd, T kappa, T cvcp, T twoom,
+    int nl, int ntr_, int nsyn, int nan, long ng, int nlon, T rd, T kappa, T cvcp, T twoom,
     const cplx<T> *__restrict__ spec, int nfs, T *__restrict__ colq, const T *__restrict__ vcg,
     const T *__restrict__ svcg, const T *__restrict__ vfsvc, T vcamp, int store) {
+    const int ntr = sizeof(T) == 8 ? 0 : ntr_;  // in FP64 no pass with tracers comes here
     __shared__ T ak[MAXLEV + 1], bk[MAXLEV + 1], ck[MAXLEV], dbk[MAXLEV], dak[MAXLEV];
     for (int i = threadIdx.x; i <= nl; i += blockDim.x) {
         ak[i] = ak_[i];
@@ -790,7 +791,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 3 : 4) void k_columns_serial(
     const T dlnpsdt = -db / ps - cb;
     psg_out[(long)mem * ng + col] = ps;
     dlnpsdt_out[(long)mem * ng + col] = dlnpsdt;
-    if (colq) {
+    if (ntr > 0 && colq) {
         // column tracer mass of the dry-mass diagnostic (dyn_run.f90:138-145)
         T s = 0;
         for (int K = 1; K <= nl; K++) {
