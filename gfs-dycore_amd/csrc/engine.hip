@@ -296,8 +296,7 @@ template <typename T> int Engine<T>::spectogrd_noalloc(const void *spec, void *g
         return GFSDC_ESTATE;
     }
     const int ldc = round_up(2 * nf, COL_PAD) + COL_SKEW;
-    const size_t o_sx = align256(sizeof(SynthDesc) * nf) + align256((size_t)nf);  // room for a descriptor and a flag each
-    const size_t o_fs = o_sx + align256(sizeof(T) * (size_t)plan.nlme * ldc);
+    const size_t o_fs = align256(sizeof(T) * (size_t)plan.nlme * ldc);
     const size_t need = o_fs + sizeof(T) * (size_t)(plan.ntrunc + 1) * plan.nlat * ldc;
     if (need > NOALLOC_SCRATCH_BYTES) {
         set_error("spectogrd_noalloc: " + std::to_string(nf) + " fields at T" + std::to_string(plan.ntrunc) + " (" +
@@ -306,7 +305,7 @@ template <typename T> int Engine<T>::spectogrd_noalloc(const void *spec, void *g
                   " MiB (use gfsdc_spectogrd, or fewer fields per call)");
         return GFSDC_EINVAL;
     }
-    T *sx = (T *)(base + o_sx), *fs = (T *)(base + o_fs);
+    T *sx = (T *)base, *fs = (T *)(base + o_fs);
     launch_gather_ref(plan, (const cplx<T> *)spec, nf, sx, ldc, stream);
     launch_leg_synth(plan, sx, ldc, fs, ldc, 2 * nf, stream);
     launch_fft_synth(plan, fs, ldc, (T *)grid, (long)plan.nlat * plan.nlon, nf, nullptr, stream);
