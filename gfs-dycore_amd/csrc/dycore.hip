@@ -1212,9 +1212,13 @@ __global__ __launch_bounds__(256) void k_area(T *__restrict__ a, const T *__rest
         __syncthreads();
     };
     // counts this workgroup in (thread 0) and says whether it was the n-th. Thread 0 has
-    // stored the workgroup's part with device-scope (write-through) stores and waits
-    // for them here, and they are read with device-scope loads: a release fence would
-    // write back the L2 of the XCD for each workgroup (16 members at T126: 60 us)
+    // stored the workgroup's part with device-scope stores and waits for them here, and
+    // they are read with device-scope loads. That orders them by what gfx950 does (other
+    // chips are refused when a context is made) and not by the memory model, for which the
+    // count would have to release and acquire: here such a store is written through to
+    // where every XCD's device-scope loads read, and vmcnt counts it until it is there. A
+    // release would write back the L2 of the XCD for each workgroup (16 members at T126:
+    // 60 us)
     auto arrive = [&](unsigned *at, int n) {
         if (tid == 0) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -208,9 +208,11 @@ template <typename T> int Engine<T>::output(const T *d, void *p, size_t n, int d
 // Host fields up to this size (in the context's element type) are copied by the host
 // into pinned memory that the first kernel reads and the last one writes over the bus,
 // instead of by two queued copies of a pageable buffer, each longer than such a kernel.
-// T42 FP64, synthesis and analysis: one field (64 KB) 42 and 40 -> 29 and 27 us, six
-// fields 56 and 48 -> 45 and 40 us. Past a megabyte (100 us) the 10 us no longer count,
-// and a context would hold more than 4 MB of such memory.
+// T42 FP64, synthesis and analysis: one field (64 KB) 38 and 43 -> 28 and 26 us; T126 one
+// field (0.6 MB) 71 and 69 -> 55 and 53 us; T170 one (1 MB, the limit) 110 and 103 -> 91
+// and 88 us. The line bounds what a context holds of such memory, 4 MB: larger fields would
+// gain as well, T254 one (2.3 MB) 197 and 167 -> 166 and 147 us, two 348 and 247 -> 304 and
+// 237 us, until at four (9 MB, 648 and 423 -> 569 and 442 us) the analysis loses.
 constexpr size_t HOST_SMALL = 1 << 20;
 
 // pinned buffer i (0, 1: inputs, 2, 3: outputs) for n values of a caller's field, or null:
