@@ -2209,8 +2209,9 @@ __global__ __launch_bounds__(256) void k_si_mfma(
     const T *__restrict__ ten2, T *__restrict__ e1_, T *__restrict__ e2_,
     const T *__restrict__ At, const T *__restrict__ Bt, const T *__restrict__ Dt,
     const T *__restrict__ sv, const T *__restrict__ tor, const T *__restrict__ disspec,
-    const T *__restrict__ diffp, const T *__restrict__ dmpp, const int2 *__restrict__ tiles, int stage, Coeffs3 cf, SiNext cn, T cimp, int do_implicit, int damp, int nl, int ntr,
-    int nfs, int nm, int ntrunc, T dt, double *__restrict__ clock, double dtd) {
+    const T *__restrict__ diffp, const T *__restrict__ dmpp, const int2 *__restrict__ tiles, int stage, Coeffs3 cf,
+    SiNext cn, T cimp, int do_implicit, int damp, int nl, int ntr, int nfs, int nm, int ntrunc, T dt,
+    double *__restrict__ clock, double dtd) {
     constexpr int C = SiCfg<T>::C, W = SiCfg<T>::W, LD = SiCfg<T>::LD;
     typedef cplx<T> V2;
     __shared__ T S0[64][LD], S1[64][LD], S2[64][LD], S3[64][LD];

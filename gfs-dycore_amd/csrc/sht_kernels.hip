@@ -1060,7 +1060,8 @@ __host__ __device__ constexpr int fft_threads(int nfft, int nc) { return fft_wav
 
 template <typename T, int NFFT, int MAXN, int NC>
 __global__ __launch_bounds__(fft_threads(NFFT, NC)) void k_fft_synth(const T *__restrict__ fs, int ldf, T *__restrict__ grid,
-                                                   T *__restrict__ grid2, int nsplit, long gstride, int nf, const unsigned char *__restrict__ rflag, int rall,
+                                                   T *__restrict__ grid2, int nsplit, long gstride, int nf,
+                                                   const unsigned char *__restrict__ rflag, int rall,
                                                    const T *__restrict__ mean, const int *__restrict__ slot,
                                                    const T *__restrict__ rcos, const cplx<T> *__restrict__ tw,
                                                    int nlon, int nlat, int ntrunc, Radices rd, int fofs,
@@ -1509,8 +1510,10 @@ __global__ __launch_bounds__(256) void k_scatter_ref(const T *__restrict__ sx, i
                 ul = buf[0][f][r - 1];
                 vl = buf[1][f][r - 1];
             }
-            qa[o] = cplx<T>{il * ((-fm * v.y - (cp * uh.x - cm * ul.x)) * rrs), il * ((fm * v.x - (cp * uh.y - cm * ul.y)) * rrs)};
-            qb[o] = cplx<T>{il * ((-fm * u.y + (cp * vh.x - cm * vl.x)) * rrs), il * ((fm * u.x + (cp * vh.y - cm * vl.y)) * rrs)};
+            qa[o] = cplx<T>{il * ((-fm * v.y - (cp * uh.x - cm * ul.x)) * rrs),
+                            il * ((fm * v.x - (cp * uh.y - cm * ul.y)) * rrs)};
+            qb[o] = cplx<T>{il * ((-fm * u.y + (cp * vh.x - cm * vl.x)) * rrs),
+                            il * ((fm * u.x + (cp * vh.y - cm * vl.y)) * rrs)};
         }
     }
 }
@@ -1985,11 +1988,10 @@ static void fft_synth_nf(const Plan<T> &p, const T *fs, int ldf, T *grid, long g
                          const int *nfdyn, const FieldMap &fmap, T rdx, const FftOpt<T> &o) {
     constexpr int MN = FftCfg<T>::MAXN;
     dim3 g(p.nhalf * ((nf + NF - 1) / NF));
-#define FFT_SYN(NC)                                                                                             \
-    hipLaunchKernelGGL((k_fft_synth<T, NF, MN, NC>), g, dim3(fft_threads(NF, NC)), 0, s, fs, ldf, grid, o.second, o.nsplit, gstride, nf,   \
-                       rflag, o.rall, mean, slot,                                                                     \
-                       p.rcos, (const cplx<T> *)p.tw, p.nlon, p.nlat, p.ntrunc, radices_of(p.nrad, p.rad), fofs, \
-                       nfdyn, fmap, rdx)
+#define FFT_SYN(NC)                                                                                              \
+    hipLaunchKernelGGL((k_fft_synth<T, NF, MN, NC>), g, dim3(fft_threads(NF, NC)), 0, s, fs, ldf, grid, o.second, \
+                       o.nsplit, gstride, nf, rflag, o.rall, mean, slot, p.rcos, (const cplx<T> *)p.tw, p.nlon,   \
+                       p.nlat, p.ntrunc, radices_of(p.nrad, p.rad), fofs, nfdyn, fmap, rdx)
     // the lengths of spectral models' grids, one wavefront per field (the general
     // kernel, any 2^a 3^b, takes workgroup barriers and run-time divisors: 256 FP32
     // fields at 192 points 29.0 us against 11.8, at 512 points 101.9 against 50.4)
@@ -2017,11 +2019,10 @@ static void fft_anal_nf(const Plan<T> &p, const T *grid, long gstride, int nf, c
                         int ldf, hipStream_t s, const int *nfdyn, const FftOpt<const T> &o) {
     constexpr int MN = FftCfg<T>::MAXN;
     dim3 g(p.nhalf * ((nf + NF - 1) / NF));
-#define FFT_ANA(NC)                                                                                             \
-    hipLaunchKernelGGL((k_fft_anal<T, NF, MN, NC>), g, dim3(fft_threads(NF, NC)), 0, s, grid, o.second, o.nsplit, gstride, nf, rflag, o.rall, \
-                       p.rcos, p.wfac,                                                                        \
-                       (const cplx<T> *)p.tw, fa, ldf, p.nlon, p.nlat, p.nhp, p.ntrunc, radices_of(p.nrad, p.rad), \
-                       nfdyn)
+#define FFT_ANA(NC)                                                                                               \
+    hipLaunchKernelGGL((k_fft_anal<T, NF, MN, NC>), g, dim3(fft_threads(NF, NC)), 0, s, grid, o.second, o.nsplit, \
+                       gstride, nf, rflag, o.rall, p.rcos, p.wfac, (const cplx<T> *)p.tw, fa, ldf, p.nlon, p.nlat, \
+                       p.nhp, p.ntrunc, radices_of(p.nrad, p.rad), nfdyn)
     if constexpr (NF > 2)  // as fft_synth_nf
         switch (p.nlon) {
         case 64: FFT_ANA(64); return;
@@ -2095,9 +2096,9 @@ void launch_anal_scatter(const Plan<T> &p, const T *sx, int ldx, const AnalDesc 
     template void launch_leg_anal<T>(const Plan<T> &, const T *, int, T *, int, int, hipStream_t, const int *); \
     template void launch_fft_synth<T>(const Plan<T> &, const T *, int, T *, long, int, const unsigned char *,  \
                                       hipStream_t, const T *, const int *, int, const int *, const FieldMap *, \
-                                      double, const FftOpt<T> &);                                                                 \
+                                      double, const FftOpt<T> &);                                              \
     template void launch_fft_anal<T>(const Plan<T> &, const T *, long, int, const unsigned char *, T *, int,   \
-                                     hipStream_t, const int *, const FftOpt<const T> &);                                             \
+                                     hipStream_t, const int *, const FftOpt<const T> &);                       \
     template void launch_anal_scatter<T>(const Plan<T> &, const T *, int, const AnalDesc *, int, cplx<T> *,    \
                                          long, long, double, hipStream_t, const int *, bool);
 INST(float)
